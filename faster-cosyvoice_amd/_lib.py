@@ -114,6 +114,9 @@ SIGNATURES = {
     "fcv_hift_create": (c_int32, [POINTER(FcvHiftDims), POINTER(c_void_p), c_int32,
                                   POINTER(c_void_p)]),
     "fcv_hift_destroy": (c_int32, [c_void_p]),
+    "fcv_hift_packed_bytes": (c_size_t, [c_void_p]),
+    "fcv_hift_pack_weights": (c_int32, [c_void_p, c_void_p, c_size_t, c_void_p]),
+    "fcv_hift_use_packed": (c_int32, [c_void_p, c_void_p, c_size_t]),
     "fcv_hift_output_samples": (ctypes.c_int64, [c_void_p, c_int32, c_int32]),
     "fcv_hift_workspace_bytes": (c_size_t, [c_void_p, POINTER(c_int32), POINTER(c_int32),
                                             c_int32]),

@@ -20,7 +20,7 @@ LIB_NAME = "libfcvdit.so"
 ARCH = "gfx950"
 
 SOURCES = ["gemm.hip", "gemv.hip", "attention.hip", "conv.hip", "elementwise.hip", "frontend.hip",
-           "hift.hip", "hift_capi.hip", "capi.hip"]
+           "hift.hip", "hift_split.hip", "hift_capi.hip", "capi.hip"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -50,7 +50,8 @@ def library_path() -> Path:
 # conversion into v_fma_mix (one rounding instead of two) in some template instantiations and
 # not in others, so an element's fp16 bits would depend on the GEMM tile shape, and with it on
 # the batch a document is packed with.
-EXACT_SOURCES = {"gemm.hip", "gemv.hip", "attention.hip", "conv.hip", "elementwise.hip", "capi.hip"}
+EXACT_SOURCES = {"gemm.hip", "gemv.hip", "attention.hip", "conv.hip", "elementwise.hip", "capi.hip",
+                 "hift_split.hip"}
 EXACT_FLAGS = ["-ffp-contract=off"]
 
 

@@ -1,8 +1,9 @@
 // HiFT vocoder kernels on gfx950 (see hift.hpp for the layout and the launch contracts).
 //
-// Every convolution of the vocoder -- the fp64 F0 predictor, conv_pre, the upsampling convs,
-// the strided source convs, the resblock convs and conv_post -- is one implicit GEMM on the
-// matrix cores (v_mfma_{f32,f64}_16x16x4): weights are the A operand (rows = output channels),
+// Every convolution of the vocoder is one implicit GEMM on the matrix cores.  The causal
+// unit-stride ones (upsampling, resblocks, conv_post) run in hift_split.hip where the handle has
+// split weights; the rest -- the fp64 F0 predictor, conv_pre, the strided source convs -- run
+// here on v_mfma_{f32,f64}_16x16x4: weights are the A operand (rows = output channels),
 // the gathered input rows the B operand, so a lane's four accumulators are four channels of one
 // time step (consecutive in fp32; four apart in fp64, whose 16x16 result is laid out by rows
 // 4 e + lane / 16).  Operands go through LDS K-contiguous, 32 (or 16) input channels of one tap
@@ -15,6 +16,7 @@
 #include <cstdlib>
 
 #include "hift.hpp"
+#include "hift_device.hpp"
 
 namespace fcv {
 namespace {
@@ -36,30 +38,13 @@ __device__ __forceinline__ f64x4 mfma_16x16x4(double a, double b, const f64x4& c
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// largest d with cu[d] <= row
-__device__ __forceinline__ int doc_of(const int32_t* cu, int n_docs, int row) {
-  int lo = 0, hi = n_docs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cu[mid] <= row) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// Snake(x) = x + sin(a x)^2 / (a + 1e-9), with inv = 1 / (a + 1e-9) precomputed in fp32.
-// sin by v_sin_f32 on the fractional part of the argument in turns (v_fract_f32 is exact).
-__device__ __forceinline__ float snake(float x, float a, float inv) {
-  const float turns = (x * a) * 0.15915494309189535f;
-  const float s = __builtin_amdgcn_sinf(__builtin_amdgcn_fractf(turns));
-  return x + inv * (s * s);
-}
-
 template <typename T>
 __device__ __forceinline__ T elu(T x) { return x > T(0) ? x : T(expm1(x)); }
 
-// epilogue of one output element (row, channel c) from its accumulator value
+// epilogue of one output element (row, channel c) from its accumulator value; m: raised to the
+// largest finite magnitude written to out (fp32)
 template <typename T>
-__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, T acc) {
+__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, T acc, float& m) {
   T v = acc + static_cast<const T*>(p.bias)[c];
   if constexpr (sizeof(T) == 8) {
     if (p.elu) v = elu(v);
@@ -71,6 +56,7 @@ __device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, 
   if constexpr (sizeof(T) == 4) {
     if (p.snake_out) v = snake(v, p.alpha[c], p.inv_alpha[c]);
     if (p.out2) static_cast<float*>(p.out2)[i] = snake(v, p.alpha2[c], p.inv_alpha2[c]);
+    m = fmaxf(m, finite_abs(v));
   }
   static_cast<T*>(p.out)[i] = v;
 }
@@ -79,7 +65,8 @@ __device__ __forceinline__ float4 ld4f(const float* q) { return *reinterpret_cas
 
 // conv_store1 for the four consecutive fp32 channels c .. c + 3 of one row, with 16-byte loads
 // and stores (same operations in the same order, so the results are bit-identical)
-__device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, const f32x4& acc) {
+__device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, const f32x4& acc,
+                                            float& m) {
   const float4 b = ld4f(static_cast<const float*>(p.bias) + c);
   float v[4] = {acc[0] + b.x, acc[1] + b.y, acc[2] + b.z, acc[3] + b.w};
   const long i = row * p.ldo + c;
@@ -104,6 +91,8 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
     for (int e = 0; e < 4; ++e) w[e] = snake(v[e], p.alpha2[c + e], p.inv_alpha2[c + e]);
     *reinterpret_cast<float4*>(static_cast<float*>(p.out2) + i) = float4{w[0], w[1], w[2], w[3]};
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) m = fmaxf(m, finite_abs(v[e]));
   *reinterpret_cast<float4*>(static_cast<float*>(p.out) + i) = float4{v[0], v[1], v[2], v[3]};
 }
 
@@ -111,16 +100,16 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
 //   fp32: channels cb + 4 lg + e;  fp64: channels cb + 4 e + lg  (e = 0..3)
 template <typename T>
 __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
-                           const typename Vec4<T>::type& acc) {
+                           const typename Vec4<T>::type& acc, float& m) {
   if constexpr (sizeof(T) == 4) {
     if (p.vec4 && cb + 4 * lg + 3 < p.cout) {
-      conv_store4(p, row, cb + 4 * lg, acc);
+      conv_store4(p, row, cb + 4 * lg, acc, m);
       return;
     }
   }
   for (int e = 0; e < 4; ++e) {
     const int c = sizeof(T) == 4 ? cb + 4 * lg + e : cb + 4 * e + lg;
-    if (c < p.cout) conv_store1<T>(p, row, c, acc[e]);
+    if (c < p.cout) conv_store1<T>(p, row, c, acc[e], m);
   }
 }
 
@@ -257,6 +246,9 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
   }
 
   // D[i = channel][j = row]: lane holds row li and four channels of each 16x16 tile
+  const int tile_doc = doc_of(docs->b, n_docs, r0);
+  const bool one_doc = min(r0 + TS, rows_out) <= docs->b[tile_doc + 1];
+  float tile_max = 0.0f;
 #pragma unroll
   for (int b = 0; b < NQ; ++b) {
     const int rr = r0 + wt * (TS / 2) + b * 16 + li;
@@ -264,32 +256,67 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
     const int d = doc_of(docs->b, n_docs, rr);
     const int pp = rr - docs->b[d];
     const long row_w = p.reflect ? (long)docs->b[d] + d + 1 + pp : rr;
+    float m = 0.0f;
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
       const int cb = co0 + wc * (TS / 2) + a * 16;
-      conv_store<T>(p, row_w, cb, lg, acc[a][b]);
+      conv_store<T>(p, row_w, cb, lg, acc[a][b], m);
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
-      if (p.reflect && pp == 1) conv_store<T>(p, (long)docs->b[d] + d, cb, lg, acc[a][b]);
+      if (p.reflect && pp == 1) conv_store<T>(p, (long)docs->b[d] + d, cb, lg, acc[a][b], m);
     }
+    if (sizeof(T) == 4 && p.amax_out) {
+      if (one_doc) tile_max = fmaxf(tile_max, m);
+      else raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m);
+    }
+  }
+  if (sizeof(T) == 4 && p.amax_out && one_doc) {
+    __shared__ float wmax[4];
+    tile_max = wave_max(tile_max);
+    if (lane == 0) wmax[wave] = tile_max;
+    __syncthreads();
+    if (tid == 0)
+      raise_amax(p.amax_out, tile_doc, blockIdx.x + blockIdx.y,
+                 fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
   }
 }
 
+// out[r][c] = snake(x[r][c]), four channels a thread
 __global__ __launch_bounds__(256) void snake_kernel(const float* __restrict__ x, int ldx,
                                                     float* __restrict__ out, int ldo, int C,
                                                     const float* __restrict__ alpha,
                                                     const float* __restrict__ inv_alpha,
+                                                    uint32_t* __restrict__ amax,
                                                     const HiftDocs* __restrict__ docs) {
   const int rows = docs->b[docs->n];
   const int q = C / 4;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)rows * q) return;
+  const long first = (long)blockIdx.x * blockDim.x, total = (long)rows * q;
+  if (first >= total) return;
+  const long i = first + threadIdx.x;
   const long r = i / q;
-  const int c = (int)(i - r * q) * 4;
-  const f32x4 v = *reinterpret_cast<const f32x4*>(x + r * ldx + c);
-  f32x4 y;
+  float m = 0.0f;
+  if (i < total) {
+    const int c = (int)(i - r * q) * 4;
+    const f32x4 v = *reinterpret_cast<const f32x4*>(x + r * ldx + c);
+    f32x4 y;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) y[e] = snake(v[e], alpha[c + e], inv_alpha[c + e]);
-  *reinterpret_cast<f32x4*>(out + r * ldo + c) = y;
+    for (int e = 0; e < 4; ++e) {
+      y[e] = snake(v[e], alpha[c + e], inv_alpha[c + e]);
+      m = fmaxf(m, finite_abs(y[e]));
+    }
+    *reinterpret_cast<f32x4*>(out + r * ldo + c) = y;
+  }
+  if (!amax) return;
+  const int d0 = doc_of(docs->b, docs->n, (int)(first / q));
+  if (min(first + 255, total - 1) / q < docs->b[d0 + 1]) {
+    __shared__ float wmax[4];
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      raise_amax(amax, d0, blockIdx.x, fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
+  } else if (i < total) {
+    raise_amax(amax, doc_of(docs->b, docs->n, (int)r), blockIdx.x, m);
+  }
 }
 
 __global__ __launch_bounds__(256) void to_f64_kernel(const float* __restrict__ x,
@@ -519,12 +546,12 @@ hipError_t hift_conv_f64(const HiftConv& p, const HiftDocs* docs, hipStream_t st
 }
 
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
-                      const float* alpha, const float* inv_alpha, const HiftDocs* docs,
-                      hipStream_t stream) {
+                      const float* alpha, const float* inv_alpha, uint32_t* amax,
+                      const HiftDocs* docs, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   const long n = (long)rows * (C / 4);
   hipLaunchKernelGGL(snake_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, x, ldx, out,
-                     ldo, C, alpha, inv_alpha, docs);
+                     ldo, C, alpha, inv_alpha, amax, docs);
   return hipGetLastError();
 }
 

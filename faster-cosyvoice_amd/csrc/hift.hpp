@@ -26,6 +26,9 @@ struct HiftDocs {
 enum { HIFT_PRO_NONE = 0, HIFT_PRO_LEAKY = 1 };
 enum { HIFT_ACC_WRITE = 0, HIFT_ACC_ADD = 1, HIFT_ACC_ADD_DIV = 2 };
 
+// Largest magnitude of a tensor per document: kAmaxWords words per document (see hift_device.hpp).
+constexpr int kAmaxSub = 16, kAmaxStride = 16, kAmaxWords = kAmaxSub * kAmaxStride;
+
 // One 1-D convolution as an implicit GEMM: out[r][co] over output rows r of every document.
 // Input position of tap j for output position p of a document:
 //   u = p * stride + j * dil - pad;  q = up > 1 ? (u >= 0 ? u / up : -1) : u
@@ -46,16 +49,35 @@ struct HiftConv {
   void* out; int ldo;
   void* out2; const float* alpha2; const float* inv_alpha2;  // out2 = snake(y) (optional)
   int vec4;                                // set by the launch: 16-byte epilogue accesses
+  // split f16 form (hift_conv_split): packed weights of co_pad channels, their inverse scales and
+  // biases ([co_pad] each, one after the other);
+  // the largest finite |input| per document (fp32 bits)
+  const void* wsplit; const float* winv; int co_pad;
+  const uint32_t* amax_in;
+  // per document, raised to the largest finite magnitude written to out / out2 (optional)
+  uint32_t* amax_out; uint32_t* amax_out2;
 };
 
 hipError_t hift_conv_f32(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
 hipError_t hift_conv_f64(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
 
+// The fp32 convolution with both operands split into two f16 halves (hift_split.hip), for the
+// shapes hift_split_eligible takes (its rule reads the shape only, not the row count): unit
+// stride, all context on the left, input channels a multiple of 32.
+bool hift_split_eligible(const HiftConv& p);
+hipError_t hift_conv_split(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
+// its packed weights: bytes, and the packing of fp32 [co_pad][k][cin] with its cout biases (inv:
+// [co_pad] inverse scales, then [co_pad] biases)
+size_t hift_split_bytes(int co_pad, int k, int cin);
+hipError_t hift_pack_split(const float* w, const float* bias, int cout, int co_pad, int k, int cin,
+                           void* dst, float* inv, hipStream_t stream);
+hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream);
+
 // out[r][c] = snake(x[r][c]) for the live rows docs->b[docs->n] (grid: `rows`) x C channels
-// (C % 4 == 0), row strides ldx / ldo
+// (C % 4 == 0), row strides ldx / ldo; amax (optional): see HiftConv::amax_out
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
-                      const float* alpha, const float* inv_alpha, const HiftDocs* docs,
-                      hipStream_t stream);
+                      const float* alpha, const float* inv_alpha, uint32_t* amax,
+                      const HiftDocs* docs, hipStream_t stream);
 
 // fp32 -> fp64 of the live rows docs->a[docs->n] (grid: `rows`) x C values
 hipError_t hift_to_f64(const float* x, double* y, int rows, int C, const HiftDocs* docs,

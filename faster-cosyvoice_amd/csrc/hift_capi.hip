@@ -35,6 +35,15 @@ struct FcvHift {
   std::vector<Graph> graphs;
   std::vector<std::vector<uintptr_t>> seen;
   long captures = 0;
+  // split f16 weights (caller-owned), by index of the fp32 weight: byte offsets of the packed
+  // block and of its inverse scales, -1 where the convolution stays on the fp32 kernel
+  struct Packed {
+    long w = -1, inv = -1;
+    int co_pad = 0;
+  };
+  std::vector<Packed> packed;
+  size_t packed_bytes = 0;
+  const char* packed_base = nullptr;
 };
 
 namespace {
@@ -134,7 +143,8 @@ struct Capacity {
   int spec, samples, src;              // STFT frames, output samples, source samples
   std::vector<int> stage, stage_w;     // upsampling-conv rows and written rows per stage
   size_t mel64, h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, r, t1, s1, si, y, fr,
-      tables, total;
+      amax, tables, total;
+  int amax_slots;                      // per document: one per tensor a split convolution reads
 };
 
 // Tables of one call, in launch order (see run): their count for n_stages stages.
@@ -171,6 +181,8 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
     *b = take(sizeof(float) * smax);
   C.y = take(sizeof(float) * C.spec * kSpecLd);
   C.fr = take(sizeof(float) * C.spec * kFrameLd);
+  C.amax_slots = 1 + d.n_stages * (1 + 2 * d.n_dilations * (1 + d.n_kernels));
+  C.amax = take(sizeof(uint32_t) * fcv::kAmaxWords * C.amax_slots * docs);
   C.tables = take(sizeof(HiftDocs) * table_count(d));
   C.total = off;
   return C;
@@ -264,38 +276,71 @@ std::vector<HiftDocs> make_tables(const FcvHiftDims& d, const Plan& P) {
   return t;
 }
 
-HiftConv conv_base(const void* x, int ldx, const void* w, const void* b, int cout, int cin_pad,
-                   int k, void* out, int ldo, int rows_out) {
+HiftConv conv_base(const void* x, int ldx, int cout, int cin_pad, int k, void* out, int ldo,
+                   int rows_out) {
   HiftConv p{};
-  p.x = x; p.ldx = ldx; p.w = w; p.bias = b; p.cout = cout; p.cin_pad = cin_pad; p.k = k;
+  p.x = x; p.ldx = ldx; p.cout = cout; p.cin_pad = cin_pad; p.k = k;
   p.stride = 1; p.dil = 1; p.pad = 0; p.up = 1; p.rows_out = rows_out;
   p.out = out; p.ldo = ldo; p.div = 1.0f;
   return p;
 }
 
+// The convolutions of one call.  Where the handle has split weights for a convolution it runs on
+// the f16 matrix cores, scaled by the largest input its producer recorded in a slot of the
+// workspace (one per tensor, `docs` values each, zeroed at the start of the call).
+struct Convs {
+  const FcvHift* h;
+  uint32_t* amax;
+  int docs_cap, slots, used = 0;
+  hipStream_t st;
+
+  // a slot for a tensor that a split convolution will read (null: the handle has no split weights)
+  uint32_t* slot() {
+    if (!h->packed_base || used >= slots) return nullptr;
+    return amax + (size_t)docs_cap * fcv::kAmaxWords * used++;
+  }
+  // p with weight index wi (bias wi + 1), its input's slot `in`
+  int run(HiftConv p, int wi, const uint32_t* in, const HiftDocs* docs) const {
+    p.w = h->w[wi];
+    p.bias = h->w[wi + 1];
+    const FcvHift::Packed& k = h->packed[wi];
+    if (h->packed_base && k.w >= 0 && in) {
+      p.wsplit = h->packed_base + k.w;
+      p.winv = reinterpret_cast<const float*>(h->packed_base + k.inv);
+      p.co_pad = k.co_pad;
+      p.amax_in = in;
+      FCV_HIP(fcv::hift_conv_split(p, docs, st));
+      return FCV_OK;
+    }
+    FCV_HIP(fcv::hift_conv_f32(p, docs, st));
+    return FCV_OK;
+  }
+};
+
 // one ResBlock (generator.py:110-116) on x (rows by `docs`, C channels): for each dilation
 // j: r = r + conv2(snake2(conv1(snake1(r)))); the last conv2 writes its result per `mode`
-// (write / accin + y / (accin + y) / div) into `out`.  `wb` points at the block's 8 * D
-// weight pointers.  x is read as the first residual; r holds the running value.  `rows` is the
-// capacity the grids cover.
-int run_resblock(const FcvHiftDims& d, const void* const* wb, int k, const int* dils,
-                 const float* x, float* r, float* t1, float* s1, float* out, int mode,
-                 const float* accin, float div, int C, int rows, const HiftDocs* docs,
-                 hipStream_t st) {
-  const int D = d.n_dilations;
-  FCV_HIP(fcv::hift_snake(x, C, s1, C, rows, C, static_cast<const float*>(wb[4]),
-                          static_cast<const float*>(wb[5]), docs, st));
+// (write / accin + y / (accin + y) / div) into `out`, its magnitude into `amax_out` (optional).
+// `wi` is the index of the block's 8 * D weights.  x is read as the first residual; r holds the
+// running value.  `rows` is the capacity the grids cover.
+int run_resblock(Convs& cv, int wi, int k, const int* dils, const float* x, float* r, float* t1,
+                 float* s1, float* out, int mode, const float* accin, float div,
+                 uint32_t* amax_out, int C, int rows, const HiftDocs* docs) {
+  const int D = cv.h->d.n_dilations;
+  auto F = [&](int i) { return static_cast<const float*>(cv.h->w[i]); };
+  uint32_t* a_s1 = cv.slot();
+  FCV_HIP(fcv::hift_snake(x, C, s1, C, rows, C, F(wi + 4), F(wi + 5), a_s1, docs, cv.st));
   for (int j = 0; j < D; ++j) {
-    const void* const* q = wb + 8 * j;
-    HiftConv c1 = conv_base(s1, C, q[0], q[1], C, C, k, t1, C, rows);
+    const int q = wi + 8 * j;
+    HiftConv c1 = conv_base(s1, C, C, C, k, t1, C, rows);
     c1.dil = dils[j];
     c1.pad = causal_padding(k, dils[j]);
     c1.snake_out = 1;
-    c1.alpha = static_cast<const float*>(q[6]);
-    c1.inv_alpha = static_cast<const float*>(q[7]);
-    FCV_HIP(fcv::hift_conv_f32(c1, docs, st));
+    c1.alpha = F(q + 6);
+    c1.inv_alpha = F(q + 7);
+    c1.amax_out = cv.slot();
+    if (int rc = cv.run(c1, q, a_s1, docs)) return rc;
     const bool last = j == D - 1;
-    HiftConv c2 = conv_base(t1, C, q[2], q[3], C, C, k, last ? out : r, C, rows);
+    HiftConv c2 = conv_base(t1, C, C, C, k, last ? out : r, C, rows);
     c2.pad = causal_padding(k, 1);
     c2.add = j == 0 ? static_cast<const void*>(x) : static_cast<const void*>(r);
     c2.ld_add = C;
@@ -303,12 +348,14 @@ int run_resblock(const FcvHiftDims& d, const void* const* wb, int k, const int* 
       c2.mode = mode;
       c2.accin = accin;
       c2.div = div;
+      c2.amax_out = amax_out;
     } else {
       c2.out2 = s1;
-      c2.alpha2 = static_cast<const float*>(wb[8 * (j + 1) + 4]);
-      c2.inv_alpha2 = static_cast<const float*>(wb[8 * (j + 1) + 5]);
+      c2.alpha2 = F(q + 8 + 4);
+      c2.inv_alpha2 = F(q + 8 + 5);
+      c2.amax_out2 = a_s1 = cv.slot();
     }
-    FCV_HIP(fcv::hift_conv_f32(c2, docs, st));
+    if (int rc = cv.run(c2, q + 2, c1.amax_out, docs)) return rc;
   }
   return FCV_OK;
 }
@@ -328,15 +375,18 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- F0 predictor (fp64) -------------------------------------------------------------
   FCV_HIP(fcv::hift_to_f64(mel, F64(C.mel64), C.frames, d.in_channels, T + 0, st));
   const int fc = d.f0_channels;
-  HiftConv c0 = conv_base(F64(C.mel64), d.in_channels, w[h->i_f0], w[h->i_f0 + 1], fc,
-                          d.in_channels, 4, F64(C.h64a), fc, C.frames);
+  HiftConv c0 = conv_base(F64(C.mel64), d.in_channels, fc, d.in_channels, 4, F64(C.h64a), fc,
+                          C.frames);
+  c0.w = w[h->i_f0];
+  c0.bias = w[h->i_f0 + 1];
   c0.elu = 1;  // right-side lookahead: no left padding, zero (or context) on the right
   FCV_HIP(fcv::hift_conv_f64(c0, T + 0, st));
   double* hin = F64(C.h64a);
   double* hout = F64(C.h64b);
   for (int l = 1; l < 5; ++l) {
-    HiftConv c = conv_base(hin, fc, w[h->i_f0 + 2 * l], w[h->i_f0 + 2 * l + 1], fc, fc, 3, hout,
-                           fc, C.frames);
+    HiftConv c = conv_base(hin, fc, fc, fc, 3, hout, fc, C.frames);
+    c.w = w[h->i_f0 + 2 * l];
+    c.bias = w[h->i_f0 + 2 * l + 1];
     c.pad = causal_padding(3, 1);
     c.elu = 1;
     FCV_HIP(fcv::hift_conv_f64(c, T + 1, st));
@@ -372,11 +422,14 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- conv_pre (lookahead on the right) -------------------------------------------------
   float* xp = F32(C.xa);
   float* xn = F32(C.xn);
+  Convs cv{h, reinterpret_cast<uint32_t*>(ws + C.amax), C.docs, C.amax_slots, 0, st};
+  if (h->packed_base) FCV_HIP(fcv::hift_zero_u32(cv.amax, C.amax_slots * C.docs * fcv::kAmaxWords, st));
+  uint32_t* a_xp = cv.slot();  // magnitude of xp
   {
-    HiftConv c = conv_base(mel, d.in_channels, w[h->i_pre], w[h->i_pre + 1], d.base_channels,
-                           d.in_channels, d.conv_pre_look_right + 1, xp, d.base_channels,
-                           C.frames);
-    FCV_HIP(fcv::hift_conv_f32(c, T + 4, st));
+    HiftConv c = conv_base(mel, d.in_channels, d.base_channels, d.in_channels,
+                           d.conv_pre_look_right + 1, xp, d.base_channels, C.frames);
+    c.amax_out = a_xp;
+    if (int rc = cv.run(c, h->i_pre, nullptr, T + 4)) return rc;
   }
 
   // ---- upsampling stages -----------------------------------------------------------------
@@ -394,20 +447,18 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
     float* si = F32(C.si);
     {
       const auto kd = source_down(d, s);
-      HiftConv c = conv_base(F32(C.specbuf), kSpecLd, w[h->i_down + 2 * s],
-                             w[h->i_down + 2 * s + 1], Cs, kSpecLd, kd.first, si, Cs, nrows);
+      HiftConv c = conv_base(F32(C.specbuf), kSpecLd, Cs, kSpecLd, kd.first, si, Cs, nrows);
       c.stride = kd.second;
       c.pad = kd.second - 1;
-      FCV_HIP(fcv::hift_conv_f32(c, t_src, st));
-      if (int rc = run_resblock(d, w + h->i_srb + rb_size * s, d.source_kernels[s],
+      if (int rc = cv.run(c, h->i_down + 2 * s, nullptr, t_src)) return rc;
+      if (int rc = run_resblock(cv, h->i_srb + rb_size * s, d.source_kernels[s],
                                 d.source_dilations[s], si, F32(C.r), F32(C.t1), F32(C.s1), si,
-                                fcv::HIFT_ACC_WRITE, nullptr, 1.0f, Cs, nrows, t_w, st))
+                                fcv::HIFT_ACC_WRITE, nullptr, 1.0f, nullptr, Cs, nrows, t_w))
         return rc;
     }
     // upsampling conv on LeakyReLU(x), plus the source branch
     {
-      HiftConv c = conv_base(xp, cprev, w[h->i_ups + 2 * s], w[h->i_ups + 2 * s + 1], Cs, cprev,
-                             d.upsample_kernels[s], xn, Cs, C.stage[s]);
+      HiftConv c = conv_base(xp, cprev, Cs, cprev, d.upsample_kernels[s], xn, Cs, C.stage[s]);
       c.up = d.upsample_rates[s];
       c.pad = d.upsample_kernels[s] - 1;
       c.pro = fcv::HIFT_PRO_LEAKY;
@@ -415,9 +466,10 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
       c.reflect = last ? 1 : 0;
       c.add = si;
       c.ld_add = Cs;
-      FCV_HIP(fcv::hift_conv_f32(c, t_up, st));
+      if (int rc = cv.run(c, h->i_ups + 2 * s, a_xp, t_up)) return rc;
     }
     // mean of the resblocks
+    a_xp = cv.slot();
     for (int j = 0; j < d.n_kernels; ++j) {
       const int K = d.n_kernels;
       int mode = fcv::HIFT_ACC_WRITE;
@@ -435,9 +487,9 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
         mode = fcv::HIFT_ACC_ADD;
         accin = F32(C.xs);
       }
-      if (int rc = run_resblock(d, w + h->i_rb + rb_size * (s * K + j), d.resblock_kernels[j],
+      if (int rc = run_resblock(cv, h->i_rb + rb_size * (s * K + j), d.resblock_kernels[j],
                                 d.resblock_dilations[j], xn, F32(C.r), F32(C.t1), F32(C.s1),
-                                out, mode, accin, div, Cs, nrows, t_w, st))
+                                out, mode, accin, div, j == K - 1 ? a_xp : nullptr, Cs, nrows, t_w))
         return rc;
     }
     cprev = Cs;
@@ -447,12 +499,11 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- conv_post on LeakyReLU(x) (slope 0.01), iSTFT, clamp ------------------------------
   {
     const int spec = d.n_fft + 2;
-    HiftConv c = conv_base(xp, cprev, w[h->i_post], w[h->i_post + 1], spec, cprev, 7, F32(C.y),
-                           kSpecLd, C.spec);
+    HiftConv c = conv_base(xp, cprev, spec, cprev, 7, F32(C.y), kSpecLd, C.spec);
     c.pad = causal_padding(7, 1);
     c.pro = fcv::HIFT_PRO_LEAKY;
     c.slope = 0.01f;
-    FCV_HIP(fcv::hift_conv_f32(c, T + 5 + 3 * S, st));
+    if (int rc = cv.run(c, h->i_post, a_xp, T + 5 + 3 * S)) return rc;
   }
   FCV_HIP(fcv::hift_istft(F32(C.y), kSpecLd, window, F32(C.fr), speech, d.audio_limit, C.spec,
                           C.samples, T + 6 + 3 * S, st));
@@ -531,9 +582,100 @@ int infer(FcvHift* h, const float* mel, const int32_t* frames, const int32_t* fi
   return FCV_OK;
 }
 
+// Lays out the split weights: every convolution of run() that hift_split_eligible takes.
+void plan_packed(FcvHift* h) {
+  const FcvHiftDims& d = h->d;
+  h->packed.assign(h->w.size(), FcvHift::Packed{});
+  size_t off = 0;
+  auto add = [&](int wi, int cout, int cin, int k, int dil, int up, float slope) {
+    HiftConv p = conv_base(nullptr, 0, cout, cin, k, nullptr, 0, 0);
+    p.dil = dil;
+    p.up = up;
+    p.pad = causal_padding(k, dil);
+    if (up > 1) p.pad = k - 1;
+    p.pro = fcv::HIFT_PRO_LEAKY;
+    p.slope = slope;
+    if (!fcv::hift_split_eligible(p)) return;
+    FcvHift::Packed& e = h->packed[wi];
+    e.co_pad = (cout + 63) / 64 * 64;
+    e.w = (long)off;
+    off += align_up(fcv::hift_split_bytes(e.co_pad, k, cin));
+    e.inv = (long)off;
+    off += align_up(2 * sizeof(float) * e.co_pad);
+  };
+  auto resblock = [&](int wi, int C, int k, const int* dils) {
+    for (int j = 0; j < d.n_dilations; ++j) {
+      add(wi + 8 * j, C, C, k, dils[j], 1, 0.0f);
+      add(wi + 8 * j + 2, C, C, k, 1, 1, 0.0f);
+    }
+  };
+  const int rb = 8 * d.n_dilations;
+  int cprev = d.base_channels;
+  for (int s = 0; s < d.n_stages; ++s) {
+    const int C = stage_channels(d, s);
+    add(h->i_ups + 2 * s, C, cprev, d.upsample_kernels[s], 1, d.upsample_rates[s], d.lrelu_slope);
+    resblock(h->i_srb + rb * s, C, d.source_kernels[s], d.source_dilations[s]);
+    for (int j = 0; j < d.n_kernels; ++j)
+      resblock(h->i_rb + rb * (s * d.n_kernels + j), C, d.resblock_kernels[j],
+               d.resblock_dilations[j]);
+    cprev = C;
+  }
+  add(h->i_post, d.n_fft + 2, cprev, 7, 1, 1, 0.01f);
+  h->packed_bytes = off;
+}
+
 }  // namespace
 
 extern "C" {
+
+size_t fcv_hift_packed_bytes(const FcvHift* hift) { return hift ? hift->packed_bytes : 0; }
+
+int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes) {
+  FCV_CHECK(hift, FCV_ERR_INVALID, "null handle");
+  FCV_CHECK(hift->packed_bytes > 0, FCV_ERR_INVALID, "no convolution of this shape has split weights");
+  FCV_CHECK(packed, FCV_ERR_INVALID, "null argument");
+  FCV_CHECK(bytes >= hift->packed_bytes, FCV_ERR_INVALID,
+            "packed weights need " + std::to_string(hift->packed_bytes) + " bytes");
+  FCV_CHECK(reinterpret_cast<uintptr_t>(packed) % kAlign == 0, FCV_ERR_INVALID,
+            "packed weights must be 256-byte aligned");
+  FCV_CHECK(hift->graphs.empty() && hift->seen.empty(), FCV_ERR_STATE,
+            "set the packed weights before the first inference");
+  hift->packed_base = static_cast<const char*>(packed);
+  return FCV_OK;
+}
+
+int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t stream) {
+  if (int rc = fcv_hift_use_packed(hift, packed, bytes)) return rc;
+  const FcvHiftDims& d = hift->d;
+  char* base = static_cast<char*>(packed);
+  auto pack = [&](int wi, int cout, int cin, int k) -> int {
+    const FcvHift::Packed& e = hift->packed[wi];
+    if (e.w < 0) return FCV_OK;
+    FCV_HIP(fcv::hift_pack_split(static_cast<const float*>(hift->w[wi]),
+                                 static_cast<const float*>(hift->w[wi + 1]), cout, e.co_pad, k,
+                                 cin, base + e.w, reinterpret_cast<float*>(base + e.inv),
+                                 stream));
+    return FCV_OK;
+  };
+  auto resblock = [&](int wi, int C, int k) -> int {
+    for (int j = 0; j < d.n_dilations; ++j)
+      for (int c = 0; c < 2; ++c)
+        if (int rc = pack(wi + 8 * j + 2 * c, C, C, k)) return rc;
+    return FCV_OK;
+  };
+  const int rb = 8 * d.n_dilations;
+  int cprev = d.base_channels;
+  for (int s = 0; s < d.n_stages; ++s) {
+    const int C = stage_channels(d, s);
+    if (int rc = pack(hift->i_ups + 2 * s, C, cprev, d.upsample_kernels[s])) return rc;
+    if (int rc = resblock(hift->i_srb + rb * s, C, d.source_kernels[s])) return rc;
+    for (int j = 0; j < d.n_kernels; ++j)
+      if (int rc = resblock(hift->i_rb + rb * (s * d.n_kernels + j), C, d.resblock_kernels[j]))
+        return rc;
+    cprev = C;
+  }
+  return pack(hift->i_post, d.n_fft + 2, cprev, 7);
+}
 
 int32_t fcv_hift_weight_count(const FcvHiftDims* dims) {
   if (check_dims(dims) != FCV_OK) return 0;
@@ -570,6 +712,7 @@ int fcv_hift_create(const FcvHiftDims* dims, const void* const* weights, int32_t
   h->i_win = i++;
   h->i_ini = i++;
   h->i_tab = i++;
+  plan_packed(h);
   *out = h;
   return FCV_OK;
 }

@@ -1,0 +1,623 @@
+// The HiFT vocoder's causal fp32 convolutions on the f16 matrix cores, at fp32 accuracy.
+//
+// Every operand is held as a sum of two f16 values, x = hi + lo (22 significant bits), scaled by a
+// power of two so that the largest magnitude lies in [2^14, 2^15): a weight row by its own
+// largest weight (once, when the weights are packed), an input row by the largest finite input of
+// its document (recorded by the kernel that wrote it).  Values down to 2^-28 of the largest then
+// keep all 22 bits and smaller ones an absolute error of 2^-39 of it.  A product is
+// lo hi + hi lo + hi hi on v_mfma_f32_32x32x16_f16 with fp32 accumulators; the scales are powers
+// of two, taken out exactly in the epilogue.  Against 64-bit results the operands' rounding adds
+// 1.7e-6 to the waveform's relative error, under a tenth of what fp32 accumulation over K =
+// 192..8192 terms leaves (2.0e-5 with v_mfma_f32_16x16x4_f32), and the 16-deep f16 form rounds
+// the accumulator less often.
+//
+// Bound: three f16 MFMAs do a product's work at 16 times the fp32 form's rate each, so the ceiling
+// is a third of the f16 peak against the fp32 peak of 157 TFLOP/s.  Measured on one MI355X against
+// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.2 ms (91 -> 203 TFLOP/s
+// of fp32 work over the whole call), one 68-frame chunk 2.30 -> 1.86 ms, the error against 64 bits
+// 2.5e-5 -> 1.6e-5.  What is left of a large launch is latency: the document table, window and
+// residual reads around 14 to 88 steps of MFMAs, and LDS reads (1.3 KB per MFMA in the 64x64
+// tile).  128x128 and 64x256 tiles (32 KB fewer weight bytes a step, twice the registers) were no
+// faster: 10.7 and 10.8 against 10.4 ms.
+//
+// A workgroup owns TR output rows x TC output channels.  For each 32 input channels it splits a
+// window of input rows (the tile's rows and the left context) into LDS once, then walks the taps
+// over it: the input is read and split once, not once per tap.  A tap's weights are one
+// contiguous block of the packed table, copied straight to LDS (global_load_lds) through a ring
+// of NS stages.  Channel chunks outermost, then taps, then k-steps, then the three products: the
+// order of every output's sum is the same in every tile shape, so results do not depend on the
+// shape a launch takes.  (Compiled without floating-point contraction, as the rounding of an
+// output must not depend on the instantiation either.)
+#include <cstdlib>
+
+#include "hift.hpp"
+#include "hift_device.hpp"
+
+namespace fcv {
+namespace {
+
+constexpr int kRowBytes = 128;  // one row of 32 channels: 4 chunks of hi, 4 of lo, 16 bytes each
+constexpr int kMaxHalo = 62;    // largest left context of a tile, in rows
+// 64x64 tiles in a launch under which 64x32 tiles run (twice the workgroups; above, the larger
+// tile's halved weight traffic is worth more: 286 frames 2.46 -> 2.38 ms at 144 tiles, 68 frames
+// 2.05 against 2.02 ms at 36)
+constexpr long kSmallBelow = 96;
+
+// position of 16-byte chunk `chunk` in LDS row `row`: 16 consecutive rows read at one chunk index
+// hit 16 distinct 16-byte bank groups
+__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+// lane l copies 16 bytes at base + voff to LDS bytes [16 l, 16 l + 16) from the scalar address
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+// every LDS access of this wave has completed
+__device__ __forceinline__ void wait_lgkm0() {
+  __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x3 << 14));
+}
+
+// 2^e as a float exponent field: the scale that brings `amax` into [2^14, 2^15) (1 for an
+// all-zero tensor; tiny tensors are raised by at most 2^100), and its inverse
+__device__ __forceinline__ int scale_field(uint32_t amax_bits) {
+  const int e = (int)(amax_bits >> 23) & 255;
+  return amax_bits == 0 ? 127 : min(max(268 - e, 14), 227);
+}
+__device__ __forceinline__ float field_to_float(int f) { return __uint_as_float((uint32_t)f << 23); }
+
+// a document's largest magnitude (fp32 bits) over its kAmaxSub words: by the whole wave, by a lane
+__device__ __forceinline__ uint32_t doc_amax(const uint32_t* amax, int d, int lane) {
+  const uint32_t v = amax[((long)d * kAmaxSub + (lane & (kAmaxSub - 1))) * kAmaxStride];
+  return __float_as_uint(wave_max(__uint_as_float(v)));
+}
+__device__ __forceinline__ uint32_t amax_serial(const uint32_t* amax, int d) {
+  uint32_t m = 0;
+  for (int i = 0; i < kAmaxSub; ++i) m = max(m, amax[((long)d * kAmaxSub + i) * kAmaxStride]);
+  return m;
+}
+
+// four values, scaled, as their f16 halves
+__device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4& lo) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x = v[e] * s;
+    const f16 h = (f16)x;
+    const float r = x - (float)h;
+    hi[e] = h;
+    // an infinite value has no remainder (inf - inf); NaN stays in hi
+    lo[e] = (f16)(fabsf(x) <= 3.402823466e38f ? r : 0.0f);
+  }
+}
+
+__device__ __forceinline__ f32x4 load4(const void* q, long i) {
+  return *reinterpret_cast<const f32x4*>(static_cast<const float*>(q) + i);
+}
+
+// an epilogue's per-channel inputs (the packed ones are padded with zeros to co_pad channels)
+struct SplitCols {
+  f32x4 bias, winv, alpha, inv_alpha, alpha2, inv_alpha2;
+  __device__ __forceinline__ void load(const HiftConv& p, int c) {
+    winv = load4(p.winv, c);
+    bias = load4(p.winv, p.co_pad + c);
+    if (p.snake_out) {
+      alpha = load4(p.alpha, c);
+      inv_alpha = load4(p.inv_alpha, c);
+    }
+    if (p.out2) {
+      alpha2 = load4(p.alpha2, c);
+      inv_alpha2 = load4(p.inv_alpha2, c);
+    }
+  }
+};
+
+// the rows an epilogue adds to channels c .. c + 3 of output row `row`
+struct SplitAdds {
+  f32x4 add, acc;
+  __device__ __forceinline__ void load(const HiftConv& p, long row, int c) {
+    if (p.add) add = load4(p.add, row * p.ld_add + c);
+    if (p.mode != HIFT_ACC_WRITE) acc = load4(p.accin, row * p.ldo + c);
+  }
+};
+
+// the epilogue of channels c .. c + 3 of one row: unscale, bias, residual, resblock sum, Snakes; m1, m2:
+// raised to the largest finite magnitudes written to out and out2
+__device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& cols,
+                                            const SplitAdds& in, long row, int c, const f32x4& acc,
+                                            float inv, float& m1, float& m2) {
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = fmaf(acc[e] * inv, cols.winv[e], cols.bias[e]);
+  const long i = row * p.ldo + c;
+  if (p.add) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] + in.add[e];
+  }
+  if (p.mode != HIFT_ACC_WRITE) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = in.acc[e] + v[e];
+    if (p.mode == HIFT_ACC_ADD_DIV) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = v[e] / p.div;
+    }
+  }
+  if (p.snake_out) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = snake(v[e], cols.alpha[e], cols.inv_alpha[e]);
+  }
+  if (p.amax_out) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m1 = fmaxf(m1, finite_abs(v[e]));
+  }
+  *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + i) = v;
+  if (p.out2) {
+    f32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = snake(v[e], cols.alpha2[e], cols.inv_alpha2[e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m2 = fmaxf(m2, finite_abs(w[e]));
+    *reinterpret_cast<f32x4*>(static_cast<float*>(p.out2) + i) = w;
+  }
+}
+
+// WC x WR waves; each wave MC x MR tiles of 32 channels x 32 rows.  NS weight stages, NI passes of
+// window loads (kThreads / 8 rows each).
+template <int WC_, int WR_, int MC_, int MR_, int NS_, int NI_>
+struct Cfg {
+  static constexpr int WC = WC_, WR = WR_, MC = MC_, MR = MR_, NS = NS_, NI = NI_;
+  static constexpr int kWaves = WC * WR, kThreads = 64 * kWaves;
+  static constexpr int TC = 32 * MC * WC, TR = 32 * MR * WR;
+  static constexpr int kWin = NI * kThreads / 8;             // window rows
+  static constexpr int kWBytes = TC * kRowBytes;             // one weight stage
+  static constexpr int kCopies = kWBytes / 1024 / kWaves;    // weight copies per wave and step
+  static constexpr int kXOff = NS * kWBytes;
+  static constexpr int kInfoOff = kXOff + (kWin + 1) * kRowBytes;  // + the zero row
+  static constexpr int kPitch = 32 * MC + 4;                 // staged epilogue row, in floats
+  static constexpr int kStage = 32 * kPitch * 4;             // per wave
+  static constexpr int kLds = kInfoOff + TR * 20;
+  static constexpr int kMinWaves = kThreads < 256 ? 1 : NI <= 3 ? 4 : 3;  // per SIMD, no spills
+  static_assert(kWBytes % (1024 * kWaves) == 0, "weight copies");
+  static_assert(kStage * kWaves <= kInfoOff, "the epilogue stages in the operand space");
+};
+
+template <class C>
+__global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
+    const HiftConv p, const HiftDocs* __restrict__ docs) {
+  __shared__ __attribute__((aligned(1024))) char smem[C::kLds];
+  char* sX = smem + C::kXOff;
+  // per tile row: window row of the first tap (of input position 0 for up > 1), position and
+  // document; then the inverse input scale
+  int4* sInfo = reinterpret_cast<int4*>(smem + C::kInfoOff);
+  float* sInv = reinterpret_cast<float*>(smem + C::kInfoOff + C::TR * 16);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wc = wave % C::WC, wr = wave / C::WC;
+  const int li = lane & 31, hl = lane >> 5;
+  const int r0 = blockIdx.x * C::TR;
+  // the document table in one round of loads (documents past 63: looked up in memory)
+  const int n_docs = docs->n;
+  const int ta = docs->a[lane], tb = docs->b[lane];
+  int rows_out, in_total, d0, in0, out0, out1;
+  if (n_docs < 64) {
+    rows_out = __builtin_amdgcn_readlane(tb, n_docs);
+    in_total = __builtin_amdgcn_readlane(ta, n_docs);
+    if (r0 >= rows_out) return;
+    d0 = __builtin_popcountll(__ballot(lane < n_docs && tb <= r0)) - 1;
+    in0 = __builtin_amdgcn_readlane(ta, d0);
+    out0 = __builtin_amdgcn_readlane(tb, d0);
+    out1 = __builtin_amdgcn_readlane(tb, d0 + 1);
+  } else {
+    rows_out = docs->b[n_docs];
+    in_total = docs->a[n_docs];
+    if (r0 >= rows_out) return;
+    d0 = doc_of(docs->b, n_docs, r0);
+    in0 = docs->a[d0];
+    out0 = docs->b[d0];
+    out1 = docs->b[d0 + 1];
+  }
+  const bool one_doc = min(r0 + C::TR, rows_out) <= out1;  // of the tile's rows
+  const int co0 = blockIdx.y * C::TC;
+  const int chunks = p.cin_pad / 32;
+  const int k = p.k;
+
+  // weight copies: step (chunk, tap) is a contiguous block of co_pad rows
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+  const char* wbase = static_cast<const char*>(p.wsplit) + (long)co0 * kRowBytes;
+  const long wstep = (long)p.co_pad * kRowBytes;
+  const uint32_t wlane = (uint32_t)(wave * C::kCopies * 1024 + lane * 16);
+  const int steps = chunks * k;
+  auto issue_w = [&](int s, int stage) {
+    const char* src = wbase + (long)s * wstep;
+    const uint32_t dst = lds0 + (uint32_t)stage * C::kWBytes + wave * C::kCopies * 1024;
+#pragma unroll
+    for (int i = 0; i < C::kCopies; ++i) lds_dma16(src, wlane + i * 1024, dst + i * 1024);
+  };
+
+#pragma unroll
+  for (int s = 0; s < C::NS - 1; ++s)
+    if (s < steps) issue_w(s, s);
+
+  // the window starts at the first input row any tap of the tile's first row reads
+  const int u0 = r0 - out0 - p.pad;
+  const int win0 = in0 + (u0 > 0 ? u0 / p.up : 0);
+  // scale of the first document, which is that of every row of most tiles
+  const int f0 = scale_field(doc_amax(p.amax_in, d0, lane));
+  auto row_field = [&](int d) {
+    return d == d0 ? f0 : scale_field(amax_serial(p.amax_in, d));
+  };
+  for (int t = tid; t < C::TR; t += C::kThreads) {
+    const int r = r0 + t;
+    int4 v{0, -(1 << 29), d0, 0};  // rows past the end read the zero row at every tap
+    float inv = 1.0f;
+    if (r < rows_out) {
+      const int d = one_doc ? d0 : doc_of(docs->b, n_docs, r);
+      v.x = (one_doc ? in0 : docs->a[d]) - win0;
+      v.y = r - (one_doc ? out0 : docs->b[d]);
+      v.z = d;
+      inv = field_to_float(254 - row_field(d));
+    }
+    sInfo[t] = v;
+    sInv[t] = inv;
+  }
+  if (tid < 8) *reinterpret_cast<f32x4*>(sX + C::kWin * kRowBytes + tid * 16) = f32x4{0, 0, 0, 0};
+
+  // window loads: pass i, thread tid -> window row i * kThreads / 8 + tid / 8, channels 4 (tid % 8)
+  const float* X = static_cast<const float*>(p.x) + (tid & 7) * 4;
+  long xoff[C::NI];
+  float xs[C::NI];
+#pragma unroll
+  for (int i = 0; i < C::NI; ++i) {
+    const int row = min(win0 + i * (C::kThreads / 8) + (tid >> 3), in_total - 1);
+    xoff[i] = (long)row * p.ldx;
+    // (rows of a window past the tile's own may belong to another document: nothing reads them)
+    xs[i] = field_to_float(one_doc ? f0 : row_field(doc_of(docs->a, n_docs, row)));
+  }
+  f32x4 xr[C::NI];
+  auto fetch_x = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < C::NI; ++i) xr[i] = *reinterpret_cast<const f32x4*>(X + xoff[i] + c * 32);
+  };
+  auto stash_x = [&]() {
+#pragma unroll
+    for (int i = 0; i < C::NI; ++i) {
+      f32x4 v = xr[i];
+      if (p.pro == HIFT_PRO_LEAKY) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * p.slope;
+      }
+      f16x4 hi, lo;
+      split4(v, xs[i], hi, lo);
+      const int row = i * (C::kThreads / 8) + (tid >> 3);
+      char* dst = sX + row * kRowBytes + (tid & 1) * 8;
+      *reinterpret_cast<f16x4*>(dst + 16 * swz(row, (tid & 7) >> 1)) = hi;
+      *reinterpret_cast<f16x4*>(dst + 16 * swz(row, 4 + ((tid & 7) >> 1))) = lo;
+    }
+  };
+
+  f32x16 acc[C::MC][C::MR];
+#pragma unroll
+  for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+    for (int b = 0; b < C::MR; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.0f;
+
+  fetch_x(0);
+  // the epilogue's per-channel inputs, loaded here so that nothing waits for them there
+  constexpr int LPR = 8 * C::MC;              // lanes per staged output row
+  const int cl = (lane % LPR) * 4;            // channel within the wave's columns
+  const int c4 = co0 + wc * C::MC * 32 + cl;
+  const bool live_c = c4 < p.cout;
+  SplitCols cols;
+  cols.load(p, live_c ? c4 : 0);
+  __syncthreads();  // the row table
+  // this lane's rows: window row and input position of tap 0; up > 1 walks (position, remainder)
+  int wrow0[C::MR], q0[C::MR], rem0[C::MR];
+#pragma unroll
+  for (int b = 0; b < C::MR; ++b) {
+    const int4 v = sInfo[(wr * C::MR + b) * 32 + li];
+    const int u = v.y - p.pad;
+    int q = u, rem = 0;
+    if (p.up > 1) {
+      q = u >= 0 ? u / p.up : -((-u + p.up - 1) / p.up);
+      rem = u - q * p.up;
+    }
+    q0[b] = q;
+    rem0[b] = rem;
+    wrow0[b] = v.x + q;
+  }
+
+  // Two fragment buffers: the reads of k-step ks + 1 are in flight while the MFMAs of ks run.  A
+  // step's second k-step runs after the barrier that publishes the next step, over that step's
+  // first reads.  In an LDS row the 16-byte chunk of k-step ks (hi, then lo) sits at byte
+  // (16 (hl ^ rot)) ^ 32 ks (^ 64 for lo), rot = (row / 2) % 8.
+  f16x8 wh[2][C::MC], wl[2][C::MC], xh[2][C::MR], xl[2][C::MR];
+  uint32_t woff[C::MC];
+#pragma unroll
+  for (int a = 0; a < C::MC; ++a) {
+    const int row = (wc * C::MC + a) * 32 + li;
+    woff[a] = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
+  }
+  uint32_t xoff_l[C::MR];
+  auto load = [&](int buf, int ks, const char* sW) {
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a) {
+      wh[buf][a] = *reinterpret_cast<const f16x8*>(sW + (woff[a] ^ (32 * ks)));
+      wl[buf][a] = *reinterpret_cast<const f16x8*>(sW + (woff[a] ^ (32 * ks + 64)));
+    }
+#pragma unroll
+    for (int b = 0; b < C::MR; ++b) {
+      xh[buf][b] = *reinterpret_cast<const f16x8*>(sX + (xoff_l[b] ^ (32 * ks)));
+      xl[buf][b] = *reinterpret_cast<const f16x8*>(sX + (xoff_l[b] ^ (32 * ks + 64)));
+    }
+  };
+  auto mma = [&](int buf) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wl[buf][a], xh[buf][b], acc[a][b]);
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wh[buf][a], xl[buf][b], acc[a][b]);
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wh[buf][a], xh[buf][b], acc[a][b]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  int s = 0, stage_s = 0;
+  for (int c = 0; c < chunks; ++c) {
+    int q[C::MR], rem[C::MR], wrow[C::MR];
+#pragma unroll
+    for (int b = 0; b < C::MR; ++b) { q[b] = q0[b]; rem[b] = rem0[b]; wrow[b] = wrow0[b]; }
+    if (c > 0) {
+      // Every wave has read the previous window: a barrier alone does not wait for a wave's reads
+      // in flight, and the window is written right after it.
+      wait_lgkm0();
+      __syncthreads();
+      mma(1);
+    }
+    stash_x();
+    for (int j = 0; j < k; ++j, ++s) {
+      // this wave's copies of step s have landed (the later steps' may be in flight), then everyone's
+      if (s + C::NS - 2 < steps)
+        wait_vm<(C::NS - 2) * C::kCopies>();
+      else
+        wait_vm<0>();
+      wait_lgkm0();  // and this wave's reads of the stage the next copies overwrite
+      __syncthreads();
+      if (s + C::NS - 1 < steps) issue_w(s + C::NS - 1, stage_s == 0 ? C::NS - 1 : stage_s - 1);
+      if (j == 0 && c + 1 < chunks) fetch_x(c + 1);
+
+      const char* sW = smem + stage_s * C::kWBytes;
+      stage_s = stage_s == C::NS - 1 ? 0 : stage_s + 1;
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b) {
+        const bool ok = q[b] >= 0 && (unsigned)wrow[b] < (unsigned)C::kWin;
+        const int row = ok ? wrow[b] : C::kWin;
+        xoff_l[b] = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
+        // next tap's input row
+        if (p.up > 1) {
+          rem[b] += 1;
+          const int step = rem[b] == p.up ? 1 : 0;
+          rem[b] = step ? 0 : rem[b];
+          q[b] += step;
+          wrow[b] += step;
+        } else {
+          q[b] += p.dil;
+          wrow[b] += p.dil;
+        }
+      }
+      load(0, 0, sW);
+      if (j > 0) mma(1);
+      load(1, 1, sW);
+      mma(0);
+    }
+  }
+  mma(1);
+  wait_vm<0>();
+  wait_lgkm0();
+  __syncthreads();  // the operand space becomes the waves' staging space
+
+  // Epilogue: lane l holds row l % 32 and, in register group g, channels 8 g + 4 (l / 32) + 0..3.
+  // Each wave stages 32 rows at a time and reads them back row-major, so loads and stores are
+  // whole 128-byte (256-byte) runs of a row.
+  float* stage = reinterpret_cast<float*>(smem + wave * C::kStage);
+  constexpr int RPI = 64 / LPR, NP = 32 / RPI;  // rows a pass, passes
+  float m1 = 0.0f, m2 = 0.0f;                   // largest finite magnitudes written
+  const int sub = blockIdx.x + blockIdx.y;
+#pragma unroll
+  for (int b = 0; b < C::MR; ++b) {
+    const int t0 = (wr * C::MR + b) * 32 + lane / LPR;
+    SplitAdds in[NP];  // in flight while the block is staged (out may be the residual itself)
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int t = t0 + i * RPI;
+      if (r0 + t < rows_out && live_c)
+        in[i].load(p, p.reflect ? (long)r0 + t + sInfo[t].z + 1 : r0 + t, c4);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2],
+                      acc[a][b][4 * g + 3]};
+        *reinterpret_cast<f32x4*>(stage + li * C::kPitch + a * 32 + g * 8 + hl * 4) = v;
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int t = t0 + i * RPI;
+      const int r = r0 + t;
+      if (r >= rows_out || !live_c) continue;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(stage + (i * RPI + lane / LPR) * C::kPitch + cl);
+      const int4 info = sInfo[t];
+      const float inv = sInv[t];
+      const long row = p.reflect ? (long)r + info.z + 1 : r;
+      float a1 = 0.0f, a2 = 0.0f;
+      split_store(p, cols, in[i], row, c4, v, inv, a1, a2);
+      // reflection padding (1, 0): row 0 of the document repeats the result's row 1
+      if (p.reflect && info.y == 1) {
+        SplitAdds first;
+        first.load(p, (long)r - 1 + info.z, c4);
+        split_store(p, cols, first, (long)r - 1 + info.z, c4, v, inv, a1, a2);
+      }
+      if (one_doc) {
+        m1 = fmaxf(m1, a1);
+        m2 = fmaxf(m2, a2);
+      } else {
+        if (p.amax_out) raise_amax(p.amax_out, info.z, sub, a1);
+        if (p.amax_out2) raise_amax(p.amax_out2, info.z, sub, a2);
+      }
+    }
+  }
+  if (one_doc && (p.amax_out || p.amax_out2)) {
+    float* wmax = sInv;  // the row scales are read
+    m1 = wave_max(m1);
+    m2 = wave_max(m2);
+    __syncthreads();
+    if (lane == 0) {
+      wmax[wave] = m1;
+      wmax[4 + wave] = m2;
+    }
+    __syncthreads();
+    if (tid < 2) {
+      uint32_t* slot = tid == 0 ? p.amax_out : p.amax_out2;
+      float m = 0.0f;
+#pragma unroll
+      for (int w = 0; w < C::kWaves; ++w) m = fmaxf(m, wmax[tid * 4 + w]);
+      if (slot) raise_amax(slot, d0, sub, m);
+    }
+  }
+}
+
+// One wave per output channel of [co_pad][k][cin] weights: the row's scale from its largest finite
+// weight, then both halves at [chunk][tap][co][64 f16], the 16-byte chunks of a row in their LDS
+// order; inv[co] = the inverse scale, inv[co_pad + co] = the bias (zero past cout).
+__global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict__ w,
+                                                        const float* __restrict__ bias, int cout,
+                                                        int co_pad, int k, int cin,
+                                                        f16* __restrict__ dst,
+                                                        float* __restrict__ inv) {
+  const int co = blockIdx.x, lane = threadIdx.x;
+  const float* row = w + (long)co * k * cin;
+  const int n = k * cin;
+  float m = 0.0f;
+  for (int i = lane; i < n; i += 64) m = fmaxf(m, finite_abs(row[i]));
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  const int f = scale_field(__float_as_uint(m));
+  const float s = field_to_float(f);
+  if (lane == 0) {
+    inv[co] = field_to_float(254 - f);
+    inv[co_pad + co] = co < cout ? bias[co] : 0.0f;
+  }
+  for (int i = lane; i < n / 4; i += 64) {
+    const int tap = i * 4 / cin, c = i * 4 - tap * cin;
+    f16x4 hi, lo;
+    split4(*reinterpret_cast<const f32x4*>(row + i * 4), s, hi, lo);
+    f16* out = dst + (((long)(c / 32) * k + tap) * co_pad + co) * 64 + (c & 4);
+    const int unit = (c & 31) >> 3;
+    *reinterpret_cast<f16x4*>(out + 8 * swz(co, unit)) = hi;
+    *reinterpret_cast<f16x4*>(out + 8 * swz(co, unit + 4)) = lo;
+  }
+}
+
+__global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ x, int n) {
+  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i < n) *reinterpret_cast<uint4*>(x + i) = uint4{0, 0, 0, 0};
+}
+
+bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
+
+template <class C>
+hipError_t launch(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
+  static_assert(C::kLds <= 160 * 1024, "LDS");
+  const dim3 grid((p.rows_out + C::TR - 1) / C::TR, (p.cout + C::TC - 1) / C::TC);
+  hipLaunchKernelGGL(split_conv_kernel<C>, grid, dim3(C::kThreads), 0, stream, p, docs);
+  return hipGetLastError();
+}
+
+// input rows a tile of TR output rows reads: its rows and the left context
+int window_rows(const HiftConv& p, int tr) {
+  return (tr - 1) / p.up + 2 + ((p.k - 1) * p.dil + p.up - 1) / p.up;
+}
+
+// the shape with the window passes the launch needs
+template <int WC, int WR, int MC, int MR, int NS, int P1, int P2, int P3>
+hipError_t launch_win(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
+  const int need = window_rows(p, 32 * MR * WR), per = 8 * WC * WR;
+  if (need <= P1 * per) return launch<Cfg<WC, WR, MC, MR, NS, P1>>(p, docs, stream);
+  if (need <= P2 * per) return launch<Cfg<WC, WR, MC, MR, NS, P2>>(p, docs, stream);
+  if (need <= P3 * per) return launch<Cfg<WC, WR, MC, MR, NS, P3>>(p, docs, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+bool hift_split_eligible(const HiftConv& p) {
+  return p.stride == 1 && p.cin_pad % 32 == 0 && p.up >= 1 && p.dil >= 1 &&
+         (p.up == 1 || p.dil == 1) && p.pad == (p.k - 1) * p.dil && p.pad <= kMaxHalo &&
+         (p.pro == HIFT_PRO_NONE || (p.slope >= -1.0f && p.slope <= 1.0f));
+}
+
+size_t hift_split_bytes(int co_pad, int k, int cin) {
+  return (size_t)(cin / 32) * k * co_pad * kRowBytes;
+}
+
+hipError_t hift_pack_split(const float* w, const float* bias, int cout, int co_pad, int k, int cin,
+                           void* dst, float* inv, hipStream_t stream) {
+  hipLaunchKernelGGL(pack_split_kernel, dim3(co_pad), dim3(64), 0, stream, w, bias, cout, co_pad, k,
+                     cin, static_cast<f16*>(dst), inv);
+  return hipGetLastError();
+}
+
+hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream) {
+  if (n <= 0) return hipSuccess;
+  if (n % 4 != 0 || !aligned16(x)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(zero_u32_kernel, dim3((n / 4 + 255) / 256), dim3(256), 0, stream, x, n);
+  return hipGetLastError();
+}
+
+hipError_t hift_conv_split(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
+  if (p.rows_out <= 0) return hipSuccess;
+  if (!hift_split_eligible(p) || !p.wsplit || !p.winv || !p.amax_in || p.co_pad % 64 != 0 ||
+      p.ldx % 4 != 0 || p.ldo % 4 != 0 || (p.add && p.ld_add % 4 != 0) ||
+      !aligned16(p.x) || !aligned16(p.out) || !aligned16(p.add) || !aligned16(p.accin) ||
+      !aligned16(p.out2) || !aligned16(p.wsplit) || !aligned16(p.winv) ||
+      // channels go four at a time: a partial last group writes zeros into the row's padding and
+      // has no other row or parameter to read
+      (p.cout % 4 != 0 && ((p.cout + 3) / 4 * 4 > p.ldo || p.add || p.snake_out || p.out2 ||
+                           p.mode != HIFT_ACC_WRITE)) ||
+      (long)p.co_pad * kRowBytes >= (1L << 31))
+    return hipErrorInvalidValue;
+  // FCV_HIFT_TILE = 32 or 64 forces a tile: a test hook, both must give the same bits
+  const char* forced = std::getenv("FCV_HIFT_TILE");
+  const int force = forced ? std::atoi(forced) : 0;
+  const long tiles64 = (long)((p.rows_out + 63) / 64) * ((p.cout + 63) / 64);
+  const bool small = force ? force == 32 : tiles64 < kSmallBelow;
+  if (p.cout <= 32)
+    return small ? launch_win<1, 1, 1, 1, 8, 4, 8, 12>(p, docs, stream)
+                 : launch_win<1, 4, 1, 1, 3, 2, 5, 6>(p, docs, stream);
+  return small ? launch_win<2, 1, 1, 1, 8, 3, 4, 6>(p, docs, stream)
+               : launch_win<2, 2, 1, 1, 3, 2, 3, 4>(p, docs, stream);
+}
+
+}  // namespace fcv

@@ -71,6 +71,7 @@ class HiFTVocoder:
         self._cdims = self._make_dims()
         self._handle: int | None = None
         self._keep: list[torch.Tensor] = []
+        self._packed: torch.Tensor | None = None
         # extra handles over the same weight table, for request groups in flight together:
         # [handle, workspace, stream]
         self._lanes: list[list] = []
@@ -199,6 +200,14 @@ class HiFTVocoder:
         self._handle = handle.value
         self._keep = keep
         self._ptrs = arr
+        # the split f16 weights of the vocoder's convolutions, shared by every lane's handle
+        need = int(self._lib.fcv_hift_packed_bytes(handle))
+        if need:
+            self._packed = torch.empty(need, dtype=torch.uint8, device=dev)
+            stream = torch.cuda.current_stream(dev)
+            _lib.check(self._lib.fcv_hift_pack_weights(handle, self._packed.data_ptr(), need,
+                                                       stream.cuda_stream))
+            stream.synchronize()  # other streams' calls read them
 
     def __del__(self):
         try:
@@ -221,6 +230,9 @@ class HiFTVocoder:
                 h = _lib.c_void_p()
                 _lib.check(self._lib.fcv_hift_create(self._cdims, self._ptrs, len(self._ptrs), h))
                 handle = h.value
+                if self._packed is not None:
+                    _lib.check(self._lib.fcv_hift_use_packed(h, self._packed.data_ptr(),
+                                                             self._packed.numel()))
             # [handle, workspace, stream, buffer sets by capacity]
             self._lanes.append([handle, None, group_stream(self.device, len(self._lanes)), {}])
         return self._lanes[i]

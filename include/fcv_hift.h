@@ -77,6 +77,17 @@ int fcv_hift_create(const FcvHiftDims* dims, const void* const* weights, int32_t
                     FcvHift** out);
 int fcv_hift_destroy(FcvHift* hift);
 
+/* Split weights (optional): the causal unit-stride convolutions with input channels a multiple of
+ * 32 then run on the f16 matrix cores at fp32 accuracy, both operands held as two f16 halves
+ * (without them, and for the other convolutions, on the fp32 matrix cores).  fcv_hift_pack_weights
+ * computes them on `stream` into caller-owned memory of fcv_hift_packed_bytes (0: no such
+ * convolution in this shape), 256-byte aligned, which must outlive the handle; it is called before
+ * the handle's first inference.  fcv_hift_use_packed gives another handle over the same weights
+ * the memory that was filled. */
+size_t fcv_hift_packed_bytes(const FcvHift* hift);
+int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t stream);
+int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes);
+
 /* Waveform samples produced for a document of `frames` Mel frames:
  * finalize != 0: frames * upsample_scale (480 for CosyVoice3); otherwise the last
  * 3 + conv_pre_look_right + 1 frames are right context and (frames - 8) * 480 samples come out

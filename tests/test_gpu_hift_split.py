@@ -1,0 +1,113 @@
+"""The vocoder's split-f16 convolutions (two f16 halves per fp32 operand, hift_split.hip) against
+the fp32 matrix-core convolutions, which a handle without packed weights runs: every tile, tap
+window and document boundary, activations far outside the f16 range, and non-finite input.
+
+Bound: an operand's halves hold 22 bits (2^-22 per product) and both kernels accumulate K <= 8192
+terms in fp32, so one convolution differs by about 1e-6; the vocoder's waveform carries the
+difference of some 80 convolutions (2e-5 measured on either side against 64 bits, so 1e-4, the bar
+of the oracle comparison, with the two errors added).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tests.gpu_helpers import rel_l2, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def _pair(fcv, monkeypatch, gain=1.0, dims=None):
+    """(vocoder with split weights, vocoder on the fp32 kernels), the same seeded weights; `gain`
+    scales conv_pre and the source convolutions, and with them every later activation, while the
+    last convolution's gain undoes it."""
+    dims = dims or fcv.synthetic.HiFTDims()
+    sd = fcv.synthetic.random_hift_state_dict(dims, seed=91)
+    g = ".parametrizations.weight.original0"
+    for name in sd:
+        if name.startswith("conv_pre") or name.startswith("source_downs"):
+            sd[name] = sd[name] * (gain if not name.endswith("original1") else 1.0)
+        if name.endswith("alpha"):
+            sd[name] = sd[name] / gain
+        if name.endswith("bias") and (name.startswith("ups") or "resblocks" in name):
+            sd[name] = sd[name] * gain
+    sd["conv_post" + g] = sd["conv_post" + g] / gain
+    buf = fcv.synthetic.random_hift_buffers(dims, max_samples=480 * 140, seed=92)
+    out = []
+    for split in (True, False):
+        v = fcv.HiFTVocoder(dims, device="cuda:0", buffers=buf)
+        v.load_reference_state_dict(sd)
+        if not split:
+            monkeypatch.setattr(v._lib, "fcv_hift_packed_bytes", lambda h: 0)
+        v.finalize_weights()
+        assert (v._packed is not None) == split
+        out.append(v)
+    monkeypatch.undo()
+    return out
+
+
+# frames per request: single rows of a tile, documents shorter than a tap window, tile edges
+# (8, 40 and 120 rows a frame in the three stages against 32- and 64-row tiles), many documents
+@pytest.mark.parametrize("frames", [[1], [3, 1, 2, 1], [8, 9], [16, 40, 1, 33], [131], [2] * 70],
+                         ids=lambda f: f"{len(f)}x{max(f)}")
+@pytest.mark.parametrize("tile", ["32", "64"])
+def test_split_matches_fp32(fcv, monkeypatch, frames, tile):
+    split, fp32 = _pair(fcv, monkeypatch)
+    g = torch.Generator().manual_seed(93)
+    mels = [torch.randn(80, n, generator=g).cuda() for n in frames]
+    say(f"[split] {frames} tile {tile}")
+    monkeypatch.setenv("FCV_HIFT_TILE", tile)
+    got = split.inference_batched(mels, graph=False)
+    ref = fp32.inference_batched(mels, graph=False)
+    err = rel_l2(torch.cat([a.reshape(-1) for a in got]), torch.cat([a.reshape(-1) for a in ref]))
+    say(f"[split] rel_l2 {err:.2e}")
+    assert err <= 1e-4
+
+
+@pytest.mark.parametrize("gain", [2.0 ** 24, 2.0 ** -40], ids=["large", "small"])
+def test_split_holds_the_fp32_range(fcv, monkeypatch, gain):
+    """Activations of 10^7 and 10^-12, past what f16 holds: the per-document scale keeps them."""
+    split, fp32 = _pair(fcv, monkeypatch, gain)
+    g = torch.Generator().manual_seed(94)
+    mels = [torch.randn(80, n, generator=g).cuda() for n in (20, 7)]
+    got, ref = split.inference_batched(mels), fp32.inference_batched(mels)
+    for a, b in zip(got, ref):
+        assert torch.isfinite(b).all() and float(b.std()) > 1e-4
+        err = rel_l2(a, b)
+        say(f"[split] gain {gain:.1e} rel_l2 {err:.2e}")
+        assert err <= 1e-4
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_non_finite_frame_stays_causal(fcv, monkeypatch, value):
+    """A non-finite Mel frame changes nothing before its convolutions' right context reaches it
+    (4 frames), and nothing of the other documents, as on the fp32 kernels."""
+    split, _ = _pair(fcv, monkeypatch)
+    g = torch.Generator().manual_seed(95)
+    mels = [torch.randn(80, n, generator=g).cuda() for n in (30, 12)]
+    bad = [mels[0].clone(), mels[1]]
+    bad[0][:, 20] = value
+    ref, got = split.inference_batched(mels), split.inference_batched(bad)
+    keep = (20 - 4 - 1) * 480
+    assert torch.isfinite(ref[0]).all()
+    assert rel_l2(got[0][:, :keep], ref[0][:, :keep]) <= 1e-5
+    assert torch.equal(got[1], ref[1])
+
+
+def test_concurrent_groups_repeat_bit_for_bit(fcv, monkeypatch):
+    """Two request groups sharing the GPU: forty passes give the same bits (a window overwritten
+    while another wave still reads it shows only under such load)."""
+    split, _ = _pair(fcv, monkeypatch)
+    g = torch.Generator().manual_seed(96)
+    mels = [torch.randn(80, n, generator=g).cuda() for n in (139, 120, 131)]
+    ref = split.inference_batched(mels)
+    for _ in range(40):
+        got = split.inference_batched(mels)
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
