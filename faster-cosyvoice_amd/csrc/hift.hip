@@ -42,9 +42,9 @@ template <typename T>
 __device__ __forceinline__ T elu(T x) { return x > T(0) ? x : T(expm1(x)); }
 
 // epilogue of one output element (row, channel c) from its accumulator value; m: raised to the
-// largest finite magnitude written to out (fp32)
+// largest finite magnitudes written to out and to the Snake output (fp32)
 template <typename T>
-__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, T acc, float& m) {
+__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, T acc, float2& m) {
   T v = acc + static_cast<const T*>(p.bias)[c];
   if constexpr (sizeof(T) == 8) {
     if (p.elu) v = elu(v);
@@ -55,8 +55,12 @@ __device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, 
   if (p.mode == HIFT_ACC_ADD_DIV) v = (static_cast<const T*>(p.accin)[i] + v) / T(p.div);
   if constexpr (sizeof(T) == 4) {
     if (p.snake_out) v = snake(v, p.alpha[c], p.inv_alpha[c]);
-    if (p.out2) static_cast<float*>(p.out2)[i] = snake(v, p.alpha2[c], p.inv_alpha2[c]);
-    m = fmaxf(m, finite_abs(v));
+    if (p.n_snakes) {
+      const float w = snake(v, p.snakes[0].alpha[c], p.snakes[0].inv_alpha[c]);
+      p.snakes[0].out[i] = w;
+      m.y = fmaxf(m.y, finite_abs(w));
+    }
+    m.x = fmaxf(m.x, finite_abs(v));
   }
   static_cast<T*>(p.out)[i] = v;
 }
@@ -66,7 +70,7 @@ __device__ __forceinline__ float4 ld4f(const float* q) { return *reinterpret_cas
 // conv_store1 for the four consecutive fp32 channels c .. c + 3 of one row, with 16-byte loads
 // and stores (same operations in the same order, so the results are bit-identical)
 __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, const f32x4& acc,
-                                            float& m) {
+                                            float2& m) {
   const float4 b = ld4f(static_cast<const float*>(p.bias) + c);
   float v[4] = {acc[0] + b.x, acc[1] + b.y, acc[2] + b.z, acc[3] + b.w};
   const long i = row * p.ldo + c;
@@ -85,14 +89,17 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
 #pragma unroll 1
     for (int e = 0; e < 4; ++e) v[e] = snake(v[e], p.alpha[c + e], p.inv_alpha[c + e]);
   }
-  if (p.out2) {
+  if (p.n_snakes) {
+    const HiftConv::Snake& q = p.snakes[0];
     float w[4];
 #pragma unroll 1
-    for (int e = 0; e < 4; ++e) w[e] = snake(v[e], p.alpha2[c + e], p.inv_alpha2[c + e]);
-    *reinterpret_cast<float4*>(static_cast<float*>(p.out2) + i) = float4{w[0], w[1], w[2], w[3]};
+    for (int e = 0; e < 4; ++e) w[e] = snake(v[e], q.alpha[c + e], q.inv_alpha[c + e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m.y = fmaxf(m.y, finite_abs(w[e]));
+    *reinterpret_cast<float4*>(q.out + i) = float4{w[0], w[1], w[2], w[3]};
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) m = fmaxf(m, finite_abs(v[e]));
+  for (int e = 0; e < 4; ++e) m.x = fmaxf(m.x, finite_abs(v[e]));
   *reinterpret_cast<float4*>(static_cast<float*>(p.out) + i) = float4{v[0], v[1], v[2], v[3]};
 }
 
@@ -100,7 +107,7 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
 //   fp32: channels cb + 4 lg + e;  fp64: channels cb + 4 e + lg  (e = 0..3)
 template <typename T>
 __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
-                           const typename Vec4<T>::type& acc, float& m) {
+                           const typename Vec4<T>::type& acc, float2& m) {
   if constexpr (sizeof(T) == 4) {
     if (p.vec4 && cb + 4 * lg + 3 < p.cout) {
       conv_store4(p, row, cb + 4 * lg, acc, m);
@@ -122,8 +129,8 @@ __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
 // in the same order with the same lane/slot -> k rule at both sizes, so the tile size does not
 // change a result.
 template <typename T, int BK, int TS>
-__global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
-                                                        const HiftDocs* __restrict__ docs) {
+__global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
+  const HiftDocs* __restrict__ docs = p.docs;
   using VT = typename Vec4<T>::type;
   constexpr int PITCH = BK + 4;  // LDS row pitch in elements (conflict-free 16-byte reads)
   constexpr int G = BK / 16;
@@ -248,7 +255,7 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
   // D[i = channel][j = row]: lane holds row li and four channels of each 16x16 tile
   const int tile_doc = doc_of(docs->b, n_docs, r0);
   const bool one_doc = min(r0 + TS, rows_out) <= docs->b[tile_doc + 1];
-  float tile_max = 0.0f;
+  float2 tile_max{0.0f, 0.0f};
 #pragma unroll
   for (int b = 0; b < NQ; ++b) {
     const int rr = r0 + wt * (TS / 2) + b * 16 + li;
@@ -256,7 +263,7 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
     const int d = doc_of(docs->b, n_docs, rr);
     const int pp = rr - docs->b[d];
     const long row_w = p.reflect ? (long)docs->b[d] + d + 1 + pp : rr;
-    float m = 0.0f;
+    float2 m{0.0f, 0.0f};
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
       const int cb = co0 + wc * (TS / 2) + a * 16;
@@ -264,19 +271,51 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p,
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
       if (p.reflect && pp == 1) conv_store<T>(p, (long)docs->b[d] + d, cb, lg, acc[a][b], m);
     }
-    if (sizeof(T) == 4 && p.amax_out) {
-      if (one_doc) tile_max = fmaxf(tile_max, m);
-      else raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m);
+    if constexpr (sizeof(T) == 4) {
+      if (one_doc) {
+        tile_max.x = fmaxf(tile_max.x, m.x);
+        tile_max.y = fmaxf(tile_max.y, m.y);
+      } else {
+        if (p.amax_out) raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m.x);
+        if (p.snakes[0].amax) raise_amax(p.snakes[0].amax, d, blockIdx.x + blockIdx.y, m.y);
+      }
     }
   }
-  if (sizeof(T) == 4 && p.amax_out && one_doc) {
+  if constexpr (sizeof(T) == 4) {
+    if (one_doc && (p.amax_out || p.snakes[0].amax)) {
+      __shared__ float wmax[2][4];
+      tile_max.x = wave_max(tile_max.x);
+      tile_max.y = wave_max(tile_max.y);
+      if (lane == 0) {
+        wmax[0][wave] = tile_max.x;
+        wmax[1][wave] = tile_max.y;
+      }
+      __syncthreads();
+      if (tid < 2) {
+        uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[0].amax;
+        const float m = fmaxf(fmaxf(wmax[tid][0], wmax[tid][1]), fmaxf(wmax[tid][2], wmax[tid][3]));
+        if (slot) raise_amax(slot, tile_doc, blockIdx.x + blockIdx.y, m);
+      }
+    }
+  }
+}
+
+// a workgroup of 256 threads at elements first.. (q a row) raises its rows' documents by each
+// thread's m (i: the thread's element)
+__device__ __forceinline__ void raise_rows_amax(uint32_t* amax, float m, long first, long i,
+                                                long total, int q,
+                                                const HiftDocs* __restrict__ docs) {
+  if (!amax) return;
+  const int d0 = doc_of(docs->b, docs->n, (int)(first / q));
+  if (min(first + 255, total - 1) / q < docs->b[d0 + 1]) {
     __shared__ float wmax[4];
-    tile_max = wave_max(tile_max);
-    if (lane == 0) wmax[wave] = tile_max;
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (tid == 0)
-      raise_amax(p.amax_out, tile_doc, blockIdx.x + blockIdx.y,
-                 fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
+    if (threadIdx.x == 0)
+      raise_amax(amax, d0, blockIdx.x, fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
+  } else if (i < total) {
+    raise_amax(amax, doc_of(docs->b, docs->n, (int)(i / q)), blockIdx.x, m);
   }
 }
 
@@ -305,18 +344,29 @@ __global__ __launch_bounds__(256) void snake_kernel(const float* __restrict__ x,
     }
     *reinterpret_cast<f32x4*>(out + r * ldo + c) = y;
   }
-  if (!amax) return;
-  const int d0 = doc_of(docs->b, docs->n, (int)(first / q));
-  if (min(first + 255, total - 1) / q < docs->b[d0 + 1]) {
-    __shared__ float wmax[4];
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      raise_amax(amax, d0, blockIdx.x, fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
-  } else if (i < total) {
-    raise_amax(amax, doc_of(docs->b, docs->n, (int)r), blockIdx.x, m);
+  raise_rows_amax(amax, m, first, i, total, q, docs);
+}
+
+// out = the mean of in.n tensors, four values a thread, summed in order
+__global__ __launch_bounds__(256) void mean_kernel(const HiftMean in, float* __restrict__ out, int C,
+                                                   uint32_t* __restrict__ amax,
+                                                   const HiftDocs* __restrict__ docs) {
+  const int q = C / 4;
+  const long first = (long)blockIdx.x * blockDim.x, total = (long)docs->b[docs->n] * q;
+  if (first >= total) return;
+  const long i = first + threadIdx.x;
+  float m = 0.0f;
+  if (i < total) {
+    f32x4 v = reinterpret_cast<const f32x4*>(in.x[0])[i];
+    for (int k = 1; k < in.n; ++k) v += reinterpret_cast<const f32x4*>(in.x[k])[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = v[e] / (float)in.n;
+      m = fmaxf(m, finite_abs(v[e]));
+    }
+    reinterpret_cast<f32x4*>(out)[i] = v;
   }
+  raise_rows_amax(amax, m, first, i, total, q, docs);
 }
 
 __global__ __launch_bounds__(256) void to_f64_kernel(const float* __restrict__ x,
@@ -504,7 +554,7 @@ unsigned blocks_for(long n, int threads) { return (unsigned)((n + threads - 1) /
 bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
 template <typename T>
-hipError_t launch_conv(const HiftConv& p_in, const HiftDocs* docs, hipStream_t stream) {
+hipError_t launch_conv(const HiftConv& p_in, hipStream_t stream) {
   if (p_in.rows_out <= 0) return hipSuccess;
   if (p_in.cin_pad % 16 != 0) return hipErrorInvalidValue;
   HiftConv p = p_in;
@@ -513,7 +563,10 @@ hipError_t launch_conv(const HiftConv& p_in, const HiftDocs* docs, hipStream_t s
            (!p.add || (p.ld_add % 4 == 0 && aligned16(p.add))) &&
            (p.mode == HIFT_ACC_WRITE || aligned16(p.accin)) &&
            (!p.snake_out || (aligned16(p.alpha) && aligned16(p.inv_alpha))) &&
-           (!p.out2 || (aligned16(p.out2) && aligned16(p.alpha2) && aligned16(p.inv_alpha2)));
+           (!p.n_snakes || (aligned16(p.snakes[0].out) && aligned16(p.snakes[0].alpha) &&
+                            aligned16(p.snakes[0].inv_alpha)));
+  if (p.n_snakes > 1 || !p.docs) return hipErrorInvalidValue;
+  if (!p.n_snakes) p.snakes[0].amax = nullptr;
   // 64x64 tiles, or 32x32 where 64x64 tiles would not give every CU one (the grid covers the
   // capacity, so a captured call and its replays use the same size; results do not depend on it).
   // FCV_HIFT_TILE=32 or 64 forces one size: a test hook, since both must give the same bits.
@@ -523,26 +576,26 @@ hipError_t launch_conv(const HiftConv& p_in, const HiftDocs* docs, hipStream_t s
   if (force == 32 || (force != 64 && tiles64 < kSmallTileBelow)) {
     const dim3 grid((p.rows_out + 31) / 32, (p.cout + 31) / 32);
     if (p.cin_pad % 32 == 0)
-      hipLaunchKernelGGL((hift_conv_kernel<T, 32, 32>), grid, dim3(256), 0, stream, p, docs);
+      hipLaunchKernelGGL((hift_conv_kernel<T, 32, 32>), grid, dim3(256), 0, stream, p);
     else
-      hipLaunchKernelGGL((hift_conv_kernel<T, 16, 32>), grid, dim3(256), 0, stream, p, docs);
+      hipLaunchKernelGGL((hift_conv_kernel<T, 16, 32>), grid, dim3(256), 0, stream, p);
     return hipGetLastError();
   }
   const dim3 grid((p.rows_out + kTileR - 1) / kTileR, (p.cout + kTileC - 1) / kTileC);
   if (p.cin_pad % 32 == 0)
-    hipLaunchKernelGGL((hift_conv_kernel<T, 32, 64>), grid, dim3(256), 0, stream, p, docs);
+    hipLaunchKernelGGL((hift_conv_kernel<T, 32, 64>), grid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((hift_conv_kernel<T, 16, 64>), grid, dim3(256), 0, stream, p, docs);
+    hipLaunchKernelGGL((hift_conv_kernel<T, 16, 64>), grid, dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t hift_conv_f32(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
-  return launch_conv<float>(p, docs, stream);
+hipError_t hift_conv_f32(const HiftConv& p, hipStream_t stream) {
+  return launch_conv<float>(p, stream);
 }
-hipError_t hift_conv_f64(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
-  return launch_conv<double>(p, docs, stream);
+hipError_t hift_conv_f64(const HiftConv& p, hipStream_t stream) {
+  return launch_conv<double>(p, stream);
 }
 
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
@@ -552,6 +605,15 @@ hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, in
   const long n = (long)rows * (C / 4);
   hipLaunchKernelGGL(snake_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, x, ldx, out,
                      ldo, C, alpha, inv_alpha, amax, docs);
+  return hipGetLastError();
+}
+
+hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* amax,
+                     const HiftDocs* docs, hipStream_t stream) {
+  if (rows <= 0) return hipSuccess;
+  if (in.n < 1 || in.n > 4 || C % 4 != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(mean_kernel, dim3(blocks_for((long)rows * (C / 4), 256)), dim3(256), 0, stream,
+                     in, out, C, amax, docs);
   return hipGetLastError();
 }
 

@@ -47,25 +47,37 @@ struct HiftConv {
   const float* alpha; const float* inv_alpha;    // snake_out: out = snake(y)
   int snake_out;
   void* out; int ldo;
-  void* out2; const float* alpha2; const float* inv_alpha2;  // out2 = snake(y) (optional)
+  // further outputs snake_i(y), for the convolutions that read them (n_snakes <= kHiftSnakes; more
+  // than one in the split form only); amax: see amax_out
+  int n_snakes;
+  struct Snake { float* out; const float* alpha; const float* inv_alpha; uint32_t* amax; };
+  Snake snakes[4];
   int vec4;                                // set by the launch: 16-byte epilogue accesses
   // split f16 form (hift_conv_split): packed weights of co_pad channels, their inverse scales and
   // biases ([co_pad] each, one after the other);
   // the largest finite |input| per document (fp32 bits)
   const void* wsplit; const float* winv; int co_pad;
   const uint32_t* amax_in;
-  // per document, raised to the largest finite magnitude written to out / out2 (optional)
-  uint32_t* amax_out; uint32_t* amax_out2;
+  // per document, raised to the largest finite magnitude written to out (optional)
+  uint32_t* amax_out;
+  const HiftDocs* docs;                    // the layout
 };
 
-hipError_t hift_conv_f32(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
-hipError_t hift_conv_f64(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
+// Independent convolutions of one launch (split form), the longest first
+constexpr int kHiftJobs = 5;
+struct HiftJobs {
+  HiftConv c[kHiftJobs];
+};
+
+hipError_t hift_conv_f32(const HiftConv& p, hipStream_t stream);
+hipError_t hift_conv_f64(const HiftConv& p, hipStream_t stream);
 
 // The fp32 convolution with both operands split into two f16 halves (hift_split.hip), for the
 // shapes hift_split_eligible takes (its rule reads the shape only, not the row count): unit
 // stride, all context on the left, input channels a multiple of 32.
 bool hift_split_eligible(const HiftConv& p);
-hipError_t hift_conv_split(const HiftConv& p, const HiftDocs* docs, hipStream_t stream);
+// n <= kHiftJobs convolutions that do not depend on each other, in one launch
+hipError_t hift_conv_split(const HiftConv* convs, int n, hipStream_t stream);
 // its packed weights: bytes, and the packing of fp32 [co_pad][k][cin] with its cout biases (inv:
 // [co_pad] inverse scales, then [co_pad] biases)
 size_t hift_split_bytes(int co_pad, int k, int cin);
@@ -78,6 +90,12 @@ hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream);
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
                       const float* alpha, const float* inv_alpha, uint32_t* amax,
                       const HiftDocs* docs, hipStream_t stream);
+
+// out[i] = (((x_0[i] + x_1[i]) + ...) / n over the live rows docs->b[docs->n] (grid: `rows`) x C
+// values (C % 4 == 0), n <= 4; amax: see HiftConv::amax_out
+struct HiftMean { const float* x[4]; int n; };
+hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* amax,
+                     const HiftDocs* docs, hipStream_t stream);
 
 // fp32 -> fp64 of the live rows docs->a[docs->n] (grid: `rows`) x C values
 hipError_t hift_to_f64(const float* x, double* y, int rows, int C, const HiftDocs* docs,

@@ -132,6 +132,13 @@ bool doc_lens(const FcvHiftDims& d, int frames, bool fin, DocLens* out) {
 }
 
 constexpr size_t kGraphPool = 4;  // captured calls kept per handle (least recently used goes)
+// Mel frames of a capacity up to which a stage's resblocks run together.  A resblock is a chain of
+// six convolutions that depend on each other; the three of a stage and the next stage's source
+// branch do not, so one launch takes one convolution of each: 79 convolution launches a call
+// become 33, each with three to four times the workgroups.  One call, apart against together: 24
+// frames 2.00 -> 1.20 ms, 68 2.05 -> 1.26, 286 2.53 -> 1.91, 900 4.68 -> 4.08, 8 requests of 3065
+// frames 10.6 either way.  It takes 16 stage buffers instead of 7 (0.5 MB a frame), hence the limit.
+constexpr int kTogetherFrames = 1 << 16;
 constexpr size_t kSeenKeys = 8;   // keys remembered for the capture-on-second-call rule
 
 // The workspace carve-up and the grids of a capacity: at most `frames` Mel frames in at most
@@ -142,8 +149,10 @@ struct Capacity {
   int frames, docs;
   int spec, samples, src;              // STFT frames, output samples, source samples
   std::vector<int> stage, stage_w;     // upsampling-conv rows and written rows per stage
-  size_t mel64, h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, r, t1, s1, si, y, fr,
-      amax, tables, total;
+  size_t mel64, h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, y, fr, amax, tables, total;
+  size_t si[2];                        // source branches of this stage and the next
+  bool together;                       // a stage's resblocks run together (see run)
+  size_t r[fcv::kHiftJobs], t1[fcv::kHiftJobs], s1[fcv::kHiftJobs];  // one set per resblock in flight
   int amax_slots;                      // per document: one per tensor a split convolution reads
 };
 
@@ -177,8 +186,15 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
   C.sines = take(sizeof(float) * frames * H);
   C.srcbuf = take(sizeof(float) * C.src);
   C.specbuf = take(sizeof(float) * C.spec * kSpecLd);
-  for (size_t* b : {&C.xa, &C.xn, &C.xs, &C.r, &C.t1, &C.s1, &C.si})
-    *b = take(sizeof(float) * smax);
+  for (size_t* b : {&C.xa, &C.xn, &C.xs, &C.si[0]}) *b = take(sizeof(float) * smax);
+  C.together = frames <= kTogetherFrames;
+  C.si[1] = C.together ? take(sizeof(float) * smax) : C.si[0];
+  for (int i = 0; i <= d.n_kernels; ++i) {
+    const bool own = i == 0 || C.together;
+    C.r[i] = own ? take(sizeof(float) * smax) : C.r[0];
+    C.t1[i] = own ? take(sizeof(float) * smax) : C.t1[0];
+    C.s1[i] = own ? take(sizeof(float) * smax) : C.s1[0];
+  }
   C.y = take(sizeof(float) * C.spec * kSpecLd);
   C.fr = take(sizeof(float) * C.spec * kFrameLd);
   C.amax_slots = 1 + d.n_stages * (1 + 2 * d.n_dilations * (1 + d.n_kernels));
@@ -277,8 +293,9 @@ std::vector<HiftDocs> make_tables(const FcvHiftDims& d, const Plan& P) {
 }
 
 HiftConv conv_base(const void* x, int ldx, int cout, int cin_pad, int k, void* out, int ldo,
-                   int rows_out) {
+                   int rows_out, const HiftDocs* docs) {
   HiftConv p{};
+  p.docs = docs;
   p.x = x; p.ldx = ldx; p.cout = cout; p.cin_pad = cin_pad; p.k = k;
   p.stride = 1; p.dil = 1; p.pad = 0; p.up = 1; p.rows_out = rows_out;
   p.out = out; p.ldo = ldo; p.div = 1.0f;
@@ -299,63 +316,109 @@ struct Convs {
     if (!h->packed_base || used >= slots) return nullptr;
     return amax + (size_t)docs_cap * fcv::kAmaxWords * used++;
   }
-  // p with weight index wi (bias wi + 1), its input's slot `in`
-  int run(HiftConv p, int wi, const uint32_t* in, const HiftDocs* docs) const {
-    p.w = h->w[wi];
-    p.bias = h->w[wi + 1];
-    const FcvHift::Packed& k = h->packed[wi];
-    if (h->packed_base && k.w >= 0 && in) {
-      p.wsplit = h->packed_base + k.w;
-      p.winv = reinterpret_cast<const float*>(h->packed_base + k.inv);
-      p.co_pad = k.co_pad;
-      p.amax_in = in;
-      FCV_HIP(fcv::hift_conv_split(p, docs, st));
+  // n independent convolutions: p[i] with weight index wi[i] (bias wi[i] + 1) and its input's slot
+  // in[i]; one launch where all of them have split weights
+  int run(HiftConv* p, const int* wi, const uint32_t* const* in, int n) const {
+    bool all = true;
+    for (int i = 0; i < n; ++i) {
+      p[i].w = h->w[wi[i]];
+      p[i].bias = h->w[wi[i] + 1];
+      const FcvHift::Packed& k = h->packed[wi[i]];
+      if (h->packed_base && k.w >= 0 && in[i]) {
+        p[i].wsplit = h->packed_base + k.w;
+        p[i].winv = reinterpret_cast<const float*>(h->packed_base + k.inv);
+        p[i].co_pad = k.co_pad;
+        p[i].amax_in = in[i];
+      } else {
+        all = false;
+      }
+    }
+    if (all) {
+      FCV_HIP(fcv::hift_conv_split(p, n, st));
       return FCV_OK;
     }
-    FCV_HIP(fcv::hift_conv_f32(p, docs, st));
+    for (int i = 0; i < n; ++i)
+      FCV_HIP(p[i].wsplit ? fcv::hift_conv_split(p + i, 1, st) : fcv::hift_conv_f32(p[i], st));
     return FCV_OK;
   }
+  int run(HiftConv p, int wi, const uint32_t* in) const { return run(&p, &wi, &in, 1); }
+  const float* f32(int i) const { return static_cast<const float*>(h->w[i]); }
 };
 
-// one ResBlock (generator.py:110-116) on x (rows by `docs`, C channels): for each dilation
-// j: r = r + conv2(snake2(conv1(snake1(r)))); the last conv2 writes its result per `mode`
-// (write / accin + y / (accin + y) / div) into `out`, its magnitude into `amax_out` (optional).
-// `wi` is the index of the block's 8 * D weights.  x is read as the first residual; r holds the
-// running value.  `rows` is the capacity the grids cover.
-int run_resblock(Convs& cv, int wi, int k, const int* dils, const float* x, float* r, float* t1,
-                 float* s1, float* out, int mode, const float* accin, float div,
-                 uint32_t* amax_out, int C, int rows, const HiftDocs* docs) {
+// One ResBlock (generator.py:110-116) on x (rows by `docs`, C channels): for each dilation j:
+// r = r + conv2(snake2(conv1(snake1(r)))); the last conv2 writes its result per `mode` (write /
+// accin + y / (accin + y) / div) into `out`, its magnitude into `amax_out` (optional).  `wi` is the
+// index of the block's 8 * D weights.  x is read as the first residual; r holds the running value.
+// s1 holds snake1(x) already, of magnitude a_s1, where `ready`.  `rows` is the capacity the grids
+// cover.
+struct ResBlock {
+  int wi, k;
+  const int* dils;
+  int C, rows;
+  const HiftDocs* docs;
+  const float* x;
+  float *r, *t1, *s1, *out;
+  uint32_t* a_s1;
+  bool ready;
+  int mode;
+  const float* accin;
+  float div;
+  uint32_t* amax_out;
+};
+
+// n resblocks that do not depend on each other, one convolution of each at a time
+int run_resblocks(Convs& cv, ResBlock* blocks, int n) {
   const int D = cv.h->d.n_dilations;
-  auto F = [&](int i) { return static_cast<const float*>(cv.h->w[i]); };
-  uint32_t* a_s1 = cv.slot();
-  FCV_HIP(fcv::hift_snake(x, C, s1, C, rows, C, F(wi + 4), F(wi + 5), a_s1, docs, cv.st));
+  // the longest first: its workgroups start first
+  std::stable_sort(blocks, blocks + n, [](const ResBlock& a, const ResBlock& b) {
+    return (long)a.k * a.rows * a.C * a.C > (long)b.k * b.rows * b.C * b.C;
+  });
+  for (int i = 0; i < n; ++i) {
+    ResBlock& b = blocks[i];
+    if (b.ready) continue;
+    b.a_s1 = cv.slot();
+    FCV_HIP(fcv::hift_snake(b.x, b.C, b.s1, b.C, b.rows, b.C, cv.f32(b.wi + 4), cv.f32(b.wi + 5),
+                            b.a_s1, b.docs, cv.st));
+  }
+  HiftConv c[fcv::kHiftJobs];
+  int wi[fcv::kHiftJobs];
+  const uint32_t* in[fcv::kHiftJobs];
   for (int j = 0; j < D; ++j) {
-    const int q = wi + 8 * j;
-    HiftConv c1 = conv_base(s1, C, C, C, k, t1, C, rows);
-    c1.dil = dils[j];
-    c1.pad = causal_padding(k, dils[j]);
-    c1.snake_out = 1;
-    c1.alpha = F(q + 6);
-    c1.inv_alpha = F(q + 7);
-    c1.amax_out = cv.slot();
-    if (int rc = cv.run(c1, q, a_s1, docs)) return rc;
     const bool last = j == D - 1;
-    HiftConv c2 = conv_base(t1, C, C, C, k, last ? out : r, C, rows);
-    c2.pad = causal_padding(k, 1);
-    c2.add = j == 0 ? static_cast<const void*>(x) : static_cast<const void*>(r);
-    c2.ld_add = C;
-    if (last) {
-      c2.mode = mode;
-      c2.accin = accin;
-      c2.div = div;
-      c2.amax_out = amax_out;
-    } else {
-      c2.out2 = s1;
-      c2.alpha2 = F(q + 8 + 4);
-      c2.inv_alpha2 = F(q + 8 + 5);
-      c2.amax_out2 = a_s1 = cv.slot();
+    for (int i = 0; i < n; ++i) {
+      const ResBlock& b = blocks[i];
+      wi[i] = b.wi + 8 * j;
+      in[i] = b.a_s1;
+      c[i] = conv_base(b.s1, b.C, b.C, b.C, b.k, b.t1, b.C, b.rows, b.docs);
+      c[i].dil = b.dils[j];
+      c[i].pad = causal_padding(b.k, b.dils[j]);
+      c[i].snake_out = 1;
+      c[i].alpha = cv.f32(wi[i] + 6);
+      c[i].inv_alpha = cv.f32(wi[i] + 7);
+      c[i].amax_out = cv.slot();
     }
-    if (int rc = cv.run(c2, q + 2, c1.amax_out, docs)) return rc;
+    if (int rc = cv.run(c, wi, in, n)) return rc;
+    for (int i = 0; i < n; ++i) {
+      ResBlock& b = blocks[i];
+      in[i] = c[i].amax_out;
+      wi[i] += 2;
+      c[i] = conv_base(b.t1, b.C, b.C, b.C, b.k, last ? b.out : b.r, b.C, b.rows, b.docs);
+      c[i].pad = causal_padding(b.k, 1);
+      c[i].add = j == 0 ? b.x : b.r;
+      c[i].ld_add = b.C;
+      if (last) {
+        c[i].mode = b.mode;
+        c[i].accin = b.accin;
+        c[i].div = b.div;
+        c[i].amax_out = b.amax_out;
+      } else {
+        b.a_s1 = cv.slot();
+        c[i].n_snakes = 1;
+        c[i].snakes[0] = {b.s1, cv.f32(b.wi + 8 * (j + 1) + 4), cv.f32(b.wi + 8 * (j + 1) + 5),
+                          b.a_s1};
+      }
+    }
+    if (int rc = cv.run(c, wi, in, n)) return rc;
   }
   return FCV_OK;
 }
@@ -376,20 +439,20 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   FCV_HIP(fcv::hift_to_f64(mel, F64(C.mel64), C.frames, d.in_channels, T + 0, st));
   const int fc = d.f0_channels;
   HiftConv c0 = conv_base(F64(C.mel64), d.in_channels, fc, d.in_channels, 4, F64(C.h64a), fc,
-                          C.frames);
+                          C.frames, T + 0);
   c0.w = w[h->i_f0];
   c0.bias = w[h->i_f0 + 1];
   c0.elu = 1;  // right-side lookahead: no left padding, zero (or context) on the right
-  FCV_HIP(fcv::hift_conv_f64(c0, T + 0, st));
+  FCV_HIP(fcv::hift_conv_f64(c0, st));
   double* hin = F64(C.h64a);
   double* hout = F64(C.h64b);
   for (int l = 1; l < 5; ++l) {
-    HiftConv c = conv_base(hin, fc, fc, fc, 3, hout, fc, C.frames);
+    HiftConv c = conv_base(hin, fc, fc, fc, 3, hout, fc, C.frames, T + 1);
     c.w = w[h->i_f0 + 2 * l];
     c.bias = w[h->i_f0 + 2 * l + 1];
     c.pad = causal_padding(3, 1);
     c.elu = 1;
-    FCV_HIP(fcv::hift_conv_f64(c, T + 1, st));
+    FCV_HIP(fcv::hift_conv_f64(c, st));
     std::swap(hin, hout);
   }
   FCV_HIP(fcv::hift_f0_head(hin, fc, static_cast<const double*>(w[h->i_cls]),
@@ -427,70 +490,98 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   uint32_t* a_xp = cv.slot();  // magnitude of xp
   {
     HiftConv c = conv_base(mel, d.in_channels, d.base_channels, d.in_channels,
-                           d.conv_pre_look_right + 1, xp, d.base_channels, C.frames);
+                           d.conv_pre_look_right + 1, xp, d.base_channels, C.frames, T + 4);
     c.amax_out = a_xp;
-    if (int rc = cv.run(c, h->i_pre, nullptr, T + 4)) return rc;
+    if (int rc = cv.run(c, h->i_pre, nullptr)) return rc;
   }
 
   // ---- upsampling stages -----------------------------------------------------------------
   int cprev = d.base_channels;
   const int rb_size = 8 * d.n_dilations;
+  const int K = d.n_kernels;
+  // source branch of stage s: strided (or 1x1) conv of the STFT frames into si[s % 2], then its
+  // resblock there, on buffer set `set`
+  auto source = [&](int s, int set, ResBlock* b) -> int {
+    const int Cs = stage_channels(d, s);
+    const auto kd = source_down(d, s);
+    float* si = F32(C.si[s & 1]);
+    *b = ResBlock{h->i_srb + rb_size * s, d.source_kernels[s], d.source_dilations[s], Cs,
+                  C.stage_w[s], T + 6 + 3 * s, si, F32(C.r[set]), F32(C.t1[set]), F32(C.s1[set]),
+                  si, cv.slot(), true, fcv::HIFT_ACC_WRITE, nullptr, 1.0f, nullptr};
+    HiftConv c = conv_base(F32(C.specbuf), kSpecLd, Cs, kSpecLd, kd.first, si, Cs, C.stage_w[s],
+                           T + 5 + 3 * s);
+    c.stride = kd.second;
+    c.pad = kd.second - 1;
+    c.n_snakes = 1;
+    c.snakes[0] = {b->s1, cv.f32(b->wi + 4), cv.f32(b->wi + 5), b->a_s1};
+    return cv.run(c, h->i_down + 2 * s, nullptr);
+  };
   for (int s = 0; s < S; ++s) {
     const int Cs = stage_channels(d, s);
-    const bool last = s == S - 1;
     const int nrows = C.stage_w[s];
-    const HiftDocs* t_src = T + 5 + 3 * s;  // (spec, rows_w)
     const HiftDocs* t_w = T + 6 + 3 * s;    // (rows_w, rows_w)
-    const HiftDocs* t_up = T + 7 + 3 * s;   // (previous rows, stage rows)
-
-    // source branch: strided (or 1x1) conv of the STFT frames, then its resblock
-    float* si = F32(C.si);
-    {
-      const auto kd = source_down(d, s);
-      HiftConv c = conv_base(F32(C.specbuf), kSpecLd, Cs, kSpecLd, kd.first, si, Cs, nrows);
-      c.stride = kd.second;
-      c.pad = kd.second - 1;
-      if (int rc = cv.run(c, h->i_down + 2 * s, nullptr, t_src)) return rc;
-      if (int rc = run_resblock(cv, h->i_srb + rb_size * s, d.source_kernels[s],
-                                d.source_dilations[s], si, F32(C.r), F32(C.t1), F32(C.s1), si,
-                                fcv::HIFT_ACC_WRITE, nullptr, 1.0f, nullptr, Cs, nrows, t_w))
-        return rc;
+    ResBlock b[fcv::kHiftJobs];
+    if (s == 0 || !C.together) {
+      if (int rc = source(s, 0, b)) return rc;
+      if (int rc = run_resblocks(cv, b, 1)) return rc;
     }
-    // upsampling conv on LeakyReLU(x), plus the source branch
+    for (int j = 0; j < K; ++j)
+      b[j] = ResBlock{h->i_rb + rb_size * (s * K + j), d.resblock_kernels[j],
+                      d.resblock_dilations[j], Cs, nrows, t_w, xn, F32(C.r[j]), F32(C.t1[j]),
+                      F32(C.s1[j]), F32(C.r[j]), nullptr, false, fcv::HIFT_ACC_WRITE, nullptr, 1.0f,
+                      nullptr};
+    // upsampling conv on LeakyReLU(x), plus the source branch (and, for resblocks that run
+    // together, their first Snakes)
     {
-      HiftConv c = conv_base(xp, cprev, Cs, cprev, d.upsample_kernels[s], xn, Cs, C.stage[s]);
+      HiftConv c = conv_base(xp, cprev, Cs, cprev, d.upsample_kernels[s], xn, Cs, C.stage[s],
+                             T + 7 + 3 * s);
       c.up = d.upsample_rates[s];
       c.pad = d.upsample_kernels[s] - 1;
       c.pro = fcv::HIFT_PRO_LEAKY;
       c.slope = d.lrelu_slope;
-      c.reflect = last ? 1 : 0;
-      c.add = si;
+      c.reflect = s == S - 1 ? 1 : 0;
+      c.add = F32(C.si[s & 1]);
       c.ld_add = Cs;
-      if (int rc = cv.run(c, h->i_ups + 2 * s, a_xp, t_up)) return rc;
+      const int wi = h->i_ups + 2 * s;
+      if (C.together && h->packed_base && h->packed[wi].w >= 0) {
+        c.n_snakes = K;
+        for (int j = 0; j < K; ++j) {
+          b[j].a_s1 = cv.slot();
+          b[j].ready = true;
+          c.snakes[j] = {b[j].s1, cv.f32(b[j].wi + 4), cv.f32(b[j].wi + 5), b[j].a_s1};
+        }
+      }
+      if (int rc = cv.run(c, wi, a_xp)) return rc;
     }
     // mean of the resblocks
     a_xp = cv.slot();
-    for (int j = 0; j < d.n_kernels; ++j) {
-      const int K = d.n_kernels;
-      int mode = fcv::HIFT_ACC_WRITE;
-      float* out = F32(C.xs);
-      const float* accin = nullptr;
-      float div = 1.0f;
-      if (K == 1) {
-        out = xn;
-      } else if (j == K - 1) {
-        mode = fcv::HIFT_ACC_ADD_DIV;
-        accin = F32(C.xs);
-        out = xn;
-        div = (float)K;
-      } else if (j > 0) {
-        mode = fcv::HIFT_ACC_ADD;
-        accin = F32(C.xs);
+    if (C.together) {
+      fcv::HiftMean mean{};
+      mean.n = K;
+      for (int j = 0; j < K; ++j) mean.x[j] = b[j].out;
+      int n = K;
+      if (s + 1 < S) {
+        if (int rc = source(s + 1, K, b + n)) return rc;
+        ++n;
       }
-      if (int rc = run_resblock(cv, h->i_rb + rb_size * (s * K + j), d.resblock_kernels[j],
-                                d.resblock_dilations[j], xn, F32(C.r), F32(C.t1), F32(C.s1),
-                                out, mode, accin, div, j == K - 1 ? a_xp : nullptr, Cs, nrows, t_w))
-        return rc;
+      if (int rc = run_resblocks(cv, b, n)) return rc;
+      FCV_HIP(fcv::hift_mean(mean, xn, nrows, Cs, a_xp, t_w, st));
+    } else {
+      for (int j = 0; j < K; ++j) {
+        ResBlock& q = b[j];
+        q.out = F32(C.xs);
+        if (j > 0) {
+          q.mode = fcv::HIFT_ACC_ADD;
+          q.accin = F32(C.xs);
+        }
+        if (j == K - 1) {
+          if (K > 1) q.mode = fcv::HIFT_ACC_ADD_DIV;
+          q.div = (float)K;
+          q.out = xn;
+          q.amax_out = a_xp;
+        }
+        if (int rc = run_resblocks(cv, &q, 1)) return rc;
+      }
     }
     cprev = Cs;
     std::swap(xp, xn);
@@ -499,11 +590,11 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- conv_post on LeakyReLU(x) (slope 0.01), iSTFT, clamp ------------------------------
   {
     const int spec = d.n_fft + 2;
-    HiftConv c = conv_base(xp, cprev, spec, cprev, 7, F32(C.y), kSpecLd, C.spec);
+    HiftConv c = conv_base(xp, cprev, spec, cprev, 7, F32(C.y), kSpecLd, C.spec, T + 5 + 3 * S);
     c.pad = causal_padding(7, 1);
     c.pro = fcv::HIFT_PRO_LEAKY;
     c.slope = 0.01f;
-    if (int rc = cv.run(c, h->i_post, a_xp, T + 5 + 3 * S)) return rc;
+    if (int rc = cv.run(c, h->i_post, a_xp)) return rc;
   }
   FCV_HIP(fcv::hift_istft(F32(C.y), kSpecLd, window, F32(C.fr), speech, d.audio_limit, C.spec,
                           C.samples, T + 6 + 3 * S, st));
@@ -588,7 +679,7 @@ void plan_packed(FcvHift* h) {
   h->packed.assign(h->w.size(), FcvHift::Packed{});
   size_t off = 0;
   auto add = [&](int wi, int cout, int cin, int k, int dil, int up, float slope) {
-    HiftConv p = conv_base(nullptr, 0, cout, cin, k, nullptr, 0, 0);
+    HiftConv p = conv_base(nullptr, 0, cout, cin, k, nullptr, 0, 0, nullptr);
     p.dil = dil;
     p.up = up;
     p.pad = causal_padding(k, dil);

@@ -28,6 +28,7 @@
 // order of every output's sum is the same in every tile shape, so results do not depend on the
 // shape a launch takes.  (Compiled without floating-point contraction, as the rounding of an
 // output must not depend on the instantiation either.)
+#include <algorithm>
 #include <cstdlib>
 
 #include "hift.hpp"
@@ -115,9 +116,9 @@ struct SplitCols {
       alpha = load4(p.alpha, c);
       inv_alpha = load4(p.inv_alpha, c);
     }
-    if (p.out2) {
-      alpha2 = load4(p.alpha2, c);
-      inv_alpha2 = load4(p.inv_alpha2, c);
+    if (p.n_snakes) {
+      alpha2 = load4(p.snakes[0].alpha, c);
+      inv_alpha2 = load4(p.snakes[0].inv_alpha, c);
     }
   }
 };
@@ -132,10 +133,10 @@ struct SplitAdds {
 };
 
 // the epilogue of channels c .. c + 3 of one row: unscale, bias, residual, resblock sum, Snakes; m1, m2:
-// raised to the largest finite magnitudes written to out and out2
+// raised to the largest finite magnitudes written to out and to each Snake output
 __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& cols,
                                             const SplitAdds& in, long row, int c, const f32x4& acc,
-                                            float inv, float& m1, float& m2) {
+                                            float inv, float& m1, float (&m2)[4]) {
   f32x4 v;
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = fmaf(acc[e] * inv, cols.winv[e], cols.bias[e]);
@@ -161,13 +162,23 @@ __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& 
     for (int e = 0; e < 4; ++e) m1 = fmaxf(m1, finite_abs(v[e]));
   }
   *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + i) = v;
-  if (p.out2) {
+  if (p.n_snakes) {
     f32x4 w;
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = snake(v[e], cols.alpha2[e], cols.inv_alpha2[e]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) m2 = fmaxf(m2, finite_abs(w[e]));
-    *reinterpret_cast<f32x4*>(static_cast<float*>(p.out2) + i) = w;
+    for (int e = 0; e < 4; ++e) m2[0] = fmaxf(m2[0], finite_abs(w[e]));
+    *reinterpret_cast<f32x4*>(p.snakes[0].out + i) = w;
+#pragma unroll
+    for (int n = 1; n < 4; ++n) {
+      if (n >= p.n_snakes) break;
+      const f32x4 a = load4(p.snakes[n].alpha, c), ia = load4(p.snakes[n].inv_alpha, c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = snake(v[e], a[e], ia[e]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m2[n] = fmaxf(m2[n], finite_abs(w[e]));
+      *reinterpret_cast<f32x4*>(p.snakes[n].out + i) = w;
+    }
   }
 }
 
@@ -193,7 +204,9 @@ struct Cfg {
 
 template <class C>
 __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
-    const HiftConv p, const HiftDocs* __restrict__ docs) {
+    const HiftJobs jobs) {
+  const HiftConv& p = jobs.c[blockIdx.z];
+  const HiftDocs* __restrict__ docs = p.docs;
   __shared__ __attribute__((aligned(1024))) char smem[C::kLds];
   char* sX = smem + C::kXOff;
   // per tile row: window row of the first tap (of input position 0 for up > 1), position and
@@ -229,6 +242,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   }
   const bool one_doc = min(r0 + C::TR, rows_out) <= out1;  // of the tile's rows
   const int co0 = blockIdx.y * C::TC;
+  if (co0 >= p.cout) return;
   const int chunks = p.cin_pad / 32;
   const int k = p.k;
 
@@ -439,7 +453,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   // whole 128-byte (256-byte) runs of a row.
   float* stage = reinterpret_cast<float*>(smem + wave * C::kStage);
   constexpr int RPI = 64 / LPR, NP = 32 / RPI;  // rows a pass, passes
-  float m1 = 0.0f, m2 = 0.0f;                   // largest finite magnitudes written
+  float m1 = 0.0f, m2[4] = {};                  // largest finite magnitudes written
   const int sub = blockIdx.x + blockIdx.y;
 #pragma unroll
   for (int b = 0; b < C::MR; ++b) {
@@ -471,7 +485,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       const int4 info = sInfo[t];
       const float inv = sInv[t];
       const long row = p.reflect ? (long)r + info.z + 1 : r;
-      float a1 = 0.0f, a2 = 0.0f;
+      float a1 = 0.0f, a2[4] = {};
       split_store(p, cols, in[i], row, c4, v, inv, a1, a2);
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
       if (p.reflect && info.y == 1) {
@@ -481,25 +495,31 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       }
       if (one_doc) {
         m1 = fmaxf(m1, a1);
-        m2 = fmaxf(m2, a2);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) m2[n] = fmaxf(m2[n], a2[n]);
       } else {
         if (p.amax_out) raise_amax(p.amax_out, info.z, sub, a1);
-        if (p.amax_out2) raise_amax(p.amax_out2, info.z, sub, a2);
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          if (n < p.n_snakes) raise_amax(p.snakes[n].amax, info.z, sub, a2[n]);
       }
     }
   }
-  if (one_doc && (p.amax_out || p.amax_out2)) {
+  if (one_doc && (p.amax_out || p.n_snakes)) {
     float* wmax = sInv;  // the row scales are read
     m1 = wave_max(m1);
-    m2 = wave_max(m2);
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (n < p.n_snakes) m2[n] = wave_max(m2[n]);
     __syncthreads();
     if (lane == 0) {
       wmax[wave] = m1;
-      wmax[4 + wave] = m2;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) wmax[4 + 4 * n + wave] = m2[n];
     }
     __syncthreads();
-    if (tid < 2) {
-      uint32_t* slot = tid == 0 ? p.amax_out : p.amax_out2;
+    if (tid <= p.n_snakes) {
+      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[tid - 1].amax;
       float m = 0.0f;
 #pragma unroll
       for (int w = 0; w < C::kWaves; ++w) m = fmaxf(m, wmax[tid * 4 + w]);
@@ -548,10 +568,11 @@ __global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ x,
 bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
 template <class C>
-hipError_t launch(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
+hipError_t launch(const HiftJobs& jobs, int n, int rows, int cout, hipStream_t stream) {
   static_assert(C::kLds <= 160 * 1024, "LDS");
-  const dim3 grid((p.rows_out + C::TR - 1) / C::TR, (p.cout + C::TC - 1) / C::TC);
-  hipLaunchKernelGGL(split_conv_kernel<C>, grid, dim3(C::kThreads), 0, stream, p, docs);
+  static_assert(C::TR >= 20, "the epilogue's maxima fit the row scales' place");
+  const dim3 grid((rows + C::TR - 1) / C::TR, (cout + C::TC - 1) / C::TC, n);
+  hipLaunchKernelGGL(split_conv_kernel<C>, grid, dim3(C::kThreads), 0, stream, jobs);
   return hipGetLastError();
 }
 
@@ -560,14 +581,31 @@ int window_rows(const HiftConv& p, int tr) {
   return (tr - 1) / p.up + 2 + ((p.k - 1) * p.dil + p.up - 1) / p.up;
 }
 
-// the shape with the window passes the launch needs
+// the shape with the window passes the launch's widest window needs
 template <int WC, int WR, int MC, int MR, int NS, int P1, int P2, int P3>
-hipError_t launch_win(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
-  const int need = window_rows(p, 32 * MR * WR), per = 8 * WC * WR;
-  if (need <= P1 * per) return launch<Cfg<WC, WR, MC, MR, NS, P1>>(p, docs, stream);
-  if (need <= P2 * per) return launch<Cfg<WC, WR, MC, MR, NS, P2>>(p, docs, stream);
-  if (need <= P3 * per) return launch<Cfg<WC, WR, MC, MR, NS, P3>>(p, docs, stream);
+hipError_t launch_win(const HiftJobs& jobs, int n, int rows, int cout, hipStream_t stream) {
+  int need = 0;
+  for (int i = 0; i < n; ++i) need = std::max(need, window_rows(jobs.c[i], 32 * MR * WR));
+  const int per = 8 * WC * WR;
+  if (need <= P1 * per) return launch<Cfg<WC, WR, MC, MR, NS, P1>>(jobs, n, rows, cout, stream);
+  if (need <= P2 * per) return launch<Cfg<WC, WR, MC, MR, NS, P2>>(jobs, n, rows, cout, stream);
+  if (need <= P3 * per) return launch<Cfg<WC, WR, MC, MR, NS, P3>>(jobs, n, rows, cout, stream);
   return hipErrorInvalidValue;
+}
+
+bool launchable(const HiftConv& p) {
+  if (!hift_split_eligible(p) || !p.docs || !p.wsplit || !p.winv || !p.amax_in ||
+      p.co_pad % 64 != 0 || p.ldx % 4 != 0 || p.ldo % 4 != 0 || (p.add && p.ld_add % 4 != 0) ||
+      !aligned16(p.x) || !aligned16(p.out) || !aligned16(p.add) || !aligned16(p.accin) ||
+      !aligned16(p.wsplit) || !aligned16(p.winv) || (long)p.co_pad * kRowBytes >= (1L << 31) ||
+      p.n_snakes < 0 || p.n_snakes > 4)
+    return false;
+  for (int i = 0; i < p.n_snakes; ++i)
+    if (!aligned16(p.snakes[i].out) || !p.snakes[i].amax) return false;
+  // channels go four at a time: a partial last group writes zeros into the row's padding and has
+  // no other row or parameter to read
+  return p.cout % 4 == 0 || ((p.cout + 3) / 4 * 4 <= p.ldo && !p.add && !p.snake_out &&
+                             !p.n_snakes && p.mode == HIFT_ACC_WRITE);
 }
 
 }  // namespace
@@ -596,28 +634,28 @@ hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t hift_conv_split(const HiftConv& p, const HiftDocs* docs, hipStream_t stream) {
-  if (p.rows_out <= 0) return hipSuccess;
-  if (!hift_split_eligible(p) || !p.wsplit || !p.winv || !p.amax_in || p.co_pad % 64 != 0 ||
-      p.ldx % 4 != 0 || p.ldo % 4 != 0 || (p.add && p.ld_add % 4 != 0) ||
-      !aligned16(p.x) || !aligned16(p.out) || !aligned16(p.add) || !aligned16(p.accin) ||
-      !aligned16(p.out2) || !aligned16(p.wsplit) || !aligned16(p.winv) ||
-      // channels go four at a time: a partial last group writes zeros into the row's padding and
-      // has no other row or parameter to read
-      (p.cout % 4 != 0 && ((p.cout + 3) / 4 * 4 > p.ldo || p.add || p.snake_out || p.out2 ||
-                           p.mode != HIFT_ACC_WRITE)) ||
-      (long)p.co_pad * kRowBytes >= (1L << 31))
-    return hipErrorInvalidValue;
+hipError_t hift_conv_split(const HiftConv* convs, int n, hipStream_t stream) {
+  if (n < 1 || n > kHiftJobs) return hipErrorInvalidValue;
+  HiftJobs jobs{};
+  int rows = 0, cout = 0;
+  long tiles64 = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!launchable(convs[i])) return hipErrorInvalidValue;
+    jobs.c[i] = convs[i];
+    rows = std::max(rows, convs[i].rows_out);
+    cout = std::max(cout, convs[i].cout);
+    tiles64 += (long)((convs[i].rows_out + 63) / 64) * ((convs[i].cout + 63) / 64);
+  }
+  if (rows <= 0) return hipSuccess;
   // FCV_HIFT_TILE = 32 or 64 forces a tile: a test hook, both must give the same bits
   const char* forced = std::getenv("FCV_HIFT_TILE");
   const int force = forced ? std::atoi(forced) : 0;
-  const long tiles64 = (long)((p.rows_out + 63) / 64) * ((p.cout + 63) / 64);
   const bool small = force ? force == 32 : tiles64 < kSmallBelow;
-  if (p.cout <= 32)
-    return small ? launch_win<1, 1, 1, 1, 8, 4, 8, 12>(p, docs, stream)
-                 : launch_win<1, 4, 1, 1, 3, 2, 5, 6>(p, docs, stream);
-  return small ? launch_win<2, 1, 1, 1, 8, 3, 4, 6>(p, docs, stream)
-               : launch_win<2, 2, 1, 1, 3, 2, 3, 4>(p, docs, stream);
+  if (cout <= 32)
+    return small ? launch_win<1, 1, 1, 1, 8, 4, 8, 12>(jobs, n, rows, cout, stream)
+                 : launch_win<1, 4, 1, 1, 3, 2, 5, 6>(jobs, n, rows, cout, stream);
+  return small ? launch_win<2, 1, 1, 1, 8, 3, 4, 6>(jobs, n, rows, cout, stream)
+               : launch_win<2, 2, 1, 1, 3, 2, 3, 4>(jobs, n, rows, cout, stream);
 }
 
 }  // namespace fcv
