@@ -13,21 +13,23 @@
 //
 // Bound: three f16 MFMAs do a product's work at 16 times the fp32 form's rate each, so the ceiling
 // is a third of the f16 peak against the fp32 peak of 157 TFLOP/s.  Measured on one MI355X against
-// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.2 ms (91 -> 203 TFLOP/s
-// of fp32 work over the whole call), one 68-frame chunk 2.30 -> 1.86 ms, the error against 64 bits
-// 2.5e-5 -> 1.6e-5.  What is left of a large launch is latency: the document table, window and
-// residual reads around 14 to 88 steps of MFMAs, and LDS reads (1.3 KB per MFMA in the 64x64
-// tile).  128x128 and 64x256 tiles (32 KB fewer weight bytes a step, twice the registers) were no
-// faster: 10.7 and 10.8 against 10.4 ms.
+// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.5 ms (91 -> 197 TFLOP/s
+// of fp32 work over the whole call), one 68-frame chunk 2.30 -> 0.94 ms (with the small form below
+// and launches shared by independent convolutions), the error against 64 bits 2.4e-5 -> 1.0e-5.
+// What is left of a large launch is latency: the document table, window and residual reads around
+// 14 to 88 steps of MFMAs, and LDS reads (1.3 KB per MFMA in the 64x64 tile).  128x128 and 64x256
+// tiles (half the weight copies, twice the registers) were no faster: 10.7 and 10.8 against 10.4
+// ms; nor were weights loaded straight into registers, which needs no barrier between steps: 10.8
+// ms with 64x128 tiles.
 //
 // A workgroup owns TR output rows x TC output channels.  For each 32 input channels it splits a
 // window of input rows (the tile's rows and the left context) into LDS once, then walks the taps
 // over it: the input is read and split once, not once per tap.  A tap's weights are one
 // contiguous block of the packed table, copied straight to LDS (global_load_lds) through a ring
-// of NS stages.  Channel chunks outermost, then taps, then k-steps, then the three products: the
-// order of every output's sum is the same in every tile shape, so results do not depend on the
-// shape a launch takes.  (Compiled without floating-point contraction, as the rounding of an
-// output must not depend on the instantiation either.)
+// of NS stages.  Channel chunks outermost (in groups, see kGroups), then taps, then k-steps, then
+// the three products: the order of every output's sum is the same in every tile shape, so results
+// do not depend on the shape a launch takes.  (Compiled without floating-point contraction, as the
+// rounding of an output must not depend on the instantiation either.)
 #include <algorithm>
 #include <cstdlib>
 
@@ -39,10 +41,10 @@ namespace {
 
 constexpr int kRowBytes = 128;  // one row of 32 channels: 4 chunks of hi, 4 of lo, 16 bytes each
 constexpr int kMaxHalo = 62;    // largest left context of a tile, in rows
-// 64x64 tiles in a launch under which 64x32 tiles run (twice the workgroups; above, the larger
-// tile's halved weight traffic is worth more: 286 frames 2.46 -> 2.38 ms at 144 tiles, 68 frames
-// 2.05 against 2.02 ms at 36)
-constexpr long kSmallBelow = 96;
+// 64x64 tiles in a launch (all its convolutions) under which the small form runs.  One call, all
+// small against all 64x64: 24 frames 0.81 and 1.52 ms, 68 0.99 and 1.49, 100 1.19 and 1.53, 200
+// 1.80 and 1.77, 286 2.35 and 1.98; by this rule 1.08, 0.95, 1.11, 1.41 and 1.74.
+constexpr long kSmallBelow = 256;
 
 // position of 16-byte chunk `chunk` in LDS row `row`: 16 consecutive rows read at one chunk index
 // hit 16 distinct 16-byte bank groups
@@ -88,6 +90,11 @@ __device__ __forceinline__ uint32_t amax_serial(const uint32_t* amax, int d) {
   for (int i = 0; i < kAmaxSub; ++i) m = max(m, amax[((long)d * kAmaxSub + i) * kAmaxStride]);
   return m;
 }
+
+// An output's sum is taken over groups of consecutive chunks, each from zero, the groups added in
+// order: at most kGroups of group_chunks(chunks).  A small launch gives each group a wave.
+constexpr int kGroups = 4;
+__device__ __forceinline__ int group_chunks(int chunks) { return (chunks + kGroups - 1) / kGroups; }
 
 // four values, scaled, as their f16 halves
 __device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4& lo) {
@@ -182,6 +189,35 @@ __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& 
   }
 }
 
+// The document of a tile's first row, looked up in one round of loads of the table (documents
+// past 63: searched in memory).
+struct TileDocs {
+  int n_docs, rows_out, in_total, d0, in0, out0, out1;
+  // false: the tile starts past the live rows
+  __device__ __forceinline__ bool load(const HiftDocs* __restrict__ docs, int r0, int lane) {
+    n_docs = docs->n;
+    const int ta = docs->a[lane], tb = docs->b[lane];
+    if (n_docs < 64) {
+      rows_out = __builtin_amdgcn_readlane(tb, n_docs);
+      in_total = __builtin_amdgcn_readlane(ta, n_docs);
+      if (r0 >= rows_out) return false;
+      d0 = __builtin_popcountll(__ballot(lane < n_docs && tb <= r0)) - 1;
+      in0 = __builtin_amdgcn_readlane(ta, d0);
+      out0 = __builtin_amdgcn_readlane(tb, d0);
+      out1 = __builtin_amdgcn_readlane(tb, d0 + 1);
+    } else {
+      rows_out = docs->b[n_docs];
+      in_total = docs->a[n_docs];
+      if (r0 >= rows_out) return false;
+      d0 = doc_of(docs->b, n_docs, r0);
+      in0 = docs->a[d0];
+      out0 = docs->b[d0];
+      out1 = docs->b[d0 + 1];
+    }
+    return true;
+  }
+};
+
 // WC x WR waves; each wave MC x MR tiles of 32 channels x 32 rows.  NS weight stages, NI passes of
 // window loads (kThreads / 8 rows each).
 template <int WC_, int WR_, int MC_, int MR_, int NS_, int NI_>
@@ -197,7 +233,7 @@ struct Cfg {
   static constexpr int kPitch = 32 * MC + 4;                 // staged epilogue row, in floats
   static constexpr int kStage = 32 * kPitch * 4;             // per wave
   static constexpr int kLds = kInfoOff + TR * 20;
-  static constexpr int kMinWaves = kThreads < 256 ? 1 : NI <= 3 ? 4 : 3;  // per SIMD, no spills
+  static constexpr int kMinWaves = kThreads < 256 ? 1 : NI <= 3 ? 4 : 3;  // per SIMD
   static_assert(kWBytes % (1024 * kWaves) == 0, "weight copies");
   static_assert(kStage * kWaves <= kInfoOff, "the epilogue stages in the operand space");
 };
@@ -219,27 +255,10 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   const int wc = wave % C::WC, wr = wave / C::WC;
   const int li = lane & 31, hl = lane >> 5;
   const int r0 = blockIdx.x * C::TR;
-  // the document table in one round of loads (documents past 63: looked up in memory)
-  const int n_docs = docs->n;
-  const int ta = docs->a[lane], tb = docs->b[lane];
-  int rows_out, in_total, d0, in0, out0, out1;
-  if (n_docs < 64) {
-    rows_out = __builtin_amdgcn_readlane(tb, n_docs);
-    in_total = __builtin_amdgcn_readlane(ta, n_docs);
-    if (r0 >= rows_out) return;
-    d0 = __builtin_popcountll(__ballot(lane < n_docs && tb <= r0)) - 1;
-    in0 = __builtin_amdgcn_readlane(ta, d0);
-    out0 = __builtin_amdgcn_readlane(tb, d0);
-    out1 = __builtin_amdgcn_readlane(tb, d0 + 1);
-  } else {
-    rows_out = docs->b[n_docs];
-    in_total = docs->a[n_docs];
-    if (r0 >= rows_out) return;
-    d0 = doc_of(docs->b, n_docs, r0);
-    in0 = docs->a[d0];
-    out0 = docs->b[d0];
-    out1 = docs->b[d0 + 1];
-  }
+  TileDocs td;
+  if (!td.load(docs, r0, lane)) return;
+  const int n_docs = td.n_docs, rows_out = td.rows_out, in_total = td.in_total;
+  const int d0 = td.d0, in0 = td.in0, out0 = td.out0, out1 = td.out1;
   const bool one_doc = min(r0 + C::TR, rows_out) <= out1;  // of the tile's rows
   const int co0 = blockIdx.y * C::TC;
   if (co0 >= p.cout) return;
@@ -320,22 +339,32 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
     }
   };
 
-  f32x16 acc[C::MC][C::MR];
+  // the sum of the chunk group at hand, and of the groups before it
+  f32x16 acc[C::MC][C::MR], total[C::MC][C::MR];
 #pragma unroll
   for (int a = 0; a < C::MC; ++a)
 #pragma unroll
     for (int b = 0; b < C::MR; ++b)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) acc[a][b][e] = total[a][b][e] = 0.0f;
+  const int per_group = group_chunks(chunks);
+  auto end_group = [&]() {
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          total[a][b][e] = total[a][b][e] + acc[a][b][e];
+          acc[a][b][e] = 0.0f;
+        }
+  };
 
   fetch_x(0);
-  // the epilogue's per-channel inputs, loaded here so that nothing waits for them there
   constexpr int LPR = 8 * C::MC;              // lanes per staged output row
   const int cl = (lane % LPR) * 4;            // channel within the wave's columns
   const int c4 = co0 + wc * C::MC * 32 + cl;
   const bool live_c = c4 < p.cout;
-  SplitCols cols;
-  cols.load(p, live_c ? c4 : 0);
   __syncthreads();  // the row table
   // this lane's rows: window row and input position of tap 0; up > 1 walks (position, remainder)
   int wrow0[C::MR], q0[C::MR], rem0[C::MR];
@@ -355,21 +384,17 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 
   // Two fragment buffers: the reads of k-step ks + 1 are in flight while the MFMAs of ks run.  A
   // step's second k-step runs after the barrier that publishes the next step, over that step's
-  // first reads.  In an LDS row the 16-byte chunk of k-step ks (hi, then lo) sits at byte
+  // first reads.  A weight block of 32 channels is 4 KB: k-steps 0 and 1, hi then lo, lane l's 16
+  // bytes at 16 l.  In an input row the 16-byte chunk of k-step ks (hi, then lo) sits at byte
   // (16 (hl ^ rot)) ^ 32 ks (^ 64 for lo), rot = (row / 2) % 8.
   f16x8 wh[2][C::MC], wl[2][C::MC], xh[2][C::MR], xl[2][C::MR];
-  uint32_t woff[C::MC];
-#pragma unroll
-  for (int a = 0; a < C::MC; ++a) {
-    const int row = (wc * C::MC + a) * 32 + li;
-    woff[a] = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
-  }
+  const uint32_t woff = wc * C::MC * 4096 + lane * 16;
   uint32_t xoff_l[C::MR];
   auto load = [&](int buf, int ks, const char* sW) {
 #pragma unroll
     for (int a = 0; a < C::MC; ++a) {
-      wh[buf][a] = *reinterpret_cast<const f16x8*>(sW + (woff[a] ^ (32 * ks)));
-      wl[buf][a] = *reinterpret_cast<const f16x8*>(sW + (woff[a] ^ (32 * ks + 64)));
+      wh[buf][a] = *reinterpret_cast<const f16x8*>(sW + woff + a * 4096 + ks * 2048);
+      wl[buf][a] = *reinterpret_cast<const f16x8*>(sW + woff + a * 4096 + ks * 2048 + 1024);
     }
 #pragma unroll
     for (int b = 0; b < C::MR; ++b) {
@@ -394,7 +419,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  int s = 0, stage_s = 0;
+  int s = 0, stage_s = 0, in_group = 0;
   for (int c = 0; c < chunks; ++c) {
     int q[C::MR], rem[C::MR], wrow[C::MR];
 #pragma unroll
@@ -405,6 +430,10 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       wait_lgkm0();
       __syncthreads();
       mma(1);
+      if (++in_group == per_group) {
+        end_group();
+        in_group = 0;
+      }
     }
     stash_x();
     for (int j = 0; j < k; ++j, ++s) {
@@ -444,6 +473,9 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
     }
   }
   mma(1);
+  end_group();
+  SplitCols cols;
+  cols.load(p, live_c ? c4 : 0);
   wait_vm<0>();
   wait_lgkm0();
   __syncthreads();  // the operand space becomes the waves' staging space
@@ -470,8 +502,8 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
     for (int a = 0; a < C::MC; ++a)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const f32x4 v{acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2],
-                      acc[a][b][4 * g + 3]};
+        const f32x4 v{total[a][b][4 * g], total[a][b][4 * g + 1], total[a][b][4 * g + 2],
+                      total[a][b][4 * g + 3]};
         *reinterpret_cast<f32x4*>(stage + li * C::kPitch + a * 32 + g * 8 + hl * 4) = v;
       }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -528,9 +560,213 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   }
 }
 
+// The small launches' form: a workgroup owns one 32x32 tile, and each of its kGroups waves sums one
+// group of input chunks, on its own window and with its weights loaded straight into registers PD
+// steps ahead: no wave waits for another until the sums are added.  A step here is latency, some
+// 900 cycles around 192 of MFMAs with one wave on a SIMD (counters of a 68-frame chunk), so the
+// shorter chain is what counts.
+template <int NI, int PD>
+__global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const HiftJobs jobs) {
+  constexpr int kWin = NI * 8, kWinBytes = kWin * kRowBytes, kPitch = 36;
+  constexpr int kStage = 32 * kPitch * 4;  // a group's 32x32 sums
+  constexpr int kPart = kWinBytes + kRowBytes > kStage ? kWinBytes + kRowBytes : kStage;
+  const HiftConv& p = jobs.c[blockIdx.z];
+  const HiftDocs* __restrict__ docs = p.docs;
+  __shared__ __attribute__((aligned(1024))) char smem[kGroups * kPart];
+  __shared__ float wmax[kGroups][5];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, hl = lane >> 5;
+  const int r0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
+  TileDocs td;
+  if (!td.load(docs, r0, lane)) return;
+  if (co0 >= p.cout) return;
+  const bool one_doc = min(r0 + 32, td.rows_out) <= td.out1;
+  const int chunks = p.cin_pad / 32, k = p.k;
+  const int per_group = group_chunks(chunks);
+  const int c_begin = wave * per_group, c_end = min(c_begin + per_group, chunks);
+  char* win = smem + wave * kPart;
+
+  const int u0 = r0 - td.out0 - p.pad;
+  const int win0 = td.in0 + (u0 > 0 ? u0 / p.up : 0);
+  const int f0 = scale_field(doc_amax(p.amax_in, td.d0, lane));
+  auto row_field = [&](int d) {
+    return d == td.d0 ? f0 : scale_field(amax_serial(p.amax_in, d));
+  };
+
+  if (c_begin < c_end) {
+    const char* wbase = static_cast<const char*>(p.wsplit) + (long)(co0 / 32) * 4096;
+    const long wstep = (long)p.co_pad * kRowBytes;
+    const int s_end = c_end * k;
+    f16x8 w[PD][4];
+    auto fetch_w = [&](f16x8 (&f)[4], int s) {
+      const char* src = wbase + (long)min(s, s_end - 1) * wstep;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        f[i] = *reinterpret_cast<const f16x8*>(src + lane * 16 + i * 1024);
+    };
+#pragma unroll
+    for (int i = 0; i < PD - 1; ++i) fetch_w(w[i], c_begin * k + i);
+
+    // window pass i, lane l: row 8 i + l / 8, channels 4 (l % 8)
+    const float* X = static_cast<const float*>(p.x) + (lane & 7) * 4;
+    long xoff[NI];
+    float xs[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int row = min(win0 + i * 8 + (lane >> 3), td.in_total - 1);
+      xoff[i] = (long)row * p.ldx;
+      xs[i] = field_to_float(one_doc ? f0 : row_field(doc_of(docs->a, td.n_docs, row)));
+    }
+    f32x4 xr[NI];
+    auto fetch_x = [&](int c) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) xr[i] = *reinterpret_cast<const f32x4*>(X + xoff[i] + c * 32);
+    };
+    auto stash_x = [&]() {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        f32x4 v = xr[i];
+        if (p.pro == HIFT_PRO_LEAKY) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * p.slope;
+        }
+        f16x4 hi, lo;
+        split4(v, xs[i], hi, lo);
+        const int row = i * 8 + (lane >> 3);
+        char* dst = win + row * kRowBytes + (lane & 1) * 8;
+        *reinterpret_cast<f16x4*>(dst + 16 * swz(row, (lane & 7) >> 1)) = hi;
+        *reinterpret_cast<f16x4*>(dst + 16 * swz(row, 4 + ((lane & 7) >> 1))) = lo;
+      }
+    };
+    fetch_x(c_begin);
+    // the wave's zero row, and this lane's row: window row and input position of tap 0
+    if (lane < 8) *reinterpret_cast<f32x4*>(win + kWinBytes + lane * 16) = f32x4{0, 0, 0, 0};
+    int q0 = -(1 << 29), rem0 = 0, wrow0 = 0;
+    if (r0 + li < td.rows_out) {
+      const int d = one_doc ? td.d0 : doc_of(docs->b, td.n_docs, r0 + li);
+      const int u = r0 + li - (one_doc ? td.out0 : docs->b[d]) - p.pad;
+      q0 = u;
+      if (p.up > 1) {
+        q0 = u >= 0 ? u / p.up : -((-u + p.up - 1) / p.up);
+        rem0 = u - q0 * p.up;
+      }
+      wrow0 = (one_doc ? td.in0 : docs->a[d]) - win0 + q0;
+    }
+    stash_x();
+    if (c_begin + 1 < c_end) fetch_x(c_begin + 1);
+
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    int q = q0, rem = rem0, wrow = wrow0, c = c_begin, j = 0;
+    for (int s0 = c_begin * k; s0 < s_end; s0 += PD) {
+#pragma unroll
+      for (int u = 0; u < PD; ++u) {
+        if (s0 + u >= s_end) break;
+        if (j == k) {  // the next chunk's window (LDS accesses of one wave stay in order)
+          j = 0;
+          ++c;
+          q = q0; rem = rem0; wrow = wrow0;
+          stash_x();
+          if (c + 1 < c_end) fetch_x(c + 1);
+        }
+        fetch_w(w[(u + PD - 1) % PD], s0 + u + PD - 1);
+        const bool ok = q >= 0 && (unsigned)wrow < (unsigned)kWin;
+        const int row = ok ? wrow : kWin;
+        const uint32_t off = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
+        if (p.up > 1) {
+          rem += 1;
+          const int step = rem == p.up ? 1 : 0;
+          rem = step ? 0 : rem;
+          q += step;
+          wrow += step;
+        } else {
+          q += p.dil;
+          wrow += p.dil;
+        }
+        ++j;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const f16x8 xh = *reinterpret_cast<const f16x8*>(win + (off ^ (32 * ks)));
+          const f16x8 xl = *reinterpret_cast<const f16x8*>(win + (off ^ (32 * ks + 64)));
+          acc = mfma32(w[u][2 * ks + 1], xh, acc);
+          acc = mfma32(w[u][2 * ks], xl, acc);
+          acc = mfma32(w[u][2 * ks], xh, acc);
+        }
+      }
+    }
+    // the sums go where the window was: this wave has read it
+    float* stage = reinterpret_cast<float*>(win);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 v{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+      *reinterpret_cast<f32x4*>(stage + li * kPitch + g * 8 + hl * 4) = v;
+    }
+  }
+
+  // eight rows a wave, eight lanes a row
+  constexpr int kRows = 32 / kGroups;
+  const int t = wave * kRows + (lane >> 3), r = r0 + t, cl = (lane & 7) * 4, c4 = co0 + cl;
+  const bool live = r < td.rows_out && c4 < p.cout;
+  SplitCols cols;
+  SplitAdds in;
+  int d = td.d0, pos = 0;
+  long row = r;
+  if (live) {
+    if (!one_doc) d = doc_of(docs->b, td.n_docs, r);
+    pos = r - (one_doc ? td.out0 : docs->b[d]);
+    if (p.reflect) row = (long)r + d + 1;
+    cols.load(p, c4);
+    in.load(p, row, c4);
+  }
+  wait_lgkm0();
+  __syncthreads();
+  float m1 = 0.0f, m2[4] = {};
+  const int sub = blockIdx.x + blockIdx.y;
+  if (live) {
+    f32x4 v{0, 0, 0, 0};
+    for (int g = 0; g * per_group < chunks; ++g)
+      v += *reinterpret_cast<const f32x4*>(smem + g * kPart + (t * kPitch + cl) * 4);
+    const float inv = field_to_float(254 - row_field(d));
+    split_store(p, cols, in, row, c4, v, inv, m1, m2);
+    // reflection padding (1, 0): row 0 of the document repeats the result's row 1
+    if (p.reflect && pos == 1) {
+      SplitAdds first;
+      first.load(p, (long)r - 1 + d, c4);
+      split_store(p, cols, first, (long)r - 1 + d, c4, v, inv, m1, m2);
+    }
+    if (!one_doc) {
+      if (p.amax_out) raise_amax(p.amax_out, d, sub, m1);
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        if (n < p.n_snakes) raise_amax(p.snakes[n].amax, d, sub, m2[n]);
+    }
+  }
+  if (one_doc && (p.amax_out || p.n_snakes)) {
+    m1 = wave_max(m1);
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (n < p.n_snakes) m2[n] = wave_max(m2[n]);
+    if (lane == 0) {
+      wmax[wave][0] = m1;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) wmax[wave][1 + n] = m2[n];
+    }
+    __syncthreads();
+    if (tid <= p.n_snakes) {
+      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[tid - 1].amax;
+      float m = 0.0f;
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) m = fmaxf(m, wmax[g][tid]);
+      if (slot) raise_amax(slot, td.d0, sub, m);
+    }
+  }
+}
+
 // One wave per output channel of [co_pad][k][cin] weights: the row's scale from its largest finite
-// weight, then both halves at [chunk][tap][co][64 f16], the 16-byte chunks of a row in their LDS
-// order; inv[co] = the inverse scale, inv[co_pad + co] = the bias (zero past cout).
+// weight, then both halves in the order the kernels' fragments take them; inv[co] = the inverse scale, inv[co_pad + co] = the bias (zero past cout).
 __global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict__ w,
                                                         const float* __restrict__ bias, int cout,
                                                         int co_pad, int k, int cin,
@@ -553,10 +789,11 @@ __global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict_
     const int tap = i * 4 / cin, c = i * 4 - tap * cin;
     f16x4 hi, lo;
     split4(*reinterpret_cast<const f32x4*>(row + i * 4), s, hi, lo);
-    f16* out = dst + (((long)(c / 32) * k + tap) * co_pad + co) * 64 + (c & 4);
-    const int unit = (c & 31) >> 3;
-    *reinterpret_cast<f16x4*>(out + 8 * swz(co, unit)) = hi;
-    *reinterpret_cast<f16x4*>(out + 8 * swz(co, unit + 4)) = lo;
+    // [step][32-channel block][k-step][hi, lo][lane][8]: lane = co % 32 + 32 ((c / 8) % 2)
+    f16* out = dst + (((long)(c / 32) * k + tap) * co_pad + (co & ~31)) * 64 +
+               ((c >> 4) & 1) * 1024 + ((co & 31) + 32 * ((c >> 3) & 1)) * 8 + (c & 4);
+    *reinterpret_cast<f16x4*>(out) = hi;
+    *reinterpret_cast<f16x4*>(out + 512) = lo;
   }
 }
 
@@ -590,6 +827,22 @@ hipError_t launch_win(const HiftJobs& jobs, int n, int rows, int cout, hipStream
   if (need <= P1 * per) return launch<Cfg<WC, WR, MC, MR, NS, P1>>(jobs, n, rows, cout, stream);
   if (need <= P2 * per) return launch<Cfg<WC, WR, MC, MR, NS, P2>>(jobs, n, rows, cout, stream);
   if (need <= P3 * per) return launch<Cfg<WC, WR, MC, MR, NS, P3>>(jobs, n, rows, cout, stream);
+  return hipErrorInvalidValue;
+}
+
+// the small form with the window passes (8 rows each) the launch needs
+template <int NI>
+hipError_t launch_small_ni(const HiftJobs& jobs, int n, int rows, int cout, hipStream_t stream) {
+  const dim3 grid((rows + 31) / 32, (cout + 31) / 32, n);
+  hipLaunchKernelGGL((split_conv_small_kernel<NI, 4>), grid, dim3(64 * kGroups), 0, stream, jobs);
+  return hipGetLastError();
+}
+hipError_t launch_small(const HiftJobs& jobs, int n, int rows, int cout, hipStream_t stream) {
+  int need = 0;
+  for (int i = 0; i < n; ++i) need = std::max(need, window_rows(jobs.c[i], 32));
+  if (need <= 4 * 8) return launch_small_ni<4>(jobs, n, rows, cout, stream);
+  if (need <= 8 * 8) return launch_small_ni<8>(jobs, n, rows, cout, stream);
+  if (need <= 12 * 8) return launch_small_ni<12>(jobs, n, rows, cout, stream);
   return hipErrorInvalidValue;
 }
 
@@ -651,11 +904,9 @@ hipError_t hift_conv_split(const HiftConv* convs, int n, hipStream_t stream) {
   const char* forced = std::getenv("FCV_HIFT_TILE");
   const int force = forced ? std::atoi(forced) : 0;
   const bool small = force ? force == 32 : tiles64 < kSmallBelow;
-  if (cout <= 32)
-    return small ? launch_win<1, 1, 1, 1, 8, 4, 8, 12>(jobs, n, rows, cout, stream)
-                 : launch_win<1, 4, 1, 1, 3, 2, 5, 6>(jobs, n, rows, cout, stream);
-  return small ? launch_win<2, 1, 1, 1, 8, 3, 4, 6>(jobs, n, rows, cout, stream)
-               : launch_win<2, 2, 1, 1, 3, 2, 3, 4>(jobs, n, rows, cout, stream);
+  if (small) return launch_small(jobs, n, rows, cout, stream);
+  if (cout <= 32) return launch_win<1, 4, 1, 1, 3, 2, 5, 6>(jobs, n, rows, cout, stream);
+  return launch_win<2, 2, 1, 1, 3, 2, 3, 4>(jobs, n, rows, cout, stream);
 }
 
 }  // namespace fcv
