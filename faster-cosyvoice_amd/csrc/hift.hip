@@ -2,15 +2,16 @@
 //
 // Every convolution of the vocoder is one implicit GEMM on the matrix cores.  The causal
 // unit-stride ones (upsampling, resblocks, conv_post) run in hift_split.hip where the handle has
-// split weights; the rest -- the fp64 F0 predictor, conv_pre, the strided source convs -- run
-// here on v_mfma_{f32,f64}_16x16x4: weights are the A operand (rows = output channels),
+// split weights; the rest -- conv_pre, the strided source convs, and the fp64 F0 predictor with a
+// kernel of its own -- run here on v_mfma_{f32,f64}_16x16x4: weights are the A operand (rows = output channels),
 // the gathered input rows the B operand, so a lane's four accumulators are four channels of one
 // time step (consecutive in fp32; four apart in fp64, whose 16x16 result is laid out by rows
-// 4 e + lane / 16).  Operands go through LDS K-contiguous, 32 (or 16) input channels of one tap
-// per chunk, with a register-prefetched double buffer.  A workgroup owns 64 time rows x 64
-// output channels (32 x 32 in launches too small to give every CU a 64 x 64 tile).  Activations that sit between two convolutions are fused: LeakyReLU into the
-// input prologue, bias, ELU, residual add, Snake and the resblock mean into the epilogue, and
-// the epilogue can also write Snake(y) as a second output for the next conv.
+// 4 e + lane / 16).  Operands of the fp32 convolutions go through LDS K-contiguous, 32 (or 16)
+// input channels of one tap per chunk, with a register-prefetched double buffer.  A workgroup owns
+// 64 time rows x 64 output channels (32 x 32 in launches too small to give every CU a 64 x 64
+// tile).  Activations that sit between two convolutions are fused: LeakyReLU into the input
+// prologue, bias, ELU, residual add, Snake and the resblock mean into the epilogue, and the
+// epilogue can also write Snake(y) as a second output for the next conv.
 #include <math.h>
 
 #include <cstdlib>
@@ -27,9 +28,6 @@ constexpr long kSmallTileBelow = 256;  // 64x64 tiles per launch under which 32x
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-template <typename T> struct Vec4;
-template <> struct Vec4<float> { using type = f32x4; };
-template <> struct Vec4<double> { using type = f64x4; };
 
 __device__ __forceinline__ f32x4 mfma_16x16x4(float a, float b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -38,31 +36,24 @@ __device__ __forceinline__ f64x4 mfma_16x16x4(double a, double b, const f64x4& c
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-template <typename T>
-__device__ __forceinline__ T elu(T x) { return x > T(0) ? x : T(expm1(x)); }
+__device__ __forceinline__ double elu(double x) { return x > 0.0 ? x : expm1(x); }
 
 // epilogue of one output element (row, channel c) from its accumulator value; m: raised to the
 // largest finite magnitudes written to out and to the Snake output (fp32)
-template <typename T>
-__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, T acc, float2& m) {
-  T v = acc + static_cast<const T*>(p.bias)[c];
-  if constexpr (sizeof(T) == 8) {
-    if (p.elu) v = elu(v);
-  }
+__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, float acc, float2& m) {
+  float v = acc + static_cast<const float*>(p.bias)[c];
   const long i = row * p.ldo + c;
-  if (p.add) v = v + static_cast<const T*>(p.add)[row * p.ld_add + c];
-  if (p.mode == HIFT_ACC_ADD) v = static_cast<const T*>(p.accin)[i] + v;
-  if (p.mode == HIFT_ACC_ADD_DIV) v = (static_cast<const T*>(p.accin)[i] + v) / T(p.div);
-  if constexpr (sizeof(T) == 4) {
-    if (p.snake_out) v = snake(v, p.alpha[c], p.inv_alpha[c]);
-    if (p.n_snakes) {
-      const float w = snake(v, p.snakes[0].alpha[c], p.snakes[0].inv_alpha[c]);
-      p.snakes[0].out[i] = w;
-      m.y = fmaxf(m.y, finite_abs(w));
-    }
-    m.x = fmaxf(m.x, finite_abs(v));
+  if (p.add) v = v + static_cast<const float*>(p.add)[row * p.ld_add + c];
+  if (p.mode == HIFT_ACC_ADD) v = static_cast<const float*>(p.accin)[i] + v;
+  if (p.mode == HIFT_ACC_ADD_DIV) v = (static_cast<const float*>(p.accin)[i] + v) / p.div;
+  if (p.snake_out) v = snake(v, p.alpha[c], p.inv_alpha[c]);
+  if (p.n_snakes) {
+    const float w = snake(v, p.snakes[0].alpha[c], p.snakes[0].inv_alpha[c]);
+    p.snakes[0].out[i] = w;
+    m.y = fmaxf(m.y, finite_abs(w));
   }
-  static_cast<T*>(p.out)[i] = v;
+  m.x = fmaxf(m.x, finite_abs(v));
+  static_cast<float*>(p.out)[i] = v;
 }
 
 __device__ __forceinline__ float4 ld4f(const float* q) { return *reinterpret_cast<const float4*>(q); }
@@ -103,21 +94,17 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
   *reinterpret_cast<float4*>(static_cast<float*>(p.out) + i) = float4{v[0], v[1], v[2], v[3]};
 }
 
-// The 16x16x4 accumulators of lane (li, lg) hold, for the tile's channel base cb:
-//   fp32: channels cb + 4 lg + e;  fp64: channels cb + 4 e + lg  (e = 0..3)
-template <typename T>
+// The 16x16x4 accumulators of lane (li, lg) hold channels cb + 4 lg + e (e = 0..3) of the tile's
+// channel base cb
 __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
-                           const typename Vec4<T>::type& acc, float2& m) {
-  if constexpr (sizeof(T) == 4) {
-    if (p.vec4 && cb + 4 * lg + 3 < p.cout) {
-      conv_store4(p, row, cb + 4 * lg, acc, m);
-      return;
-    }
+                           const f32x4& acc, float2& m) {
+  const int c = cb + 4 * lg;
+  if (p.vec4 && c + 3 < p.cout) {
+    conv_store4(p, row, c, acc, m);
+    return;
   }
-  for (int e = 0; e < 4; ++e) {
-    const int c = sizeof(T) == 4 ? cb + 4 * lg + e : cb + 4 * e + lg;
-    if (c < p.cout) conv_store1<T>(p, row, c, acc[e], m);
-  }
+  for (int e = 0; e < 4; ++e)
+    if (c + e < p.cout) conv_store1(p, row, c + e, acc[e], m);
 }
 
 // BK input channels of one tap per chunk (cin_pad % BK == 0), each lane feeding
@@ -128,16 +115,16 @@ __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
 // waves 2-3 the input rows, the same groups each.  Every output element accumulates the chunks
 // in the same order with the same lane/slot -> k rule at both sizes, so the tile size does not
 // change a result.
-template <typename T, int BK, int TS>
+template <int BK, int TS>
 __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
   const HiftDocs* __restrict__ docs = p.docs;
-  using VT = typename Vec4<T>::type;
+  using VT = f32x4;
   constexpr int PITCH = BK + 4;  // LDS row pitch in elements (conflict-free 16-byte reads)
   constexpr int G = BK / 16;
   constexpr int NQ = TS / 32;    // 16x16 accumulator tiles per wave along each side
   static_assert(TS == 64 || TS == 32, "tile size");
-  __shared__ __attribute__((aligned(16))) T sA[2][TS][PITCH];
-  __shared__ __attribute__((aligned(16))) T sB[2][TS][PITCH];
+  __shared__ __attribute__((aligned(16))) float sA[2][TS][PITCH];
+  __shared__ __attribute__((aligned(16))) float sB[2][TS][PITCH];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -166,8 +153,8 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
     in_base = docs->a[d];
     in_len = docs->a[d + 1] - in_base;
   }
-  const T* X = static_cast<const T*>(p.x);
-  const T* W = static_cast<const T*>(p.w) + (long)(co0 + lr) * kcin + 4 * lq;
+  const float* X = static_cast<const float*>(p.x);
+  const float* W = static_cast<const float*>(p.w) + (long)(co0 + lr) * kcin + 4 * lq;
 
   // Two register sets: the loads of chunk kc + 2 are issued while chunk kc is computed and
   // chunk kc + 1 (loaded one iteration earlier) is written to LDS, so every load has about two
@@ -179,11 +166,11 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
     const int u = pos * p.stride + tap * p.dil - p.pad;
     const int q = p.up > 1 ? (u >= 0 ? u / p.up : -1) : u;
     const bool live = valid && q >= 0 && q < in_len;
-    const T* xr = X + (long)(in_base + q) * p.ldx + c0;
+    const float* xr = X + (long)(in_base + q) * p.ldx + c0;
 #pragma unroll
     for (int m = 0; m < G; ++m) {
       if (ld_w) a[m] = *reinterpret_cast<const VT*>(W + (long)kc * BK + 16 * m);
-      b[m] = VT{T(0), T(0), T(0), T(0)};
+      b[m] = VT{0.0f, 0.0f, 0.0f, 0.0f};
       if (live) b[m] = *reinterpret_cast<const VT*>(xr + 16 * m);
     }
   };
@@ -192,11 +179,9 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
 #pragma unroll
     for (int m = 0; m < G; ++m) {
       VT bm = b[m];
-      if constexpr (sizeof(T) == 4) {
-        if (p.pro == HIFT_PRO_LEAKY) {
+      if (p.pro == HIFT_PRO_LEAKY) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) bm[e] = bm[e] > 0.0f ? bm[e] : bm[e] * p.slope;
-        }
+        for (int e = 0; e < 4; ++e) bm[e] = bm[e] > 0.0f ? bm[e] : bm[e] * p.slope;
       }
       if (ld_w) *reinterpret_cast<VT*>(&sA[buf][lr][16 * m + 4 * lq]) = a[m];
       if (ld_x) *reinterpret_cast<VT*>(&sB[buf][lr][16 * m + 4 * lq]) = bm;
@@ -207,7 +192,7 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
 #pragma unroll
   for (int a = 0; a < NQ; ++a)
 #pragma unroll
-    for (int b = 0; b < NQ; ++b) acc[a][b] = VT{T(0), T(0), T(0), T(0)};
+    for (int b = 0; b < NQ; ++b) acc[a][b] = VT{0.0f, 0.0f, 0.0f, 0.0f};
 
   auto compute = [&](int cur) {
 #pragma unroll
@@ -267,35 +252,31 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
       const int cb = co0 + wc * (TS / 2) + a * 16;
-      conv_store<T>(p, row_w, cb, lg, acc[a][b], m);
+      conv_store(p, row_w, cb, lg, acc[a][b], m);
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
-      if (p.reflect && pp == 1) conv_store<T>(p, (long)docs->b[d] + d, cb, lg, acc[a][b], m);
+      if (p.reflect && pp == 1) conv_store(p, (long)docs->b[d] + d, cb, lg, acc[a][b], m);
     }
-    if constexpr (sizeof(T) == 4) {
-      if (one_doc) {
-        tile_max.x = fmaxf(tile_max.x, m.x);
-        tile_max.y = fmaxf(tile_max.y, m.y);
-      } else {
-        if (p.amax_out) raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m.x);
-        if (p.snakes[0].amax) raise_amax(p.snakes[0].amax, d, blockIdx.x + blockIdx.y, m.y);
-      }
+    if (one_doc) {
+      tile_max.x = fmaxf(tile_max.x, m.x);
+      tile_max.y = fmaxf(tile_max.y, m.y);
+    } else {
+      if (p.amax_out) raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m.x);
+      if (p.snakes[0].amax) raise_amax(p.snakes[0].amax, d, blockIdx.x + blockIdx.y, m.y);
     }
   }
-  if constexpr (sizeof(T) == 4) {
-    if (one_doc && (p.amax_out || p.snakes[0].amax)) {
-      __shared__ float wmax[2][4];
-      tile_max.x = wave_max(tile_max.x);
-      tile_max.y = wave_max(tile_max.y);
-      if (lane == 0) {
-        wmax[0][wave] = tile_max.x;
-        wmax[1][wave] = tile_max.y;
-      }
-      __syncthreads();
-      if (tid < 2) {
-        uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[0].amax;
-        const float m = fmaxf(fmaxf(wmax[tid][0], wmax[tid][1]), fmaxf(wmax[tid][2], wmax[tid][3]));
-        if (slot) raise_amax(slot, tile_doc, blockIdx.x + blockIdx.y, m);
-      }
+  if (one_doc && (p.amax_out || p.snakes[0].amax)) {
+    __shared__ float wmax[2][4];
+    tile_max.x = wave_max(tile_max.x);
+    tile_max.y = wave_max(tile_max.y);
+    if (lane == 0) {
+      wmax[0][wave] = tile_max.x;
+      wmax[1][wave] = tile_max.y;
+    }
+    __syncthreads();
+    if (tid < 2) {
+      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[0].amax;
+      const float m = fmaxf(fmaxf(wmax[tid][0], wmax[tid][1]), fmaxf(wmax[tid][2], wmax[tid][3]));
+      if (slot) raise_amax(slot, tile_doc, blockIdx.x + blockIdx.y, m);
     }
   }
 }
@@ -369,12 +350,96 @@ __global__ __launch_bounds__(256) void mean_kernel(const HiftMean in, float* __r
   raise_rows_amax(amax, m, first, i, total, q, docs);
 }
 
-__global__ __launch_bounds__(256) void to_f64_kernel(const float* __restrict__ x,
-                                                     double* __restrict__ y, int C,
-                                                     const HiftDocs* __restrict__ docs) {
-  const long n = (long)docs->a[docs->n] * C;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = (double)x[i];
+// One layer of the fp64 F0 predictor on v_mfma_f64_16x16x4: out[r][co] = elu(b[co] + sum_k W[co][k]
+// x[r + tap][c]), k = tap * cin + c.  A workgroup owns a 16 T x 16 T tile and its four waves a
+// quarter of K each (added in order in LDS), straight from global memory: these products have 72 to
+// a few thousand rows, so what counts is the chain of MFMAs a wave runs (64 cycles each), and a
+// quarter of K on four times the waves cuts it to a quarter.  One layer at 72 rows 44 -> 15 us
+// against 32x32 tiles with K in one chain through LDS (1664 rows: the same); T = 2 halves the operand reads where 16x16
+// tiles would be many (the sums are the same).
+template <typename X, int T>
+__global__ __launch_bounds__(256) void f0_conv_kernel(const HiftConv p) {
+  constexpr int TS = 16 * T;
+  const HiftDocs* __restrict__ docs = p.docs;
+  __shared__ double part[4][TS][TS + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int n_docs = docs->n, rows_out = docs->b[n_docs];
+  const int r0 = blockIdx.x * TS, co0 = blockIdx.y * TS;
+  if (r0 >= rows_out) return;
+  const int K = p.k * p.cin_pad, quarter = K / 4;
+  const int k_begin = wave * quarter, k_end = k_begin + quarter;
+
+  // lane (li, lg) holds k = k0 + 4 lg + 0..3 of weight row li and of input row li
+  const double* W[T];
+  int pos[T], in_base[T], in_len[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    W[i] = static_cast<const double*>(p.w) + (long)(co0 + 16 * i + li) * K + 4 * lg;
+    const int r = r0 + 16 * i + li;
+    pos[i] = -(1 << 29);
+    in_base[i] = in_len[i] = 0;
+    if (r < rows_out) {
+      const int d = doc_of(docs->b, n_docs, r);
+      pos[i] = r - docs->b[d] - p.pad;
+      in_base[i] = docs->a[d];
+      in_len[i] = docs->a[d + 1] - in_base[i];
+    }
+  }
+  const X* x = static_cast<const X*>(p.x) + 4 * lg;
+  constexpr int PD = T == 1 ? 4 : 2;
+  f64x4 wa[PD][T], xb[PD][T];
+  auto fetch = [&](int slot, int k0) {
+    const int tap = k0 / p.cin_pad, c = k0 - tap * p.cin_pad;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      wa[slot][i] = *reinterpret_cast<const f64x4*>(W[i] + k0);
+      const int q = pos[i] + tap;
+      xb[slot][i] = f64x4{0.0, 0.0, 0.0, 0.0};
+      if (q >= 0 && q < in_len[i]) {
+        typedef X x4 __attribute__((ext_vector_type(4)));
+        const x4 v = *reinterpret_cast<const x4*>(x + (long)(in_base[i] + q) * p.ldx + c);
+        xb[slot][i] = f64x4{(double)v[0], (double)v[1], (double)v[2], (double)v[3]};
+      }
+    }
+  };
+  f64x4 acc[T][T];
+#pragma unroll
+  for (int a = 0; a < T; ++a)
+#pragma unroll
+    for (int b = 0; b < T; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < PD - 1; ++u) fetch(u, min(k_begin + 16 * u, k_end - 16));
+  for (int k0 = k_begin; k0 < k_end; k0 += 16 * PD) {
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+      const int kk = k0 + 16 * u;
+      if (kk >= k_end) break;
+      fetch((u + PD - 1) % PD, min(kk + 16 * (PD - 1), k_end - 16));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int a = 0; a < T; ++a)
+#pragma unroll
+          for (int b = 0; b < T; ++b)
+            acc[a][b] = mfma_16x16x4(wa[u][a][e], xb[u][b][e], acc[a][b]);
+    }
+  }
+  // D: lane holds row li, channels 4 e + lg
+#pragma unroll
+  for (int a = 0; a < T; ++a)
+#pragma unroll
+    for (int b = 0; b < T; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[wave][16 * b + li][16 * a + 4 * e + lg] = acc[a][b][e];
+  __syncthreads();
+  for (int i = tid; i < TS * TS; i += 256) {
+    const int t = i / TS, c = i - t * TS;
+    if (r0 + t >= rows_out || co0 + c >= p.cout) continue;
+    const double v = ((part[0][t][c] + part[1][t][c]) + part[2][t][c]) + part[3][t][c];
+    static_cast<double*>(p.out)[(long)(r0 + t) * p.ldo + co0 + c] =
+        elu(v + static_cast<const double*>(p.bias)[co0 + c]);
+  }
 }
 
 __global__ __launch_bounds__(64) void f0_head_kernel(const double* __restrict__ h, int C,
@@ -391,20 +456,24 @@ __global__ __launch_bounds__(64) void f0_head_kernel(const double* __restrict__ 
   if (threadIdx.x == 0) f0[r] = (float)fabs(s + b[0]);
 }
 
-// One thread per (document, harmonic): the per-frame phase increment of harmonic h is
+// One workgroup per (document, harmonic): the per-frame phase increment of harmonic h is
 // rad = frac(f0 (h+1) / sr); the frame-rate value is the linear interpolation the reference
 // takes from the sample-rate sequence (whose first sample also carries rand_ini[h]); the
 // phase is the running sum in frame order, times 2 pi, times the upsampling scale.  The running
 // sum is held in fp64 and rounded to fp32 at every frame, which is what the reference's
 // torch.cumsum over the fp32 rad values (cosyvoice/hifigan/generator.py:255) computes on the
 // CPU, whose kernel accumulates fp32 in double: an fp32 running sum drifts by ~1e-6 relative
-// per few hundred frames, and the phase multiplies that by 2 pi x 480.
-__global__ __launch_bounds__(64) void source_phase_kernel(const HiftSource p,
-                                                          const HiftDocs* __restrict__ docs) {
+// per few hundred frames, and the phase multiplies that by 2 pi x 480.  The sum is a scan over
+// blocks of 256 frames (lanes, waves, blocks): fp64 holds these sums of fp32 values below 2
+// exactly unless a value is under 2^-20 of them, so its order does not show.  One thread a harmonic
+// that walks the frames took 690 us for 900 frames.
+__global__ __launch_bounds__(256) void source_phase_kernel(const HiftSource p,
+                                                           const HiftDocs* __restrict__ docs) {
 #pragma clang fp contract(off)
-  const int d = blockIdx.x;
-  const int h = threadIdx.x;
-  if (h >= p.H || d >= docs->n) return;
+  const int d = blockIdx.x, h = blockIdx.y;
+  if (d >= docs->n) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ double wsum[2][4];
   const int f_base = docs->a[d];
   const int T = docs->a[d + 1] - f_base;
   const long L = (long)T * p.scale;
@@ -417,20 +486,39 @@ __global__ __launch_bounds__(64) void source_phase_kernel(const HiftSource p,
     if (i == 0) v = v + p.rand_ini[h];
     return v;
   };
-  double c = 0.0;
-  for (int t = 0; t < T; ++t) {
-    float src = scale * ((float)t + 0.5f) - 0.5f;
-    if (src < 0.0f) src = 0.0f;
-    const long i0 = (long)src;
-    const float l1 = fminf(fmaxf(src - (float)i0, 0.0f), 1.0f);
-    const float l0 = 1.0f - l1;
-    const long i1 = i0 + (i0 < L - 1 ? 1 : 0);
-    const float a = l0 * rad_at(i0);
-    const float b = l1 * rad_at(i1);
-    c = c + (double)(a + b);
-    float ph = ((float)c * 2.0f) * 3.14159265358979323846f;
-    ph = ph * scale;
-    p.sines[(long)(f_base + t) * p.H + h] = sinf(ph) * p.sine_amp;
+  double before = 0.0;  // the sum of the earlier blocks
+  for (int t0 = 0, par = 0; t0 < T; t0 += 256, par ^= 1) {
+    const int t = t0 + tid;
+    double c = 0.0;
+    if (t < T) {
+      float src = scale * ((float)t + 0.5f) - 0.5f;
+      if (src < 0.0f) src = 0.0f;
+      const long i0 = (long)src;
+      const float l1 = fminf(fmaxf(src - (float)i0, 0.0f), 1.0f);
+      const float l0 = 1.0f - l1;
+      const long i1 = i0 + (i0 < L - 1 ? 1 : 0);
+      const float a = l0 * rad_at(i0);
+      const float b = l1 * rad_at(i1);
+      c = (double)(a + b);
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const double o = __shfl_up(c, off, 64);
+      if (lane >= off) c = o + c;
+    }
+    if (lane == 63) wsum[par][wave] = c;
+    __syncthreads();  // (the next block writes the other half)
+    double base = before;
+    for (int w = 0; w < 4; ++w) {
+      if (w == wave) c = base + c;
+      base = base + wsum[par][w];
+    }
+    before = base;
+    if (t < T) {
+      float ph = ((float)c * 2.0f) * 3.14159265358979323846f;
+      ph = ph * scale;
+      p.sines[(long)(f_base + t) * p.H + h] = sinf(ph) * p.sine_amp;
+    }
   }
 }
 
@@ -553,13 +641,12 @@ unsigned blocks_for(long n, int threads) { return (unsigned)((n + threads - 1) /
 
 bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
-template <typename T>
 hipError_t launch_conv(const HiftConv& p_in, hipStream_t stream) {
   if (p_in.rows_out <= 0) return hipSuccess;
   if (p_in.cin_pad % 16 != 0) return hipErrorInvalidValue;
   HiftConv p = p_in;
   // 16-byte epilogue accesses when every row pitch and base the epilogue touches allows them
-  p.vec4 = sizeof(T) == 4 && p.ldo % 4 == 0 && aligned16(p.out) && aligned16(p.bias) &&
+  p.vec4 = p.ldo % 4 == 0 && aligned16(p.out) && aligned16(p.bias) &&
            (!p.add || (p.ld_add % 4 == 0 && aligned16(p.add))) &&
            (p.mode == HIFT_ACC_WRITE || aligned16(p.accin)) &&
            (!p.snake_out || (aligned16(p.alpha) && aligned16(p.inv_alpha))) &&
@@ -576,26 +663,23 @@ hipError_t launch_conv(const HiftConv& p_in, hipStream_t stream) {
   if (force == 32 || (force != 64 && tiles64 < kSmallTileBelow)) {
     const dim3 grid((p.rows_out + 31) / 32, (p.cout + 31) / 32);
     if (p.cin_pad % 32 == 0)
-      hipLaunchKernelGGL((hift_conv_kernel<T, 32, 32>), grid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((hift_conv_kernel<32, 32>), grid, dim3(256), 0, stream, p);
     else
-      hipLaunchKernelGGL((hift_conv_kernel<T, 16, 32>), grid, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((hift_conv_kernel<16, 32>), grid, dim3(256), 0, stream, p);
     return hipGetLastError();
   }
   const dim3 grid((p.rows_out + kTileR - 1) / kTileR, (p.cout + kTileC - 1) / kTileC);
   if (p.cin_pad % 32 == 0)
-    hipLaunchKernelGGL((hift_conv_kernel<T, 32, 64>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((hift_conv_kernel<32, 64>), grid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((hift_conv_kernel<T, 16, 64>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((hift_conv_kernel<16, 64>), grid, dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t hift_conv_f32(const HiftConv& p, hipStream_t stream) {
-  return launch_conv<float>(p, stream);
-}
-hipError_t hift_conv_f64(const HiftConv& p, hipStream_t stream) {
-  return launch_conv<double>(p, stream);
+  return launch_conv(p, stream);
 }
 
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
@@ -617,13 +701,28 @@ hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* 
   return hipGetLastError();
 }
 
-hipError_t hift_to_f64(const float* x, double* y, int rows, int C, const HiftDocs* docs,
-                       hipStream_t stream) {
-  const long n = (long)rows * C;
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(to_f64_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, x, y, C,
-                     docs);
+namespace {
+template <typename X>
+hipError_t launch_f0(const HiftConv& p, hipStream_t stream) {
+  // 16x16 tiles up to two 32x32 tiles a CU
+  const long tiles32 = (long)((p.rows_out + 31) / 32) * ((p.cout + 31) / 32);
+  const int ts = tiles32 > 512 ? 32 : 16;
+  const dim3 grid((p.rows_out + ts - 1) / ts, (p.cout + ts - 1) / ts);
+  if (ts == 32)
+    hipLaunchKernelGGL((f0_conv_kernel<X, 2>), grid, dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((f0_conv_kernel<X, 1>), grid, dim3(256), 0, stream, p);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t hift_f0_conv(const HiftConv& p, int x_f32, hipStream_t stream) {
+  if (p.rows_out <= 0) return hipSuccess;
+  // K in four equal runs of 16-value groups, each inside one tap
+  if (!p.docs || p.cin_pad % 16 != 0 || (p.k * p.cin_pad) % 64 != 0 || p.ldx % 4 != 0 ||
+      p.stride != 1 || p.dil != 1 || p.up != 1 || !aligned16(p.w))
+    return hipErrorInvalidValue;
+  return x_f32 ? launch_f0<float>(p, stream) : launch_f0<double>(p, stream);
 }
 
 hipError_t hift_f0_head(const double* h, int C, const double* cls_w, const double* cls_b,
@@ -636,7 +735,7 @@ hipError_t hift_f0_head(const double* h, int C, const double* cls_w, const doubl
 
 hipError_t hift_source(const HiftSource& p, const HiftDocs* docs, hipStream_t stream) {
   if (p.docs_cap <= 0) return hipSuccess;
-  hipLaunchKernelGGL(source_phase_kernel, dim3(p.docs_cap), dim3(64), 0, stream, p, docs);
+  hipLaunchKernelGGL(source_phase_kernel, dim3(p.docs_cap, p.H), dim3(256), 0, stream, p, docs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (p.samples_cap <= 0) return hipSuccess;

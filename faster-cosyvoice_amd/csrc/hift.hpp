@@ -41,7 +41,6 @@ struct HiftConv {
   int rows_out;                            // capacity the grid covers (live: docs->b[docs->n])
   int reflect;                             // write row p + 1 (row 0 = row 2 of the result)
   int pro; float slope;                    // prologue on the inputs (fp32 only)
-  int elu;                                 // epilogue ELU (fp64 only)
   const void* add; int ld_add;             // y += add[row] (layout of out)
   int mode; const void* accin; float div;  // y = accin + y  or  (accin + y) / div
   const float* alpha; const float* inv_alpha;    // snake_out: out = snake(y)
@@ -70,7 +69,8 @@ struct HiftJobs {
 };
 
 hipError_t hift_conv_f32(const HiftConv& p, hipStream_t stream);
-hipError_t hift_conv_f64(const HiftConv& p, hipStream_t stream);
+// one layer of the fp64 F0 predictor: unit stride, weights and output fp64, ELU; x fp32 or fp64
+hipError_t hift_f0_conv(const HiftConv& p, int x_f32, hipStream_t stream);
 
 // The fp32 convolution with both operands split into two f16 halves (hift_split.hip), for the
 // shapes hift_split_eligible takes (its rule reads the shape only, not the row count): unit
@@ -96,10 +96,6 @@ hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, in
 struct HiftMean { const float* x[4]; int n; };
 hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* amax,
                      const HiftDocs* docs, hipStream_t stream);
-
-// fp32 -> fp64 of the live rows docs->a[docs->n] (grid: `rows`) x C values
-hipError_t hift_to_f64(const float* x, double* y, int rows, int C, const HiftDocs* docs,
-                       hipStream_t stream);
 
 // f0[r] = (float)|cls_w . h[r] + cls_b| (fp64 dot over C channels), one wave per live row
 // docs->b[docs->n] (grid: `rows`)

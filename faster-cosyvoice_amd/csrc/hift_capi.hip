@@ -149,7 +149,7 @@ struct Capacity {
   int frames, docs;
   int spec, samples, src;              // STFT frames, output samples, source samples
   std::vector<int> stage, stage_w;     // upsampling-conv rows and written rows per stage
-  size_t mel64, h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, y, fr, amax, tables, total;
+  size_t h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, y, fr, amax, tables, total;
   size_t si[2];                        // source branches of this stage and the next
   bool together;                       // a stage's resblocks run together (see run)
   size_t r[fcv::kHiftJobs], t1[fcv::kHiftJobs], s1[fcv::kHiftJobs];  // one set per resblock in flight
@@ -179,7 +179,6 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
   const int H = d.nb_harmonics + 1;
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += align_up(bytes); return o; };
-  C.mel64 = take(sizeof(double) * frames * d.in_channels);
   C.h64a = take(sizeof(double) * frames * d.f0_channels);
   C.h64b = take(sizeof(double) * frames * d.f0_channels);
   C.f0buf = take(sizeof(float) * frames);
@@ -436,14 +435,13 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   const int S = d.n_stages;
 
   // ---- F0 predictor (fp64) -------------------------------------------------------------
-  FCV_HIP(fcv::hift_to_f64(mel, F64(C.mel64), C.frames, d.in_channels, T + 0, st));
   const int fc = d.f0_channels;
-  HiftConv c0 = conv_base(F64(C.mel64), d.in_channels, fc, d.in_channels, 4, F64(C.h64a), fc,
+  HiftConv c0 = conv_base(mel, d.in_channels, fc, d.in_channels, 4, F64(C.h64a), fc,
                           C.frames, T + 0);
   c0.w = w[h->i_f0];
   c0.bias = w[h->i_f0 + 1];
-  c0.elu = 1;  // right-side lookahead: no left padding, zero (or context) on the right
-  FCV_HIP(fcv::hift_conv_f64(c0, st));
+  // right-side lookahead: no left padding, zero (or context) on the right
+  FCV_HIP(fcv::hift_f0_conv(c0, 1, st));
   double* hin = F64(C.h64a);
   double* hout = F64(C.h64b);
   for (int l = 1; l < 5; ++l) {
@@ -451,8 +449,7 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
     c.w = w[h->i_f0 + 2 * l];
     c.bias = w[h->i_f0 + 2 * l + 1];
     c.pad = causal_padding(3, 1);
-    c.elu = 1;
-    FCV_HIP(fcv::hift_conv_f64(c, st));
+    FCV_HIP(fcv::hift_f0_conv(c, 0, st));
     std::swap(hin, hout);
   }
   FCV_HIP(fcv::hift_f0_head(hin, fc, static_cast<const double*>(w[h->i_cls]),
