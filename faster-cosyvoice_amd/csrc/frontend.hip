@@ -8,12 +8,12 @@
 //   conv2: Y^T[o][t]  = W2[o][k] . G[k][t],  k = tap * C + c,  G[tap*C+c][t] = h(t - 2 + tap)[c]
 // with the weights as the A operand (rows = output channels) and the gathered token rows as
 // the B operand, so a lane's four accumulators are four consecutive channels of one token and
-// leave as one 16-byte store.  Both operands are staged through LDS K-contiguous, 16 K values
-// per chunk; lane (i, g) of the 16x16x4 MFMA feeds k = 4g + s at step s, so one 16-byte LDS
-// read covers four steps.  conv2 (80 outputs, K = 3072) splits K eight ways into partial sums
-// that a finishing kernel adds in a fixed order together with the bias, the residual and the
-// repeat to Mel rows.  No tile or split depends on the batch, so a document's result does not
-// depend on what it is packed with.  The per-document prefix sums travel by value in the kernel
+// leave as one 16-byte store.  Both operands are read from global memory, 16 K values per chunk;
+// lane (i, g) of the 16x16x4 MFMA feeds k = 4g + s at step s, so one 16-byte read covers four
+// steps.  A call has 10 to a few thousand tokens, so what bounds it is the chain of a wave's loads and
+// MFMAs: the waves of a workgroup split K (conv1 by taps, conv2 eight ways) and add their sums in
+// LDS in a fixed order.  No split depends on the batch, so a document's result does not depend on
+// what it is packed with.  The per-document prefix sums travel by value in the kernel
 // arguments (DocTables, at most kMaxDocs documents), so a call needs no host-to-device copy and
 // no synchronisation.
 #include <mutex>
@@ -28,10 +28,13 @@ namespace {
 
 constexpr int kFeat = 80;     // supported feat_dim
 constexpr int kBK = 16;       // K values per LDS chunk
-constexpr int kPitch = 20;    // LDS row pitch in floats (16 + 4: conflict-free 16-byte reads)
 constexpr int kSplit = 8;     // conv2 K split (fixed)
-constexpr int kTileT = 64;    // token rows per workgroup (both convolutions)
-constexpr int kTileC = 128;   // conv1 output channels per workgroup
+constexpr int kPitch = 20;    // LDS row pitch in floats (16 + 4: conflict-free 16-byte reads)
+constexpr int kTileT = 64;    // token rows per workgroup of the longer calls' convolutions
+constexpr int kTileC = 128;   // conv1 output channels per workgroup there
+// Output tokens from which the longer calls' forms run, whose tiles read the operands fewer times: at
+// 2298 tokens 35 + 27.5 + 4.7 us in three kernels against 37 + 43 in the short calls' two.
+constexpr int kWideFrom = 512;
 constexpr size_t kAlign = 256;
 constexpr int kMaxDocs = FCV_FLOW_MAX_DOCS;
 
@@ -59,9 +62,99 @@ __device__ __forceinline__ int find_doc(const int32_t* cu, int n_docs, int row) 
 __device__ __forceinline__ float leaky_relu(float x) { return x > 0.0f ? x : 0.01f * x; }
 
 // ---- conv1: h[t][c] = leaky_relu(b1[c] + sum_k W1[c][k] E[k][t]) ---------------------------
-// Workgroup tile 128 channels x 64 tokens; wave (wc, wt) owns 64 channels x 32 tokens.
+// Workgroup tile 32 channels x 32 tokens; wave w sums taps w, w + 4, .. from global memory, a tap's
+// five chunks of 16 K values in flight together, and the four sums are added in LDS in wave order.  A
+// tile of 128 channels x 64 tokens with K in one chain through LDS ran 16 workgroups of 20 steps for
+// a streaming chunk: 90 tokens 20.7 -> 5.8 us.
 // tab.a = token prefix sums, tab.b = output-token prefix sums
 __global__ __launch_bounds__(256) void lookahead_conv1_kernel(
+    const int32_t* __restrict__ tokens, const DocTables tab, int n_docs, int n_out,
+    const float* __restrict__ embed, int vocab, const float* __restrict__ W1,
+    const float* __restrict__ b1, int C, int taps, float* __restrict__ h) {
+  constexpr int CPT = kFeat / kBK;  // chunks per tap
+  constexpr int N = 2, TS = 16 * N;
+  __shared__ __attribute__((aligned(16))) float part[4][TS][TS + 4];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int t0 = blockIdx.x * TS;
+  const int c0 = blockIdx.y * TS;
+  const long K = (long)taps * kFeat;
+
+  // lane (li, lg): K values 4 lg .. 4 lg + 3 of a chunk, of channel / token li of each 16-tile
+  int tb[N], n_left[N];  // token index of tap 0 and tokens left in the document from there
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    const int t = t0 + 16 * b + li;
+    tb[b] = n_left[b] = 0;
+    if (t < n_out) {
+      const int d = find_doc(tab.b, n_docs, t);
+      tb[b] = tab.a[d] + (t - tab.b[d]);
+      n_left[b] = tab.a[d + 1] - tb[b];
+    }
+  }
+  f32x4 acc[N][N];
+#pragma unroll
+  for (int a = 0; a < N; ++a)
+#pragma unroll
+    for (int b = 0; b < N; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int tap = wave; tap < taps; tap += 4) {
+    const float* w = W1 + (c0 + li) * K + tap * kFeat + 4 * lg;
+    const float* e[N];
+    bool live[N];
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      live[b] = tap < n_left[b];
+      const int id = live[b] ? min(max(tokens[tb[b] + tap], 0), vocab - 1) : 0;
+      e[b] = embed + (long)id * kFeat + 4 * lg;
+    }
+    f32x4 av[CPT][N], bv[CPT][N];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+#pragma unroll
+      for (int a = 0; a < N; ++a)
+        av[c][a] = *reinterpret_cast<const f32x4*>(w + 16 * a * K + c * kBK);
+#pragma unroll
+      for (int b = 0; b < N; ++b) {
+        bv[c][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (live[b]) bv[c][b] = *reinterpret_cast<const f32x4*>(e[b] + c * kBK);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int a = 0; a < N; ++a)
+#pragma unroll
+          for (int b = 0; b < N; ++b) acc[a][b] = mfma16(av[c][a][s], bv[c][b][s], acc[a][b]);
+  }
+  // D[i = channel][j = token]: lane holds token li, channels 4 lg + 0..3 of each tile
+#pragma unroll
+  for (int a = 0; a < N; ++a)
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+      *reinterpret_cast<f32x4*>(&part[wave][16 * b + li][16 * a + 4 * lg]) = acc[a][b];
+  __syncthreads();
+  constexpr int TPT = TS / 4;  // threads a token
+  const int cl = tid % TPT * 4;
+  const f32x4 bias = *reinterpret_cast<const f32x4*>(b1 + c0 + cl);
+  for (int tl = tid / TPT; tl < TS && t0 + tl < n_out; tl += 256 / TPT) {
+    f32x4 v = *reinterpret_cast<const f32x4*>(&part[0][tl][cl]);
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v += *reinterpret_cast<const f32x4*>(&part[q][tl][cl]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = leaky_relu(v[i] + bias[i]);
+    *reinterpret_cast<f32x4*>(h + (long)(t0 + tl) * C + c0 + cl) = v;
+  }
+}
+
+// ---- conv1 of longer calls (from kWideFrom tokens, at most four taps): the same sums ----------
+// Workgroup tile 128 channels x 64 tokens; wave (wc, wt) owns 64 channels x 32 tokens.
+// tab.a = token prefix sums, tab.b = output-token prefix sums
+__global__ __launch_bounds__(256) void lookahead_conv1_wide_kernel(
     const int32_t* __restrict__ tokens, const DocTables tab, int n_docs, int n_out,
     const float* __restrict__ embed, int vocab, const float* __restrict__ W1,
     const float* __restrict__ b1, int C, int taps, float* __restrict__ h) {
@@ -109,11 +202,12 @@ __global__ __launch_bounds__(256) void lookahead_conv1_kernel(
     *reinterpret_cast<f32x4*>(&sB[buf][lr][4 * lq]) = rb;
   };
 
-  f32x4 acc[4][2];
+  // the tap's sum, and the sum of the taps before it (a tap is a wave's sum in the short form)
+  f32x4 acc[4][2], total[4][2];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < 2; ++b) acc[a][b] = total[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   fetch(0);
   stash(0);
@@ -138,6 +232,15 @@ __global__ __launch_bounds__(256) void lookahead_conv1_kernel(
       for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = mfma16(av[a][s], bv[b][s], acc[a][b]);
+    if ((kc + 1) % CPT == 0) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          total[a][b] += acc[a][b];
+          acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
     stash(cur ^ 1);
     __syncthreads();
   }
@@ -153,17 +256,91 @@ __global__ __launch_bounds__(256) void lookahead_conv1_kernel(
       const f32x4 bias = *reinterpret_cast<const f32x4*>(b1 + c);
       f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = leaky_relu(acc[a][b][e] + bias[e]);
+      for (int e = 0; e < 4; ++e) v[e] = leaky_relu(total[a][b][e] + bias[e]);
       *reinterpret_cast<f32x4*>(h + (long)t * C + c) = v;
     }
   }
+}
+
+// ---- conv2: mu rows ratio*t .. +ratio-1 = b2 + sum_k W2[o][k] G[k][t] + e(t) ------------------
+// The short calls' form (below kWideFrom tokens; the same sums as the two kernels below).  Workgroup
+// tile 16 outputs x 16 tokens; its kSplit waves take an equal run of K each, straight from global
+// memory kDepth chunks ahead, and the sums are added in LDS in order, with the bias, the residual and
+// the repeat.  90 tokens: 18.3 + 3.9 us in two kernels, 15.4 in this one; 2298 tokens 27.5 + 4.7
+// against 43 (the weights are read once per 16 tokens).
+// tab.a = token prefix sums, tab.b = output-token prefix sums
+__global__ __launch_bounds__(64 * kSplit) void lookahead_conv2_kernel(
+    const float* __restrict__ h, const int32_t* __restrict__ tokens, const DocTables tab, int n_docs,
+    int n_out, const float* __restrict__ W2, int C, const float* __restrict__ embed, int vocab,
+    const float* __restrict__ b2, int ratio, float* __restrict__ mu) {
+  constexpr int TAPS = 3, kDepth = 6;
+  __shared__ __attribute__((aligned(16))) float part[kSplit][16][20];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int split = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int t0 = blockIdx.x * 16;
+  const int o0 = blockIdx.y * 16;
+  const int CPT = C / kBK;
+  const int run = TAPS * CPT / kSplit;
+  const int kc_begin = split * run, kc_end = kc_begin + run;
+
+  int pos = -(1 << 29);  // position of the lane's token in its document (far below 0: past the batch)
+  if (t0 + li < n_out) pos = t0 + li - tab.b[find_doc(tab.b, n_docs, t0 + li)];
+  const float* W = W2 + (long)(o0 + li) * TAPS * C + 4 * lg;
+  f32x4 av[kDepth], bv[kDepth];
+  auto fetch = [&](int slot, int kc) {
+    const int tap = kc / CPT;
+    const int cc = (kc - tap * CPT) * kBK;
+    av[slot] = *reinterpret_cast<const f32x4*>(W + kc * kBK);
+    bv[slot] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // h row t - 2 + tap, which lies in the same document iff pos - 2 + tap >= 0
+    if (pos + tap >= TAPS - 1)
+      bv[slot] = *reinterpret_cast<const f32x4*>(
+          h + (long)(t0 + li - (TAPS - 1) + tap) * C + cc + 4 * lg);
+  };
+  f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int u = 0; u < kDepth - 1; ++u) fetch(u, min(kc_begin + u, kc_end - 1));
+  for (int k0 = kc_begin; k0 < kc_end; k0 += kDepth) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      if (k0 + u >= kc_end) break;
+      fetch((u + kDepth - 1) % kDepth, min(k0 + u + kDepth - 1, kc_end - 1));
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = mfma16(av[u][s], bv[u][s], acc);
+    }
+  }
+  *reinterpret_cast<f32x4*>(&part[split][li][4 * lg]) = acc;
+  __syncthreads();
+  if (tid >= 64) return;
+  const int tl = tid >> 2, ol = (tid & 3) * 4;  // four threads a token
+  const int t = t0 + tl;
+  if (t >= n_out) return;
+  const int d = find_doc(tab.b, n_docs, t);
+  const int id = min(max(tokens[tab.a[d] + (t - tab.b[d])], 0), vocab - 1);
+  const f32x4 bias = *reinterpret_cast<const f32x4*>(b2 + o0 + ol);
+  const f32x4 res = *reinterpret_cast<const f32x4*>(embed + (long)id * kFeat + o0 + ol);
+  f32x4 s = *reinterpret_cast<const f32x4*>(&part[0][tl][ol]);
+#pragma unroll
+  for (int k = 1; k < kSplit; ++k) {
+    const f32x4 q = *reinterpret_cast<const f32x4*>(&part[k][tl][ol]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] += q[e];
+  }
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = (s[e] + bias[e]) + res[e];
+  for (int j = 0; j < ratio; ++j)
+    *reinterpret_cast<f32x4*>(mu + ((long)t * ratio + j) * kFeat + o0 + ol) = y;
 }
 
 // ---- conv2 partial sums: part[s][t][o] = sum over split s of W2[o][k] G[k][t] --------------
 // Workgroup tile 80 outputs x 64 tokens, K range split blockIdx.y of kSplit; wave w owns
 // tokens 16 w .. 16 w + 15 and all five 16-output tiles.
 // tab.b = output-token prefix sums
-__global__ __launch_bounds__(256) void lookahead_conv2_kernel(
+__global__ __launch_bounds__(256) void lookahead_conv2_part_kernel(
     const float* __restrict__ h, const DocTables tab, int n_docs, int n_out,
     const float* __restrict__ W2, int C, float* __restrict__ part) {
   constexpr int TAPS = 3;
@@ -267,29 +444,35 @@ __global__ __launch_bounds__(256) void lookahead_finish_kernel(
     *reinterpret_cast<f32x4*>(mu + ((long)t * ratio + j) * kFeat + o) = y;
 }
 
-// ---- speaker: out[n] = W (x / max(||x||, 1e-12)) + b; one wave per x-vector ----------------
-__global__ __launch_bounds__(64) void speaker_kernel(const float* __restrict__ x, int D,
-                                                     const float* __restrict__ W,
-                                                     const float* __restrict__ b, int F,
-                                                     float* __restrict__ out) {
-  __shared__ float sx[256];
+// ---- speaker: out[n] = W (x / max(||x||, 1e-12)) + b -----------------------------------------
+// One workgroup per x-vector; each wave keeps the normalised vector in registers (lane l: elements
+// l, l + 64, ..) and takes every 16th output, so a weight row is one coalesced read.  (A lane a
+// row, in one wave, walked the rows element by element: 7.4 us for one vector, now 4.4.)
+__global__ __launch_bounds__(1024) void speaker_kernel(const float* __restrict__ x, int D,
+                                                       const float* __restrict__ W,
+                                                       const float* __restrict__ b, int F,
+                                                       float* __restrict__ out) {
+  constexpr int E = 4;  // D <= 256
   const int n = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float v[E];
   float ss = 0.0f;
-  for (int i = lane; i < D; i += 64) {
-    const float v = x[(long)n * D + i];
-    sx[i] = v;
-    ss = fmaf(v, v, ss);
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    v[i] = lane + 64 * i < D ? x[(long)n * D + lane + 64 * i] : 0.0f;
+    ss = fmaf(v[i], v[i], ss);
   }
   const float denom = fmaxf(sqrtf(wave_sum(ss)), 1e-12f);
-  __syncthreads();
-  for (int i = lane; i < D; i += 64) sx[i] = sx[i] / denom;
-  __syncthreads();
-  for (int o = lane; o < F; o += 64) {
+#pragma unroll
+  for (int i = 0; i < E; ++i) v[i] = v[i] / denom;
+  for (int o = wave; o < F; o += 16) {
     const float* w = W + (long)o * D;
     float acc = 0.0f;
-    for (int i = 0; i < D; ++i) acc = fmaf(w[i], sx[i], acc);
-    out[(long)n * F + o] = acc + b[o];
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+      if (lane + 64 * i < D) acc = fmaf(w[lane + 64 * i], v[i], acc);
+    acc = wave_sum(acc);
+    if (lane == 0) out[(long)n * F + o] = acc + b[o];
   }
 }
 
@@ -329,7 +512,7 @@ int check_dims(const FcvFlowDims* dims) {
   FCV_CHECK(dims, FCV_ERR_INVALID, "null dims");
   const FcvFlowDims& d = *dims;
   FCV_CHECK(d.feat_dim == kFeat, FCV_ERR_INVALID, "feat_dim must be 80");
-  FCV_CHECK(d.channels > 0 && d.channels % kTileC == 0, FCV_ERR_INVALID,
+  FCV_CHECK(d.channels > 0 && d.channels % 128 == 0, FCV_ERR_INVALID,
             "channels must be a positive multiple of 128");
   FCV_CHECK(d.lookahead >= 0 && d.lookahead <= 7, FCV_ERR_INVALID, "lookahead must be in [0, 7]");
   FCV_CHECK(d.token_mel_ratio >= 1 && d.token_mel_ratio <= 8, FCV_ERR_INVALID,
@@ -379,20 +562,33 @@ int prepare_token_features(const FcvFlowDims* dims, const FcvFlowWeights* weight
   return FCV_OK;
 }
 
-// The three kernels of a checked call, with the workspace at `ws` (flow_layout of n_out).
+// The kernels of a checked call, with the workspace at `ws` (flow_layout of n_out).
 int launch_token_features(const FcvFlowDims& d, const FcvFlowWeights& w, const int32_t* tokens,
                           const DocTables& tab, int n_docs, int n_out, float* mu_out, char* ws,
                           hipStream_t stream) {
   const FlowLayout L = flow_layout(d, n_out);
   float* hid = reinterpret_cast<float*>(ws + L.hidden);
-  float* part = reinterpret_cast<float*>(ws + L.part);
-  const int t_tiles = (n_out + kTileT - 1) / kTileT;
-  hipLaunchKernelGGL(lookahead_conv1_kernel, dim3(t_tiles, d.channels / kTileC), dim3(256), 0,
-                     stream, tokens, tab, n_docs, n_out, w.embed, d.vocab, w.la1_w, w.la1_b,
-                     d.channels, d.lookahead + 1, hid);
+  const bool wide = n_out >= kWideFrom;
+  if (wide && d.lookahead < 4)
+    hipLaunchKernelGGL(lookahead_conv1_wide_kernel,
+                       dim3((n_out + kTileT - 1) / kTileT, d.channels / kTileC), dim3(256), 0, stream,
+                       tokens, tab, n_docs, n_out, w.embed, d.vocab, w.la1_w, w.la1_b, d.channels,
+                       d.lookahead + 1, hid);
+  else
+    hipLaunchKernelGGL(lookahead_conv1_kernel, dim3((n_out + 31) / 32, d.channels / 32), dim3(256), 0,
+                       stream, tokens, tab, n_docs, n_out, w.embed, d.vocab, w.la1_w, w.la1_b,
+                       d.channels, d.lookahead + 1, hid);
   FCV_HIP(hipGetLastError());
-  hipLaunchKernelGGL(lookahead_conv2_kernel, dim3(t_tiles, kSplit), dim3(256), 0, stream, hid,
-                     tab, n_docs, n_out, w.la2_w, d.channels, part);
+  if (!wide) {
+    hipLaunchKernelGGL(lookahead_conv2_kernel, dim3((n_out + 15) / 16, kFeat / 16),
+                       dim3(64 * kSplit), 0, stream, hid, tokens, tab, n_docs, n_out, w.la2_w,
+                       d.channels, w.embed, d.vocab, w.la2_b, d.token_mel_ratio, mu_out);
+    FCV_HIP(hipGetLastError());
+    return FCV_OK;
+  }
+  float* part = reinterpret_cast<float*>(ws + L.part);
+  hipLaunchKernelGGL(lookahead_conv2_part_kernel, dim3((n_out + kTileT - 1) / kTileT, kSplit),
+                     dim3(256), 0, stream, hid, tab, n_docs, n_out, w.la2_w, d.channels, part);
   FCV_HIP(hipGetLastError());
   const long items = (long)n_out * (kFeat / 4);
   hipLaunchKernelGGL(lookahead_finish_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0,
@@ -518,7 +714,7 @@ int fcv_flow_speaker(const FcvFlowDims* dims, const FcvFlowWeights* weights, con
   FCV_CHECK(weights && weights->spk_w && weights->spk_b, FCV_ERR_INVALID, "null weight pointer");
   FCV_CHECK(xvec && spks_out, FCV_ERR_INVALID, "null argument");
   FCV_CHECK(n >= 1, FCV_ERR_INVALID, "need at least one x-vector");
-  hipLaunchKernelGGL(fcv::speaker_kernel, dim3(n), dim3(64), 0, stream, xvec, dims->spk_dim,
+  hipLaunchKernelGGL(fcv::speaker_kernel, dim3(n), dim3(1024), 0, stream, xvec, dims->spk_dim,
                      weights->spk_w, weights->spk_b, dims->feat_dim, spks_out);
   FCV_HIP(hipGetLastError());
   return FCV_OK;

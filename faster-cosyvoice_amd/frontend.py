@@ -213,9 +213,14 @@ class FlowFrontEnd(nn.Module):
             if p.shape[1] > max_mel:  # the reference's padded copy cannot hold it either
                 raise RuntimeError(f"prompt of {p.shape[1]} frames exceeds the longest "
                                    f"document ({max_mel} frames)")
-        prompt = (torch.cat([p[0] for p in prompt_features]) if sum(plens) else
-                  torch.zeros(1, self.output_size))
+        if len(plens) == 1 and plens[0]:
+            prompt = prompt_features[0][0]  # no copy to pack a single prompt
+        else:
+            prompt = (torch.cat([p[0] for p in prompt_features]) if sum(plens) else
+                      torch.zeros(1, self.output_size))
         prompt = prompt.to(device=self.device, dtype=torch.float32).contiguous()
+        if prompt.data_ptr() % 16:  # a caller's own tensor may start anywhere
+            prompt = prompt.clone()
         cu_p, cu_m = [0], [0]
         for p, m in zip(plens, mel_lengths):
             cu_p.append(cu_p[-1] + p)
