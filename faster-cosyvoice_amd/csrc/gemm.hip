@@ -55,7 +55,7 @@ struct TileCfg {
   static constexpr int B_INSTR = BN / ROWS_PER_COPY / kWaves;
   static constexpr int LOADS = A_INSTR + B_INSTR;
   static constexpr int kLds = STAGES * (BM + BN) * BK * 2;
-  static constexpr int kOcc = (160 * 1024) / kLds >= 2 ? 2 : 1;  // workgroups per CU
+  static constexpr int kOcc = (160 * 1024) / kLds >= 2 && kWaves >= 4 ? 2 : 1;  // waves per SIMD
   static constexpr int kGroupM = 1024 / BM > 0 ? 1024 / BM : 1;  // ~1024 A rows per L2 group
   static_assert(BK == 32 || BK == 64, "slice depth");
   static_assert(STAGES >= 2 && (STAGES - 2) * LOADS < 64, "ring depth");
@@ -143,7 +143,7 @@ struct direct_layout : std::false_type {};
 template <class E>
 struct direct_layout<E, std::void_t<decltype(&E::finish_direct)>> : std::true_type {};
 
-// workgroups per CU with the epilogue's row_info array in LDS as well
+// waves per SIMD with the epilogue's row_info array in LDS as well
 template <class C, class Epi>
 constexpr int occupancy() {
   return (160 * 1024) / (C::kLds + (Epi::kRowInfo ? C::BM * 4 : 0)) >= 2 ? C::kOcc : 1;
@@ -716,6 +716,8 @@ using Tile128x128x3 = TileCfg<128, 128, 2, 2, 64, 3>;  // one workgroup per CU
 using Tile32x128x4 = TileCfg<32, 128, 1, 4, 64, 4>;
 using Tile64x64x3 = TileCfg<64, 64, 2, 2, 64, 3>;    // three workgroups per CU
 using Tile64x64x5 = TileCfg<64, 64, 2, 2, 64, 5>;    // two workgroups per CU
+using Tile32x64x4 = TileCfg<32, 64, 1, 2, 64, 4>;    // three workgroups per CU
+using Tile32x64x6 = TileCfg<32, 64, 1, 2, 64, 6>;    // two workgroups per CU
 using Tile128x64x3 = TileCfg<128, 64, 2, 2, 64, 3>;  // two workgroups per CU
 using Tile128x64x4 = TileCfg<128, 64, 2, 2, 64, 4>;  // one workgroup per CU
 using Tile64x128x3 = TileCfg<64, 128, 2, 2, 64, 3>;  // two workgroups per CU
@@ -750,19 +752,24 @@ hipError_t launch_tile(const f16* A, int lda, const f16* W, int ldw, int M, int 
 // width measured in eager 22-block solves (weights streamed from HBM as in production) at the
 // capacities one request plans into (340-3090 rows) with every shape and ring depth forced;
 // its pick is within 3 % of the fastest at every measured size, and the four GEMMs of a block
-// take 12-20 % less time at 340-1170 rows than the estimate's pick.  The choice only changes
+// take 12-20 % less time at 340-1170 rows than the estimate's pick.  32x64 tiles of two waves (six
+// stages while two per CU hold every tile, four and three per CU above; eight were no better) give the 1024-column GEMMs
+// twice the workgroups where 64x64 tiles leave CUs idle, and QKV an even share where 64x64 tiles put
+// two on some CUs: whole solves of one request -5 % at 270-400 rows, -3 % at 460-530, -1 to -3 % at
+// 590-780 for the former (even at 910), -4 to -5 % at 366-398 rows for the latter (+1 to +7 % outside).  The choice only changes
 // which rows and columns share a workgroup: every output element still accumulates its K
 // slices in the same order, so results are bitwise identical for every tile shape (batch
 // invariance holds).
 constexpr int kCus = 256;
-constexpr int kTileShapes = 11;
+constexpr int kTileShapes = 12;
 constexpr int kTileShape[kTileShapes][2] = {{256, 256}, {192, 256}, {128, 256}, {256, 128},
                                             {128, 128}, {32, 128},  {160, 256}, {96, 128},
-                                            {64, 64},   {128, 64},  {64, 128}};
+                                            {64, 64},   {128, 64},  {64, 128},  {32, 64}};
 // 0: chosen from the small-launch table only
 constexpr float kTileRate[kTileShapes] = {1.0f, 0.97f, 0.80f, 0.78f, 0.85f, 0.45f, 0.75f, 0.66f,
-                                          0.0f, 0.0f,  0.0f};
-constexpr int kTile128x128 = 4, kTile96x128 = 7, kTile64x64 = 8, kTile128x64 = 9, kTile64x128 = 10;
+                                          0.0f, 0.0f,  0.0f,  0.0f};
+constexpr int kTile128x128 = 4, kTile96x128 = 7, kTile64x64 = 8, kTile128x64 = 9, kTile64x128 = 10,
+              kTile32x64 = 11;
 
 inline long tile_count(int M, int N, int bm, int bn) { return (long)((M + bm - 1) / bm) * (N / bn); }
 
@@ -771,12 +778,12 @@ struct SmallStep {
   int max_m, shape;
 };
 constexpr SmallStep kSmall1024[] = {  // output projection and FF2 (K 1024 and 2048)
-    {1024, kTile64x64}, {2100, kTile128x64}, {3072, kTile96x128}};
+    {800, kTile32x64}, {1024, kTile64x64}, {2100, kTile128x64}, {3072, kTile96x128}};
 constexpr SmallStep kSmall2048[] = {  // FF1
     {600, kTile64x64}, {1000, kTile128x64}, {1536, kTile96x128}, {2048, kTile128x128},
     {2200, kTile128x64}};
 constexpr SmallStep kSmall3072[] = {  // QKV
-    {400, kTile64x64}, {850, kTile128x64}, {1000, kTile64x128}, {1200, kTile128x64},
+    {350, kTile64x64}, {400, kTile32x64}, {850, kTile128x64}, {1000, kTile64x128}, {1200, kTile128x64},
     {1440, kTile64x128}, {2100, kTile96x128}};
 
 template <int L>
@@ -847,6 +854,11 @@ hipError_t launch(const f16* A, int lda, const f16* W, int ldw, int M, int N, in
       if (tile_count(M, N, 128, 64) <= 288)
         return launch_tile<Tile128x64x4>(A, lda, W, ldw, M, N, K, epi, stream, m_live);
       return launch_tile<Tile128x64x3>(A, lda, W, ldw, M, N, K, epi, stream, m_live);
+    case kTile32x64:
+      // six stages while two per CU hold every tile, four (three per CU) above
+      if (tile_count(M, N, 32, 64) <= 2 * kCus)
+        return launch_tile<Tile32x64x6>(A, lda, W, ldw, M, N, K, epi, stream, m_live);
+      return launch_tile<Tile32x64x4>(A, lda, W, ldw, M, N, K, epi, stream, m_live);
     case kTile64x128:
       return launch_tile<Tile64x128x3>(A, lda, W, ldw, M, N, K, epi, stream, m_live);
     case 7:

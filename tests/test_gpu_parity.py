@@ -476,6 +476,22 @@ def test_every_gemm_tile_shape_gives_the_same_bits(fcv, stress2, monkeypatch):
     monkeypatch.delenv("FCV_GEMM_TILE", raising=False)
 
 
+@pytest.mark.parametrize("lengths", [[1], [31, 33], [90, 90], [175, 184], [200, 65, 120]], ids=str)
+def test_32x64_gemm_tile_gives_the_same_bits(fcv, stress2, monkeypatch, lengths):
+    """The 32x64 tile (shape 11: four or six ring stages by its tile count) against the table's
+    pick, at row counts on both sides of its tile edges and of the table's steps."""
+    _, est = stress2
+    x, mu, cond, spks, tt = random_packed(lengths, seed=68, t=0.4)
+    run = lambda: est.forward_packed(x, mu, cond, spks, tt[:1], lengths, streaming=True).clone()
+    monkeypatch.delenv("FCV_GEMM_TILE", raising=False)
+    say(f"[32x64] {lengths}")
+    ref = run()
+    for shape in ("11", "8"):
+        monkeypatch.setenv("FCV_GEMM_TILE", shape)
+        assert torch.equal(run(), ref), shape
+
+
+
 def test_streaming_prefix_stability_gate_a(fcv, stress2):
     """Reference Gate A (tests/gpu/test_flashinfer_streaming_estimator.py:58-89): with the
     chunk-causal mask the first floor(160/50)*50 frames of T=160 and T=200 agree; with full
