@@ -1,31 +1,58 @@
 // Causal grouped conv1d + Mish (CausalConvPositionEmbedding) as an implicit GEMM on MFMA.
 //
-// Per (row tile of 128 frames, group g of 64 channels):
+// Per (row tile, group g of 64 channels):
 //   y[r, co] = mish(bias[co] + sum_{j<taps} sum_{ci<64} W[g][j][co][ci] * x[r - (taps-1) + j, ci])
-// The 128 + taps - 1 input rows of the group's 64 channels are staged in LDS once; every tap
-// j reads the same window shifted by j rows, so no im2col buffer exists.  Each tap's 64x64
-// weight slice streams through an LDS double buffer.  Packed documents are handled per row:
-// the input fragment of output row r at tap j is zeroed when the input row lies before r's
-// document start, i.e. when pos[r] + j < taps - 1 (the per-document left zero padding of
-// the reference's F.pad).
+// The tile's input rows and the taps - 1 before them are staged in LDS once for the group's 64
+// channels; every tap j reads the same window shifted by j rows, so no im2col buffer exists.  Packed
+// documents are handled per row: the input fragment of output row r at tap j is zeroed when the
+// input row lies before r's document start, i.e. when pos[r] + j < taps - 1 (the per-document left
+// zero padding of the reference's F.pad).
+//
+// An output's sum is taken over kTapGroups groups of consecutive taps, each from zero, the groups
+// added in order, whatever the tile: small launches give each group a wave.  A launch of few rows is
+// bound by one workgroup's chain of taps, each a barrier and an LDS round trip, on a part of the CUs
+// (48 of 256 at 300 rows); a large one by the LDS reads of its MFMAs.  Three forms; a forward of one
+// block holds two launches, and took on one MI355X (us, at 16 channel groups), in turn:
+//   rows                        60    300   500   520   700   1000  1040  1500  4500
+//   32 rows, a group a wave     90    97    104   122+  .     .     157+  168   340
+//   64 rows, a group a wave     94    100   112+  112   122   125   146+  158   293
+//   128 rows, all taps a wave   102   109   .     120+  .     .     140   152   248
+//   (+ at 550 and 1100 rows.)  128 rows in one chain of taps, the channel groups on the grid's slow
+//   axis, was the only form before: 103, 112, 118, 120, 129, 135, 140, 152, 248.
 #include "kernels.hpp"
 
 namespace fcv {
 namespace {
 
-constexpr int TM = 128;       // output rows per workgroup
 constexpr int CG = 64;        // channels per group
+constexpr int kTapGroups = 4;
 constexpr int LDP = CG + 8;   // padded LDS row (f16): 16 consecutive rows hit distinct banks
 constexpr int MAX_TAPS = 31;
-constexpr int WIN = TM + MAX_TAPS - 1;
 constexpr int SPITCH = CG + 4;  // fp32 staging row
-constexpr int X_BYTES = WIN * LDP * 2;
 constexpr int W_BYTES = 2 * CG * LDP * 2;
 constexpr int STAGE_BYTES = 4 * 32 * SPITCH * 4;
-constexpr int SMEM_BYTES = X_BYTES + W_BYTES > STAGE_BYTES ? X_BYTES + W_BYTES : STAGE_BYTES;
 
-// 4 waves x 32 output rows x 64 output channels; MFMA 32x32x16 with the weights as the A
-// operand, so lane l accumulates output row l % 32 and, in register group g of channel tile t,
+constexpr int kCUs = 256;
+
+// taps of a group: even, so that a group's first tap is on the weights' first buffer
+__device__ __forceinline__ constexpr int tap_group(int taps) {
+  return (taps + 2 * kTapGroups - 1) / (2 * kTapGroups) * 2;
+}
+
+// one output element group of the epilogue: mish(v + bias) to f16, or added to the residual's row
+__device__ __forceinline__ void conv_finish(const f32x4& v, const float4& b, const float4& hv,
+                                            long at, f16* out_f16, float* h) {
+  const float4 y = {mish(v[0] + b.x), mish(v[1] + b.y), mish(v[2] + b.z), mish(v[3] + b.w)};
+  if (h)
+    *reinterpret_cast<float4*>(h + at) = float4{hv.x + y.x, hv.y + y.y, hv.z + y.z, hv.w + y.w};
+  else
+    *reinterpret_cast<f16x4*>(out_f16 + at) = f2h4(y.x, y.y, y.z, y.w);
+}
+
+// 4 waves x 32 output rows x 64 output channels.  Each tap's 64x64 weight slice streams through an
+// LDS double buffer.  (64 rows a wave, for 1 KB of LDS read per MFMA and not 1.5, measured no faster
+// from 1100 rows up: two workgroups of 128 rows on a CU hide each other's taps, one of 256 has
+// nothing beside it.)  MFMA 32x32x16 with the weights as the A operand, so lane l accumulates output row l % 32 and, in register group g of channel tile t,
 // channels 32 t + 8 g + 4 (l / 32) + 0..3.  The epilogue stages each wave's 32 x 64 block
 // through LDS and reads it back row-major (16 lanes per row), so stores are contiguous runs of
 // 128 B (f16 out) or 256 B (fp32 residual); the residual form issues all its h loads before
@@ -37,14 +64,17 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const f16* __restrict__ x,
                                                       f16* __restrict__ out_f16,
                                                       float* __restrict__ h,
                                                       const int32_t* __restrict__ rows_live) {
+  constexpr int TM = 128;
+  constexpr int X_BYTES = (TM + MAX_TAPS - 1) * LDP * 2;
+  constexpr int SMEM_BYTES = X_BYTES + W_BYTES > STAGE_BYTES ? X_BYTES + W_BYTES : STAGE_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM_BYTES];
   f16 (*sX)[LDP] = reinterpret_cast<f16 (*)[LDP]>(smem);
   f16 (*sW)[CG][LDP] = reinterpret_cast<f16 (*)[CG][LDP]>(smem + X_BYTES);
 
   if (rows_live) rows = *rows_live;  // live rows of a capacity-sized grid
-  const int m0 = blockIdx.x * TM;
+  const int m0 = blockIdx.y * TM;
   if (m0 >= rows) return;
-  const int g = blockIdx.y;
+  const int g = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -78,12 +108,12 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const f16* __restrict__ x,
   const int col_lane = (lane & 15) * 4;  // epilogue: 4 channels of one row per lane
   const float4 bias4 = *reinterpret_cast<const float4*>(bias + g * CG + col_lane);
 
-  f32x16 acc[2];
+  // the tap group's sum, and the sum of the groups before it
+  f32x16 acc[2], total[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[t][e] = 0.0f;
-
+    for (int e = 0; e < 16; ++e) acc[t][e] = total[t][e] = 0.0f;
   const f16x8 zero8 = {};
   auto tap = [&](int j, int buf) {
     // rows before the row's document start read as zero (per-document causal padding)
@@ -108,54 +138,168 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const f16* __restrict__ x,
   stash(ra, 0);
   fetch(ra, min(1, taps - 1));
   __syncthreads();
-  for (int j = 0; j < taps; j += 2) {
-    fetch(rb, min(j + 2, taps - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    tap(j, 0);
-    stash(ra, 1);
-    __syncthreads();
-    if (j + 1 < taps) {
-      fetch(ra, min(j + 3, taps - 1));
+  for (int j0 = 0; j0 < taps; j0 += tap_group(taps)) {
+    const int j1 = min(j0 + tap_group(taps), taps);
+    for (int j = j0; j < j1; j += 2) {
+      fetch(rb, min(j + 2, taps - 1));
       __builtin_amdgcn_sched_barrier(0);
-      tap(j + 1, 1);
-      stash(rb, 0);
+      tap(j, 0);
+      stash(ra, 1);
       __syncthreads();
+      if (j + 1 < j1) {
+        fetch(ra, min(j + 3, taps - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        tap(j + 1, 1);
+        stash(rb, 0);
+        __syncthreads();
+      }
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        total[t][e] = total[t][e] + acc[t][e];
+        acc[t][e] = 0.0f;
+      }
   }
 
   // epilogue (the loop's last barrier freed the window and weight buffers)
   float* stage = reinterpret_cast<float*>(smem) + wave * 32 * SPITCH;
+  const int col = g * CG + col_lane;
+  const int row0 = m0 + wave * 32;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<f32x4*>(stage + fr * SPITCH + t * 32 + q * 8 + fh * 4) =
-          f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+      *reinterpret_cast<f32x4*>(stage + fr * SPITCH + t * 32 + q * 8 + fh * 4) = f32x4{
+          total[t][4 * q], total[t][4 * q + 1], total[t][4 * q + 2], total[t][4 * q + 3]};
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int col = g * CG + col_lane;
   f32x4 v[8];
   float4 hv[8];
 #pragma unroll
   for (int p = 0; p < 8; ++p) {
     const int r = p * 4 + (lane >> 4);
     v[p] = *reinterpret_cast<const f32x4*>(stage + r * SPITCH + col_lane);
-    const int row = min(m0 + wave * 32 + r, rows - 1);
+    const int row = min(row0 + r, rows - 1);
     if (h) hv[p] = *reinterpret_cast<const float4*>(h + (long)row * C + col);
   }
 #pragma unroll
   for (int p = 0; p < 8; ++p) {
-    const int row = m0 + wave * 32 + p * 4 + (lane >> 4);
-    const float4 y = {mish(v[p][0] + bias4.x), mish(v[p][1] + bias4.y), mish(v[p][2] + bias4.z),
-                      mish(v[p][3] + bias4.w)};
-    if (h) {
-      const float4 r4 = {hv[p].x + y.x, hv[p].y + y.y, hv[p].z + y.z, hv[p].w + y.w};
-      if (row < rows) *reinterpret_cast<float4*>(h + (long)row * C + col) = r4;
-    } else {
-      const f16x4 yb = f2h4(y.x, y.y, y.z, y.w);
-      if (row < rows) *reinterpret_cast<f16x4*>(out_f16 + (long)row * C + col) = yb;
+    const int row = row0 + p * 4 + (lane >> 4);
+    if (row < rows) conv_finish(v[p], bias4, hv[p], (long)row * C + col, out_f16, h);
+  }
+}
+
+// The small launches' form: a workgroup owns 32 MR rows x 64 channels and each of its waves one group
+// of taps, with the weights straight from global memory two taps ahead, so no wave waits for another
+// between the window and the sums' addition in LDS.
+template <int MR>
+__global__ __launch_bounds__(64 * kTapGroups, 2) void conv_small_kernel(
+    const f16* __restrict__ x, int C, const f16* __restrict__ w, const float* __restrict__ bias,
+    int taps, const int32_t* __restrict__ pos, int rows, f16* __restrict__ out_f16,
+    float* __restrict__ h, const int32_t* __restrict__ rows_live) {
+  constexpr int TM = 32 * MR;
+  constexpr int X_BYTES = (TM + MAX_TAPS - 1) * LDP * 2;
+  constexpr int PART_BYTES = kTapGroups * TM * SPITCH * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[X_BYTES > PART_BYTES ? X_BYTES
+                                                                                  : PART_BYTES];
+  f16 (*sX)[LDP] = reinterpret_cast<f16 (*)[LDP]>(smem);
+  float (*part)[TM][SPITCH] = reinterpret_cast<float (*)[TM][SPITCH]>(smem);
+
+  if (rows_live) rows = *rows_live;  // live rows of a capacity-sized grid
+  const int m0 = blockIdx.y * TM;
+  if (m0 >= rows) return;
+  const int g = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int fr = lane & 31, fh = lane >> 5;
+  const int halo = taps - 1;
+  const int group = tap_group(taps);
+  const int j0 = wave * group, j1 = min(j0 + group, taps);
+
+  // this wave's first taps' weights: fragment (t, ks) of lane l is channel 32 t + l % 32, inputs
+  // 16 ks + 8 (l / 32) + 0..7
+  constexpr int PD = 3;
+  f16x8 wr[PD][8];
+  const f16* wg = w + ((long)g * taps * CG + fr) * CG + fh * 8;
+  auto fetch = [&](f16x8 (&f)[8], int j) {
+    const f16* src = wg + (long)min(j, taps - 1) * CG * CG;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        f[4 * t + ks] = *reinterpret_cast<const f16x8*>(src + t * 32 * CG + ks * 16);
+  };
+#pragma unroll
+  for (int u = 0; u < PD - 1; ++u) fetch(wr[u], j0 + u);
+
+  const int chunk_c = (tid & 7) * 8;
+  for (int r = tid >> 3; r < TM + halo; r += 32) {
+    const int src = min(max(m0 - halo + r, 0), rows - 1);
+    *reinterpret_cast<f16x8*>(&sX[r][chunk_c]) =
+        *reinterpret_cast<const f16x8*>(x + (long)src * C + g * CG + chunk_c);
+  }
+  int lpos[MR];
+#pragma unroll
+  for (int b = 0; b < MR; ++b) lpos[b] = pos[min(m0 + fr + 32 * b, rows - 1)];
+  // the epilogue's 8 MR rows a wave, four channels of 2 MR rows a lane
+  const int tr = wave * 8 * MR + (lane >> 4), col_lane = (lane & 15) * 4, col = g * CG + col_lane;
+  const float4 bias4 = *reinterpret_cast<const float4*>(bias + col);
+  float4 hv[2 * MR];
+#pragma unroll
+  for (int p = 0; p < 2 * MR; ++p) {
+    const int row = min(m0 + tr + 4 * p, rows - 1);
+    if (h) hv[p] = *reinterpret_cast<const float4*>(h + (long)row * C + col);
+  }
+  __syncthreads();
+
+  f32x16 acc[2][MR];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int b = 0; b < MR; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[t][b][e] = 0.0f;
+  const f16x8 zero8 = {};
+  for (int jb = j0; jb < j1; jb += PD) {
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+      const int j = jb + u;
+      if (j >= j1) break;
+      fetch(wr[(u + PD - 1) % PD], j + PD - 1);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int b = 0; b < MR; ++b) {
+          // rows before the row's document start read as zero (per-document causal padding)
+          const f16x8 v = *reinterpret_cast<const f16x8*>(&sX[fr + 32 * b + j][ks * 16 + fh * 8]);
+          const f16x8 xb = lpos[b] + j >= halo ? v : zero8;
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[t][b] = mfma32(wr[u][4 * t + ks], xb, acc[t][b]);
+        }
     }
+  }
+  __syncthreads();  // every wave has read the window: the sums take its place
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int b = 0; b < MR; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(&part[wave][fr + 32 * b][t * 32 + q * 8 + fh * 4]) = f32x4{
+            acc[t][b][4 * q], acc[t][b][4 * q + 1], acc[t][b][4 * q + 2], acc[t][b][4 * q + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < 2 * MR; ++p) {
+    const int r = tr + 4 * p, row = m0 + r;
+    f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < kTapGroups; ++k)
+      v += *reinterpret_cast<const f32x4*>(&part[k][r][col_lane]);
+    if (row < rows) conv_finish(v, bias4, hv[p], (long)row * C + col, out_f16, h);
   }
 }
 
@@ -166,9 +310,16 @@ hipError_t conv_causal_mish(const f16* x, int C, const f16* w, const float* bias
                             hipStream_t stream, const int32_t* rows_live) {
   if (rows <= 0) return hipSuccess;
   if (taps < 1 || taps > MAX_TAPS || C % CG != 0) return hipErrorInvalidValue;
-  dim3 grid((rows + TM - 1) / TM, C / CG);
-  hipLaunchKernelGGL(conv_kernel, grid, dim3(256), 0, stream, x, C, w, bias, taps, pos, rows,
-                     out_f16, h, rows_live);
+  // Channel groups are the grid's fast axis: consecutive workgroups go to the XCDs in turn, so an XCD
+  // holds the weights of C/CG / 8 groups in its L2 and reads each once, not all of them.
+  // The rule is on the launch's capacity, so that a captured launch and its replays take one form.
+  const int groups = C / CG;
+  const auto tiles = [&](int tm) { return (rows + tm - 1) / tm; };
+  const int tm = tiles(32) * groups <= kCUs ? 32 : tiles(64) * groups <= kCUs ? 64 : 128;
+  const dim3 grid(groups, tiles(tm));
+  auto kernel = tm == 32 ? conv_small_kernel<1> : tm == 64 ? conv_small_kernel<2> : conv_kernel;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, C, w, bias, taps, pos, rows, out_f16, h,
+                     rows_live);
   return hipGetLastError();
 }
 

@@ -491,6 +491,24 @@ def test_32x64_gemm_tile_gives_the_same_bits(fcv, stress2, monkeypatch, lengths)
         assert torch.equal(run(), ref), shape
 
 
+@pytest.mark.parametrize("lengths", [[1, 30, 1], [31, 2], [480, 32], [481, 32], [500, 13, 500, 11],
+                                     [500, 13, 500, 12]])
+def test_position_conv_forms_give_the_same_bits(fcv, stress2, lengths):
+    """A document alone (32 rows a tile, the taps split over the waves) and within packs on both
+    sides of the steps to 64 and 128 rows a tile (512 and 1024 rows at 16 channel groups), with
+    documents shorter than the taps and tiles that end on and off the document's edge."""
+    _, est = stress2
+    x, mu, cond, spks, tt = random_packed(lengths, seed=69, t=0.4)
+    say(f"[conv forms] {lengths}")
+    out = est.forward_packed(x, mu, cond, spks, tt[:1], lengths, streaming=True).clone()
+    at = 0
+    for i, n in enumerate(lengths):
+        cut = slice(at, at + n)
+        one = est.forward_packed(x[cut], mu[cut], cond[cut], spks[i:i + 1], tt[:1], [n],
+                                 streaming=True)
+        assert torch.equal(out[cut], one), (i, n)
+        at += n
+
 
 def test_streaming_prefix_stability_gate_a(fcv, stress2):
     """Reference Gate A (tests/gpu/test_flashinfer_streaming_estimator.py:58-89): with the
