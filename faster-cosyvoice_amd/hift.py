@@ -32,8 +32,8 @@ def _ceil(v: int, m: int) -> int:
 # Smallest capacity (Mel frames of one packed call) whose call replays its captured graph when
 # the caller leaves ``graph`` to the vocoder.  The eager call is one C-ABI call that enqueues the
 # launch sequence faster than the GPU drains it, so a replay saves host time but no device time:
-# on one MI355X a 68-frame streaming chunk took 2.31 ms either way, and config 3's packed
-# groups 19.4 ms either way.  Small calls (streaming chunks) therefore launch eagerly.
+# on one MI355X a 68-frame streaming chunk took 0.788 ms replayed and 0.784 eagerly, and config 3's
+# packed groups 8.71 and 8.69 ms.  Small calls (streaming chunks) therefore launch eagerly.
 HIFT_GRAPH_MIN_FRAMES = 1024
 
 
@@ -338,8 +338,7 @@ class HiFTVocoder:
 
         The requests run as ``concurrency`` groups (default: 2 when there are at least 2),
         balanced by Mel frames, each a packed call on its own handle over the shared weights
-        and its own stream, all in flight together (one packed call of 8 requests at config 3:
-        23.5 ms; two groups: 22.1 ms).
+        and its own stream, all in flight together.
 
         Each call runs in a capacity bucket (``capacity_bucket``); with ``graph`` the launch
         sequence is captured on a bucket's second call and replayed for every later layout in
