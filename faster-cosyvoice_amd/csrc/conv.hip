@@ -9,23 +9,26 @@
 // zero padding of the reference's F.pad).
 //
 // An output's sum is taken over kTapGroups groups of consecutive taps, each from zero, the groups
-// added in order, whatever the tile: small launches give each group a wave.  A launch of few rows is
-// bound by one workgroup's chain of taps, each a barrier and an LDS round trip, on a part of the CUs
-// (48 of 256 at 300 rows); a large one by the LDS reads of its MFMAs.  Three forms; a forward of one
-// block holds two launches, and took on one MI355X (us, at 16 channel groups), in turn:
-//   rows                        60    300   500   520   700   1000  1040  1500  4500
-//   32 rows, a group a wave     90    97    104   122+  .     .     157+  168   340
-//   64 rows, a group a wave     94    100   112+  112   122   125   146+  158   293
-//   128 rows, all taps a wave   102   109   .     120+  .     .     140   152   248
-//   (+ at 550 and 1100 rows.)  128 rows in one chain of taps, the channel groups on the grid's slow
-//   axis, was the only form before: 103, 112, 118, 120, 129, 135, 140, 152, 248.
+// added in order, whatever the tile: small launches give each group waves of its own.  A launch of
+// few rows is bound by one workgroup's chain of taps, each a barrier and an LDS round trip, on a part
+// of the CUs (48 of 256 at 300 rows with 128-row tiles); a large one by the LDS reads of its MFMAs.
+// Hence three forms.  A forward of one block holds two launches and took on one MI355X (us, at 16
+// channel groups):
+//   rows                        60    300   500   520   700   1000  1040  1500  4500  9000
+//   this rule                   90    97    104   113   123   132   143   159   263   439
+//   128 rows in one chain of taps, the channel groups on the grid's slow axis (the only form before)
+//                               103   111   119   121   129   139   146   160   266   439
+// and with four groups of taps, a wave each, at other sizes in another run: 32-row tiles 122 at
+// 550 rows, 157 at 1100; 64-row ones 112 and 146; 128-row ones 120 and 141.  So each form runs while
+// its workgroups are at most one per CU.  Four groups cost the large form 1.6 us a launch in the
+// additions (two: none that shows) and gained the small ones nothing over two.
 #include "kernels.hpp"
 
 namespace fcv {
 namespace {
 
 constexpr int CG = 64;        // channels per group
-constexpr int kTapGroups = 4;
+constexpr int kTapGroups = 2;
 constexpr int LDP = CG + 8;   // padded LDS row (f16): 16 consecutive rows hit distinct banks
 constexpr int MAX_TAPS = 31;
 constexpr int SPITCH = CG + 4;  // fp32 staging row
@@ -193,10 +196,10 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const f16* __restrict__ x,
 }
 
 // The small launches' form: a workgroup owns 32 MR rows x 64 channels and each of its waves one group
-// of taps, with the weights straight from global memory two taps ahead, so no wave waits for another
+// of taps for 32 of the channels, with the weights straight from global memory two taps ahead, so no wave waits for another
 // between the window and the sums' addition in LDS.
 template <int MR>
-__global__ __launch_bounds__(64 * kTapGroups, 2) void conv_small_kernel(
+__global__ __launch_bounds__(128 * kTapGroups, 2) void conv_small_kernel(
     const f16* __restrict__ x, int C, const f16* __restrict__ w, const float* __restrict__ bias,
     int taps, const int32_t* __restrict__ pos, int rows, f16* __restrict__ out_f16,
     float* __restrict__ h, const int32_t* __restrict__ rows_live) {
@@ -218,20 +221,18 @@ __global__ __launch_bounds__(64 * kTapGroups, 2) void conv_small_kernel(
   const int fr = lane & 31, fh = lane >> 5;
   const int halo = taps - 1;
   const int group = tap_group(taps);
-  const int j0 = wave * group, j1 = min(j0 + group, taps);
+  const int tile = wave & 1;  // the wave's channel tile, of the tap group wave / 2
+  const int j0 = (wave >> 1) * group, j1 = min(j0 + group, taps);
 
-  // this wave's first taps' weights: fragment (t, ks) of lane l is channel 32 t + l % 32, inputs
+  // this wave's first taps' weights: fragment ks of lane l is channel 32 tile + l % 32, inputs
   // 16 ks + 8 (l / 32) + 0..7
   constexpr int PD = 3;
-  f16x8 wr[PD][8];
-  const f16* wg = w + ((long)g * taps * CG + fr) * CG + fh * 8;
-  auto fetch = [&](f16x8 (&f)[8], int j) {
+  f16x8 wr[PD][4];
+  const f16* wg = w + ((long)g * taps * CG + tile * 32 + fr) * CG + fh * 8;
+  auto fetch = [&](f16x8 (&f)[4], int j) {
     const f16* src = wg + (long)min(j, taps - 1) * CG * CG;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-        f[4 * t + ks] = *reinterpret_cast<const f16x8*>(src + t * 32 * CG + ks * 16);
+    for (int ks = 0; ks < 4; ++ks) f[ks] = *reinterpret_cast<const f16x8*>(src + ks * 16);
   };
 #pragma unroll
   for (int u = 0; u < PD - 1; ++u) fetch(wr[u], j0 + u);
@@ -256,13 +257,11 @@ __global__ __launch_bounds__(64 * kTapGroups, 2) void conv_small_kernel(
   }
   __syncthreads();
 
-  f32x16 acc[2][MR];
+  f32x16 acc[MR];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int b = 0; b < MR; ++b)
 #pragma unroll
-    for (int b = 0; b < MR; ++b)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[t][b][e] = 0.0f;
+    for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
   const f16x8 zero8 = {};
   for (int jb = j0; jb < j1; jb += PD) {
 #pragma unroll
@@ -277,20 +276,17 @@ __global__ __launch_bounds__(64 * kTapGroups, 2) void conv_small_kernel(
           // rows before the row's document start read as zero (per-document causal padding)
           const f16x8 v = *reinterpret_cast<const f16x8*>(&sX[fr + 32 * b + j][ks * 16 + fh * 8]);
           const f16x8 xb = lpos[b] + j >= halo ? v : zero8;
-#pragma unroll
-          for (int t = 0; t < 2; ++t) acc[t][b] = mfma32(wr[u][4 * t + ks], xb, acc[t][b]);
+          acc[b] = mfma32(wr[u][ks], xb, acc[b]);
         }
     }
   }
   __syncthreads();  // every wave has read the window: the sums take its place
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int b = 0; b < MR; ++b)
 #pragma unroll
-    for (int b = 0; b < MR; ++b)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<f32x4*>(&part[wave][fr + 32 * b][t * 32 + q * 8 + fh * 4]) = f32x4{
-            acc[t][b][4 * q], acc[t][b][4 * q + 1], acc[t][b][4 * q + 2], acc[t][b][4 * q + 3]};
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f32x4*>(&part[wave >> 1][fr + 32 * b][tile * 32 + q * 8 + fh * 4]) =
+          f32x4{acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2], acc[b][4 * q + 3]};
   __syncthreads();
 #pragma unroll
   for (int p = 0; p < 2 * MR; ++p) {
