@@ -99,4 +99,23 @@ __device__ __forceinline__ float mish(float x) {
 
 __device__ __forceinline__ float silu(float x) { return x * hw_rcp(1.0f + hw_exp2(-1.4426950408889634f * x)); }
 
+// Lane-strided 16-byte global -> LDS copy: lane l copies the 16 bytes at base + voff (its own
+// 32-bit byte offset from a wave-uniform 64-bit base held in SGPRs) to bytes [16 l, 16 l + 16)
+// from the wave-uniform LDS address `lds`.  With the base and the LDS address scalar, a copy
+// costs one m0 write and one load instruction; the K advance is a scalar add on the base.
+// Issued as inline asm so the compiler does not treat every later LDS read as dependent on it
+// (it would wait for vmcnt(0) before each one); the K loop orders these copies with explicit
+// vmcnt waits and barriers instead.  (m0 is named as a clobber on purpose: the copy's LDS base
+// lives there.)  gfx9 needs one wait state between a scalar write of m0 and an LDS copy that reads
+// it; the compiler's hazard pass does not look inside an asm, so the s_nop is part of it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 }  // namespace fcv

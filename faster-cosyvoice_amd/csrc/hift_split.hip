@@ -50,17 +50,6 @@ constexpr long kSmallBelow = 256;
 // hit 16 distinct 16-byte bank groups
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// lane l copies 16 bytes at base + voff to LDS bytes [16 l, 16 l + 16) from the scalar address
-__device__ __forceinline__ void lds_dma16(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(voff), "s"(base)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   static_assert(N < 64, "vmcnt");
