@@ -494,9 +494,9 @@ def test_32x64_gemm_tile_gives_the_same_bits(fcv, stress2, monkeypatch, lengths)
 @pytest.mark.parametrize("lengths", [[1, 30, 1], [31, 2], [480, 32], [481, 32], [500, 13, 500, 11],
                                      [500, 13, 500, 12]])
 def test_position_conv_forms_give_the_same_bits(fcv, stress2, lengths):
-    """A document alone (32 rows a tile, the taps split over the waves) and within packs on both
-    sides of the steps to 64 and 128 rows a tile (512 and 1024 rows at 16 channel groups), with
-    documents shorter than the taps and tiles that end on and off the document's edge."""
+    """A document alone (32 rows a tile) and within packs on both sides of the step to 128 rows a
+    tile (512 rows at 16 channel groups), with documents shorter than the taps and tiles that end on
+    and off the document's edge."""
     _, est = stress2
     x, mu, cond, spks, tt = random_packed(lengths, seed=69, t=0.4)
     say(f"[conv forms] {lengths}")
