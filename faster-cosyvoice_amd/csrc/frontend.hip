@@ -8,11 +8,11 @@
 //   conv2: Y^T[o][t]  = W2[o][k] . G[k][t],  k = tap * C + c,  G[tap*C+c][t] = h(t - 2 + tap)[c]
 // with the weights as the A operand (rows = output channels) and the gathered token rows as
 // the B operand, so a lane's four accumulators are four consecutive channels of one token and
-// leave as one 16-byte store.  Both operands are read from global memory, 16 K values per chunk;
-// lane (i, g) of the 16x16x4 MFMA feeds k = 4g + s at step s, so one 16-byte read covers four
-// steps.  A call has 10 to a few thousand tokens, so what bounds it is the chain of a wave's loads and
-// MFMAs: the waves of a workgroup split K (conv1 by taps, conv2 eight ways) and add their sums in
-// LDS in a fixed order.  No split depends on the batch, so a document's result does not depend on
+// leave as one 16-byte store.  Operands go 16 K values per chunk, straight from global memory in short
+// calls and through LDS in longer ones; lane (i, g) of the 16x16x4 MFMA feeds k = 4g + s at step s, so
+// one 16-byte read covers four steps.  A call has 10 to a few thousand tokens, so what bounds it is the
+// chain of a wave's loads and MFMAs.  conv1's sums are one chain over K, conv2's eight, added in a fixed
+// order; neither depends on the batch or the form, so a document's result does not depend on
 // what it is packed with.  The per-document prefix sums travel by value in the kernel
 // arguments (DocTables, at most kMaxDocs documents), so a call needs no host-to-device copy and
 // no synchronisation.
@@ -32,11 +32,14 @@ constexpr int kSplit = 8;     // conv2 K split (fixed)
 constexpr int kPitch = 20;    // LDS row pitch in floats (16 + 4: conflict-free 16-byte reads)
 constexpr int kTileT = 64;    // token rows per workgroup of the longer calls' convolutions
 constexpr int kTileC = 128;   // conv1 output channels per workgroup there
-// Output tokens from which the longer calls' forms run, whose tiles read the operands fewer times: at
-// 2298 tokens 35 + 27.5 + 4.7 us in three kernels against 37 + 43 in the short calls' two.
-constexpr int kWideFrom = 512;
+// The short calls' forms run while conv2's workgroups there (five to 16 tokens) are at most one a CU:
+// all token features in them and in the longer calls', us: 90 tokens 22 and 41, 300 27 and 42, 512 27
+// and 42, 600 32 and 45, 700 32 and 45, 800 37 and 46; past that 850 50 and 46, 1000 51 and 44, 2298
+// 83 and 62.
+constexpr int kShortGroups = 256;
 constexpr size_t kAlign = 256;
 constexpr int kMaxDocs = FCV_FLOW_MAX_DOCS;
+constexpr int kMaxTaps = 8;   // conv1: lookahead + 1
 
 // two exclusive prefix sums over the documents of a call, passed by value
 struct DocTables {
@@ -62,96 +65,67 @@ __device__ __forceinline__ int find_doc(const int32_t* cu, int n_docs, int row) 
 __device__ __forceinline__ float leaky_relu(float x) { return x > 0.0f ? x : 0.01f * x; }
 
 // ---- conv1: h[t][c] = leaky_relu(b1[c] + sum_k W1[c][k] E[k][t]) ---------------------------
-// Workgroup tile 32 channels x 32 tokens; wave w sums taps w, w + 4, .. from global memory, a tap's
-// five chunks of 16 K values in flight together, and the four sums are added in LDS in wave order.  A
-// tile of 128 channels x 64 tokens with K in one chain through LDS ran 16 workgroups of 20 steps for
-// a streaming chunk: 90 tokens 20.7 -> 5.8 us.
+// An output's sum is one chain over K in both forms.  The short calls' form: a workgroup owns 32
+// channels x 32 tokens and each wave a 16x16 tile of them, its operands straight from global memory,
+// two taps (ten chunks of 16 K values) in flight.  A tile of 128 channels x 64 tokens walks K through
+// LDS, a barrier a chunk, in 16 workgroups for a streaming chunk: 90 tokens 20.7 us there, 8.1 here.
+// (Four waves with a tap each, added in LDS: 5.8, but not the longer form's rounding.)
 // tab.a = token prefix sums, tab.b = output-token prefix sums
 __global__ __launch_bounds__(256) void lookahead_conv1_kernel(
     const int32_t* __restrict__ tokens, const DocTables tab, int n_docs, int n_out,
     const float* __restrict__ embed, int vocab, const float* __restrict__ W1,
     const float* __restrict__ b1, int C, int taps, float* __restrict__ h) {
   constexpr int CPT = kFeat / kBK;  // chunks per tap
-  constexpr int N = 2, TS = 16 * N;
-  __shared__ __attribute__((aligned(16))) float part[4][TS][TS + 4];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const int t0 = blockIdx.x * TS;
-  const int c0 = blockIdx.y * TS;
+  const int t = blockIdx.x * 32 + (wave >> 1) * 16 + li;  // this lane's token
+  const int c0 = blockIdx.y * 32 + (wave & 1) * 16;       // this wave's channels
   const long K = (long)taps * kFeat;
 
-  // lane (li, lg): K values 4 lg .. 4 lg + 3 of a chunk, of channel / token li of each 16-tile
-  int tb[N], n_left[N];  // token index of tap 0 and tokens left in the document from there
-#pragma unroll
-  for (int b = 0; b < N; ++b) {
-    const int t = t0 + 16 * b + li;
-    tb[b] = n_left[b] = 0;
-    if (t < n_out) {
-      const int d = find_doc(tab.b, n_docs, t);
-      tb[b] = tab.a[d] + (t - tab.b[d]);
-      n_left[b] = tab.a[d + 1] - tb[b];
-    }
+  int tb = 0, n_left = 0;  // token index of tap 0 and tokens left in the document from there
+  if (t < n_out) {
+    const int d = find_doc(tab.b, n_docs, t);
+    tb = tab.a[d] + (t - tab.b[d]);
+    n_left = tab.a[d + 1] - tb;
   }
-  f32x4 acc[N][N];
+  int id[kMaxTaps];
 #pragma unroll
-  for (int a = 0; a < N; ++a)
-#pragma unroll
-    for (int b = 0; b < N; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int tap = wave; tap < taps; tap += 4) {
-    const float* w = W1 + (c0 + li) * K + tap * kFeat + 4 * lg;
-    const float* e[N];
-    bool live[N];
-#pragma unroll
-    for (int b = 0; b < N; ++b) {
-      live[b] = tap < n_left[b];
-      const int id = live[b] ? min(max(tokens[tb[b] + tap], 0), vocab - 1) : 0;
-      e[b] = embed + (long)id * kFeat + 4 * lg;
-    }
-    f32x4 av[CPT][N], bv[CPT][N];
+  for (int j = 0; j < kMaxTaps; ++j)
+    id[j] = j < taps && j < n_left ? min(max(tokens[tb + j], 0), vocab - 1) : 0;
+  // lane (li, lg): K values 4 lg .. 4 lg + 3 of a chunk, of channel / token li
+  const float* w = W1 + (c0 + li) * K + 4 * lg;
+  f32x4 av[2][CPT], bv[2][CPT];
+  auto fetch = [&](int buf, int j, int token) {
+    const float* e = embed + (long)token * kFeat + 4 * lg;
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-#pragma unroll
-      for (int a = 0; a < N; ++a)
-        av[c][a] = *reinterpret_cast<const f32x4*>(w + 16 * a * K + c * kBK);
-#pragma unroll
-      for (int b = 0; b < N; ++b) {
-        bv[c][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (live[b]) bv[c][b] = *reinterpret_cast<const f32x4*>(e[b] + c * kBK);
-      }
+      av[buf][c] = *reinterpret_cast<const f32x4*>(w + (j * CPT + c) * kBK);
+      bv[buf][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (j < n_left) bv[buf][c] = *reinterpret_cast<const f32x4*>(e + c * kBK);
     }
+  };
+  f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+  fetch(0, 0, id[0]);
+#pragma unroll
+  for (int j = 0; j < kMaxTaps; ++j) {
+    if (j >= taps) break;
+    if (j + 1 < taps) fetch((j + 1) & 1, j + 1, id[(j + 1) % kMaxTaps]);
 #pragma unroll
     for (int c = 0; c < CPT; ++c)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int a = 0; a < N; ++a)
-#pragma unroll
-          for (int b = 0; b < N; ++b) acc[a][b] = mfma16(av[c][a][s], bv[c][b][s], acc[a][b]);
+      for (int s = 0; s < 4; ++s) acc = mfma16(av[j & 1][c][s], bv[j & 1][c][s], acc);
   }
-  // D[i = channel][j = token]: lane holds token li, channels 4 lg + 0..3 of each tile
+  // D[i = channel][j = token]: lane holds token li, channels 4 lg + 0..3
+  if (t >= n_out) return;
+  const int c = c0 + 4 * lg;
+  const f32x4 bias = *reinterpret_cast<const f32x4*>(b1 + c);
+  f32x4 v;
 #pragma unroll
-  for (int a = 0; a < N; ++a)
-#pragma unroll
-    for (int b = 0; b < N; ++b)
-      *reinterpret_cast<f32x4*>(&part[wave][16 * b + li][16 * a + 4 * lg]) = acc[a][b];
-  __syncthreads();
-  constexpr int TPT = TS / 4;  // threads a token
-  const int cl = tid % TPT * 4;
-  const f32x4 bias = *reinterpret_cast<const f32x4*>(b1 + c0 + cl);
-  for (int tl = tid / TPT; tl < TS && t0 + tl < n_out; tl += 256 / TPT) {
-    f32x4 v = *reinterpret_cast<const f32x4*>(&part[0][tl][cl]);
-#pragma unroll
-    for (int q = 1; q < 4; ++q) v += *reinterpret_cast<const f32x4*>(&part[q][tl][cl]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = leaky_relu(v[i] + bias[i]);
-    *reinterpret_cast<f32x4*>(h + (long)(t0 + tl) * C + c0 + cl) = v;
-  }
+  for (int e = 0; e < 4; ++e) v[e] = leaky_relu(acc[e] + bias[e]);
+  *reinterpret_cast<f32x4*>(h + (long)t * C + c) = v;
 }
 
-// ---- conv1 of longer calls (from kWideFrom tokens, at most four taps): the same sums ----------
+// ---- conv1 of longer calls (see kShortGroups): the same sums -------------------------------------
 // Workgroup tile 128 channels x 64 tokens; wave (wc, wt) owns 64 channels x 32 tokens.
 // tab.a = token prefix sums, tab.b = output-token prefix sums
 __global__ __launch_bounds__(256) void lookahead_conv1_wide_kernel(
@@ -202,12 +176,11 @@ __global__ __launch_bounds__(256) void lookahead_conv1_wide_kernel(
     *reinterpret_cast<f32x4*>(&sB[buf][lr][4 * lq]) = rb;
   };
 
-  // the tap's sum, and the sum of the taps before it (a tap is a wave's sum in the short form)
-  f32x4 acc[4][2], total[4][2];
+  f32x4 acc[4][2];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = total[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   fetch(0);
   stash(0);
@@ -232,15 +205,6 @@ __global__ __launch_bounds__(256) void lookahead_conv1_wide_kernel(
       for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = mfma16(av[a][s], bv[b][s], acc[a][b]);
-    if ((kc + 1) % CPT == 0) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          total[a][b] += acc[a][b];
-          acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    }
     stash(cur ^ 1);
     __syncthreads();
   }
@@ -256,14 +220,14 @@ __global__ __launch_bounds__(256) void lookahead_conv1_wide_kernel(
       const f32x4 bias = *reinterpret_cast<const f32x4*>(b1 + c);
       f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = leaky_relu(total[a][b][e] + bias[e]);
+      for (int e = 0; e < 4; ++e) v[e] = leaky_relu(acc[a][b][e] + bias[e]);
       *reinterpret_cast<f32x4*>(h + (long)t * C + c) = v;
     }
   }
 }
 
 // ---- conv2: mu rows ratio*t .. +ratio-1 = b2 + sum_k W2[o][k] G[k][t] + e(t) ------------------
-// The short calls' form (below kWideFrom tokens; the same sums as the two kernels below).  Workgroup
+// The short calls' form (see kShortGroups; the same sums as the two kernels below).  Workgroup
 // tile 16 outputs x 16 tokens; its kSplit waves take an equal run of K each, straight from global
 // memory kDepth chunks ahead, and the sums are added in LDS in order, with the bias, the residual and
 // the repeat.  90 tokens: 18.3 + 3.9 us in two kernels, 15.4 in this one; 2298 tokens 27.5 + 4.7
@@ -445,35 +409,50 @@ __global__ __launch_bounds__(256) void lookahead_finish_kernel(
 }
 
 // ---- speaker: out[n] = W (x / max(||x||, 1e-12)) + b -----------------------------------------
-// One workgroup per x-vector; each wave keeps the normalised vector in registers (lane l: elements
-// l, l + 64, ..) and takes every 16th output, so a weight row is one coalesced read.  (A lane a
-// row, in one wave, walked the rows element by element: 7.4 us for one vector, now 4.4.)
-__global__ __launch_bounds__(1024) void speaker_kernel(const float* __restrict__ x, int D,
-                                                       const float* __restrict__ W,
-                                                       const float* __restrict__ b, int F,
-                                                       float* __restrict__ out) {
-  constexpr int E = 4;  // D <= 256
-  const int n = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float v[E];
-  float ss = 0.0f;
+// One wave per x-vector and 16 outputs: a lane walks the row of one output, in order, 64 values of it
+// in flight: one vector 4.0 us.  (One wave for all outputs, a value at a time: 7.4.)
+__global__ __launch_bounds__(64) void speaker_kernel(const float* __restrict__ x, int D,
+                                                     const float* __restrict__ W,
+                                                     const float* __restrict__ b, int F,
+                                                     float* __restrict__ out) {
+  typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));  // a row starts anywhere
+  constexpr int kPart = 64;
+  __shared__ __attribute__((aligned(16))) float sx[256];  // D <= 256
+  const int n = blockIdx.x, lane = threadIdx.x;
+  const int o = blockIdx.y * 16 + lane;
+  const bool live = lane < 16 && o < F;
+  const float* w = W + (long)(live ? o : 0) * D;
+  f32x4 r[kPart / 4];
+  auto fetch = [&](int i0) {
 #pragma unroll
-  for (int i = 0; i < E; ++i) {
-    v[i] = lane + 64 * i < D ? x[(long)n * D + lane + 64 * i] : 0.0f;
-    ss = fmaf(v[i], v[i], ss);
+    for (int i = 0; i < kPart / 4; ++i)
+      if (live && i0 + 4 * i + 4 <= D) r[i] = *reinterpret_cast<const row4*>(w + i0 + 4 * i);
+  };
+  fetch(0);
+  float ss = 0.0f;
+  for (int i = lane; i < D; i += 64) {
+    const float v = x[(long)n * D + i];
+    sx[i] = v;
+    ss = fmaf(v, v, ss);
   }
   const float denom = fmaxf(sqrtf(wave_sum(ss)), 1e-12f);
+  __syncthreads();
+  for (int i = lane; i < D; i += 64) sx[i] = sx[i] / denom;
+  __syncthreads();
+  float acc = 0.0f;
+  for (int i0 = 0; i0 < D; i0 += kPart) {
+    if (i0) fetch(i0);
 #pragma unroll
-  for (int i = 0; i < E; ++i) v[i] = v[i] / denom;
-  for (int o = wave; o < F; o += 16) {
-    const float* w = W + (long)o * D;
-    float acc = 0.0f;
+    for (int i = 0; i < kPart / 4; ++i) {
+      if (i0 + 4 * i + 4 > D) break;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(sx + i0 + 4 * i);
 #pragma unroll
-    for (int i = 0; i < E; ++i)
-      if (lane + 64 * i < D) acc = fmaf(w[lane + 64 * i], v[i], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) out[(long)n * F + o] = acc + b[o];
+      for (int e = 0; e < 4; ++e) acc = fmaf(r[i][e], v[e], acc);
+    }
   }
+  if (!live) return;
+  for (int i = D & ~3; i < D; ++i) acc = fmaf(w[i], sx[i], acc);
+  out[(long)n * F + o] = acc + b[o];
 }
 
 // ---- prompt copy: cond[row] = prompt[...] for the first min(plen, mel_len) rows, else 0 ------
@@ -568,8 +547,8 @@ int launch_token_features(const FcvFlowDims& d, const FcvFlowWeights& w, const i
                           hipStream_t stream) {
   const FlowLayout L = flow_layout(d, n_out);
   float* hid = reinterpret_cast<float*>(ws + L.hidden);
-  const bool wide = n_out >= kWideFrom;
-  if (wide && d.lookahead < 4)
+  const bool wide = (n_out + 15) / 16 * (kFeat / 16) > kShortGroups;
+  if (wide)
     hipLaunchKernelGGL(lookahead_conv1_wide_kernel,
                        dim3((n_out + kTileT - 1) / kTileT, d.channels / kTileC), dim3(256), 0, stream,
                        tokens, tab, n_docs, n_out, w.embed, d.vocab, w.la1_w, w.la1_b, d.channels,
@@ -714,8 +693,8 @@ int fcv_flow_speaker(const FcvFlowDims* dims, const FcvFlowWeights* weights, con
   FCV_CHECK(weights && weights->spk_w && weights->spk_b, FCV_ERR_INVALID, "null weight pointer");
   FCV_CHECK(xvec && spks_out, FCV_ERR_INVALID, "null argument");
   FCV_CHECK(n >= 1, FCV_ERR_INVALID, "need at least one x-vector");
-  hipLaunchKernelGGL(fcv::speaker_kernel, dim3(n), dim3(1024), 0, stream, xvec, dims->spk_dim,
-                     weights->spk_w, weights->spk_b, dims->feat_dim, spks_out);
+  hipLaunchKernelGGL(fcv::speaker_kernel, dim3(n, (dims->feat_dim + 15) / 16), dim3(64), 0, stream,
+                     xvec, dims->spk_dim, weights->spk_w, weights->spk_b, dims->feat_dim, spks_out);
   FCV_HIP(hipGetLastError());
   return FCV_OK;
 }

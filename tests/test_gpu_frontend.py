@@ -227,3 +227,39 @@ def test_flow_inference_batched_end_to_end(fcv):
         err = rel_l2(out[b].cpu(), want)
         say(f"[fe e2e] request {b} mel rel_l2 {err:.2e}")
         assert err <= 2e-2
+
+
+@pytest.mark.parametrize("lookahead", [0, 1, 4, 6, 7])
+def test_token_features_other_lookaheads(fcv, lookahead):
+    """Every accepted number of conv1 taps, in the short calls' form and in packs on both sides of the
+    step to the longer calls' form (816 tokens): against the oracle, and bit for bit alone or packed."""
+    dims = fcv.synthetic.FlowDims(vocab=97, channels=256, lookahead=lookahead)
+    sd = fcv.synthetic.random_flow_state_dict(dims, seed=8)
+    fe = _frontend(fcv, dims, sd)
+    g = torch.Generator().manual_seed(9)
+    lengths = [1, 5, 8, 33, 769, 1]
+    toks = [torch.randint(0, 97, (n,), generator=g).tolist() for n in lengths]
+    say(f"[fe lookahead {lookahead}]")
+    alone = [fe.token_features([t])[0] for t in toks]
+    for part in (slice(0, 5), slice(0, 6)):  # 816 and 817 tokens
+        mu, _ = fe.token_features(toks[part])
+        assert torch.equal(mu, torch.cat(alone[part]))
+    ref = torch.cat([F.streaming_token_features(sd, t, True, lookahead=lookahead)[0] for t in toks])
+    assert rel_l2(mu, ref) <= FEAT_TOL
+
+
+@pytest.mark.parametrize("dim", [1, 3, 64, 190, 255, 256])
+def test_speaker_projection_other_widths(fcv, dim):
+    """x-vector widths off the four-value loads and at the largest."""
+    dims = fcv.synthetic.FlowDims(vocab=5, channels=128)
+    sd = fcv.synthetic.random_flow_state_dict(dims, seed=3)
+    g = torch.Generator().manual_seed(10)
+    sd["spk_embed_affine_layer.weight"] = torch.randn(80, dim, generator=g)
+    fe = fcv.FlowFrontEnd(vocab_size=5, channels=128, spk_embed_dim=dim, device="cuda:0")
+    fe.load_reference_state_dict(sd)
+    fe.finalize_weights()
+    x = torch.randn(5, dim, generator=g)
+    say(f"[fe speaker {dim}]")
+    ref = F.speaker_projection(x, sd["spk_embed_affine_layer.weight"],
+                               sd["spk_embed_affine_layer.bias"])
+    assert rel_l2(fe.speaker(x), ref) <= FEAT_TOL
