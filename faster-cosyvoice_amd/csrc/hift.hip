@@ -38,21 +38,15 @@ __device__ __forceinline__ f64x4 mfma_16x16x4(double a, double b, const f64x4& c
 
 __device__ __forceinline__ double elu(double x) { return x > 0.0 ? x : expm1(x); }
 
-// epilogue of one output element (row, channel c) from its accumulator value; m: raised to the
-// largest finite magnitudes written to out and to the Snake output (fp32)
-__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, float acc, float2& m) {
+// epilogue of one output element (row, channel c) from its accumulator value
+__device__ __forceinline__ void conv_store1(const HiftConv& p, long row, int c, float acc) {
   float v = acc + static_cast<const float*>(p.bias)[c];
   const long i = row * p.ldo + c;
   if (p.add) v = v + static_cast<const float*>(p.add)[row * p.ld_add + c];
   if (p.mode == HIFT_ACC_ADD) v = static_cast<const float*>(p.accin)[i] + v;
   if (p.mode == HIFT_ACC_ADD_DIV) v = (static_cast<const float*>(p.accin)[i] + v) / p.div;
   if (p.snake_out) v = snake(v, p.alpha[c], p.inv_alpha[c]);
-  if (p.n_snakes) {
-    const float w = snake(v, p.snakes[0].alpha[c], p.snakes[0].inv_alpha[c]);
-    p.snakes[0].out[i] = w;
-    m.y = fmaxf(m.y, finite_abs(w));
-  }
-  m.x = fmaxf(m.x, finite_abs(v));
+  if (p.n_snakes) p.snakes[0].out[i] = snake(v, p.snakes[0].alpha[c], p.snakes[0].inv_alpha[c]);
   static_cast<float*>(p.out)[i] = v;
 }
 
@@ -60,8 +54,7 @@ __device__ __forceinline__ float4 ld4f(const float* q) { return *reinterpret_cas
 
 // conv_store1 for the four consecutive fp32 channels c .. c + 3 of one row, with 16-byte loads
 // and stores (same operations in the same order, so the results are bit-identical)
-__device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, const f32x4& acc,
-                                            float2& m) {
+__device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, const f32x4& acc) {
   const float4 b = ld4f(static_cast<const float*>(p.bias) + c);
   float v[4] = {acc[0] + b.x, acc[1] + b.y, acc[2] + b.z, acc[3] + b.w};
   const long i = row * p.ldo + c;
@@ -85,26 +78,22 @@ __device__ __forceinline__ void conv_store4(const HiftConv& p, long row, int c, 
     float w[4];
 #pragma unroll 1
     for (int e = 0; e < 4; ++e) w[e] = snake(v[e], q.alpha[c + e], q.inv_alpha[c + e]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) m.y = fmaxf(m.y, finite_abs(w[e]));
     *reinterpret_cast<float4*>(q.out + i) = float4{w[0], w[1], w[2], w[3]};
   }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) m.x = fmaxf(m.x, finite_abs(v[e]));
   *reinterpret_cast<float4*>(static_cast<float*>(p.out) + i) = float4{v[0], v[1], v[2], v[3]};
 }
 
 // The 16x16x4 accumulators of lane (li, lg) hold channels cb + 4 lg + e (e = 0..3) of the tile's
 // channel base cb
 __device__ void conv_store(const HiftConv& p, long row, int cb, int lg,
-                           const f32x4& acc, float2& m) {
+                           const f32x4& acc) {
   const int c = cb + 4 * lg;
   if (p.vec4 && c + 3 < p.cout) {
-    conv_store4(p, row, c, acc, m);
+    conv_store4(p, row, c, acc);
     return;
   }
   for (int e = 0; e < 4; ++e)
-    if (c + e < p.cout) conv_store1(p, row, c + e, acc[e], m);
+    if (c + e < p.cout) conv_store1(p, row, c + e, acc[e]);
 }
 
 // BK input channels of one tap per chunk (cin_pad % BK == 0), each lane feeding
@@ -238,9 +227,6 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
   }
 
   // D[i = channel][j = row]: lane holds row li and four channels of each 16x16 tile
-  const int tile_doc = doc_of(docs->b, n_docs, r0);
-  const bool one_doc = min(r0 + TS, rows_out) <= docs->b[tile_doc + 1];
-  float2 tile_max{0.0f, 0.0f};
 #pragma unroll
   for (int b = 0; b < NQ; ++b) {
     const int rr = r0 + wt * (TS / 2) + b * 16 + li;
@@ -248,55 +234,13 @@ __global__ __launch_bounds__(256) void hift_conv_kernel(const HiftConv p) {
     const int d = doc_of(docs->b, n_docs, rr);
     const int pp = rr - docs->b[d];
     const long row_w = p.reflect ? (long)docs->b[d] + d + 1 + pp : rr;
-    float2 m{0.0f, 0.0f};
 #pragma unroll
     for (int a = 0; a < NQ; ++a) {
       const int cb = co0 + wc * (TS / 2) + a * 16;
-      conv_store(p, row_w, cb, lg, acc[a][b], m);
+      conv_store(p, row_w, cb, lg, acc[a][b]);
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
-      if (p.reflect && pp == 1) conv_store(p, (long)docs->b[d] + d, cb, lg, acc[a][b], m);
+      if (p.reflect && pp == 1) conv_store(p, (long)docs->b[d] + d, cb, lg, acc[a][b]);
     }
-    if (one_doc) {
-      tile_max.x = fmaxf(tile_max.x, m.x);
-      tile_max.y = fmaxf(tile_max.y, m.y);
-    } else {
-      if (p.amax_out) raise_amax(p.amax_out, d, blockIdx.x + blockIdx.y, m.x);
-      if (p.snakes[0].amax) raise_amax(p.snakes[0].amax, d, blockIdx.x + blockIdx.y, m.y);
-    }
-  }
-  if (one_doc && (p.amax_out || p.snakes[0].amax)) {
-    __shared__ float wmax[2][4];
-    tile_max.x = wave_max(tile_max.x);
-    tile_max.y = wave_max(tile_max.y);
-    if (lane == 0) {
-      wmax[0][wave] = tile_max.x;
-      wmax[1][wave] = tile_max.y;
-    }
-    __syncthreads();
-    if (tid < 2) {
-      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[0].amax;
-      const float m = fmaxf(fmaxf(wmax[tid][0], wmax[tid][1]), fmaxf(wmax[tid][2], wmax[tid][3]));
-      if (slot) raise_amax(slot, tile_doc, blockIdx.x + blockIdx.y, m);
-    }
-  }
-}
-
-// a workgroup of 256 threads at elements first.. (q a row) raises its rows' documents by each
-// thread's m (i: the thread's element)
-__device__ __forceinline__ void raise_rows_amax(uint32_t* amax, float m, long first, long i,
-                                                long total, int q,
-                                                const HiftDocs* __restrict__ docs) {
-  if (!amax) return;
-  const int d0 = doc_of(docs->b, docs->n, (int)(first / q));
-  if (min(first + 255, total - 1) / q < docs->b[d0 + 1]) {
-    __shared__ float wmax[4];
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-      raise_amax(amax, d0, blockIdx.x, fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
-  } else if (i < total) {
-    raise_amax(amax, doc_of(docs->b, docs->n, (int)(i / q)), blockIdx.x, m);
   }
 }
 
@@ -305,49 +249,29 @@ __global__ __launch_bounds__(256) void snake_kernel(const float* __restrict__ x,
                                                     float* __restrict__ out, int ldo, int C,
                                                     const float* __restrict__ alpha,
                                                     const float* __restrict__ inv_alpha,
-                                                    uint32_t* __restrict__ amax,
                                                     const HiftDocs* __restrict__ docs) {
-  const int rows = docs->b[docs->n];
   const int q = C / 4;
-  const long first = (long)blockIdx.x * blockDim.x, total = (long)rows * q;
-  if (first >= total) return;
-  const long i = first + threadIdx.x;
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long r = i / q;
-  float m = 0.0f;
-  if (i < total) {
-    const int c = (int)(i - r * q) * 4;
-    const f32x4 v = *reinterpret_cast<const f32x4*>(x + r * ldx + c);
-    f32x4 y;
+  if (r >= docs->b[docs->n]) return;
+  const int c = (int)(i - r * q) * 4;
+  const f32x4 v = *reinterpret_cast<const f32x4*>(x + r * ldx + c);
+  f32x4 y;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      y[e] = snake(v[e], alpha[c + e], inv_alpha[c + e]);
-      m = fmaxf(m, finite_abs(y[e]));
-    }
-    *reinterpret_cast<f32x4*>(out + r * ldo + c) = y;
-  }
-  raise_rows_amax(amax, m, first, i, total, q, docs);
+  for (int e = 0; e < 4; ++e) y[e] = snake(v[e], alpha[c + e], inv_alpha[c + e]);
+  *reinterpret_cast<f32x4*>(out + r * ldo + c) = y;
 }
 
 // out = the mean of in.n tensors, four values a thread, summed in order
 __global__ __launch_bounds__(256) void mean_kernel(const HiftMean in, float* __restrict__ out, int C,
-                                                   uint32_t* __restrict__ amax,
                                                    const HiftDocs* __restrict__ docs) {
-  const int q = C / 4;
-  const long first = (long)blockIdx.x * blockDim.x, total = (long)docs->b[docs->n] * q;
-  if (first >= total) return;
-  const long i = first + threadIdx.x;
-  float m = 0.0f;
-  if (i < total) {
-    f32x4 v = reinterpret_cast<const f32x4*>(in.x[0])[i];
-    for (int k = 1; k < in.n; ++k) v += reinterpret_cast<const f32x4*>(in.x[k])[i];
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long)docs->b[docs->n] * (C / 4)) return;
+  f32x4 v = reinterpret_cast<const f32x4*>(in.x[0])[i];
+  for (int k = 1; k < in.n; ++k) v += reinterpret_cast<const f32x4*>(in.x[k])[i];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] = v[e] / (float)in.n;
-      m = fmaxf(m, finite_abs(v[e]));
-    }
-    reinterpret_cast<f32x4*>(out)[i] = v;
-  }
-  raise_rows_amax(amax, m, first, i, total, q, docs);
+  for (int e = 0; e < 4; ++e) v[e] = v[e] / (float)in.n;
+  reinterpret_cast<f32x4*>(out)[i] = v;
 }
 
 // One layer of the fp64 F0 predictor on v_mfma_f64_16x16x4: out[r][co] = elu(b[co] + sum_k W[co][k]
@@ -653,7 +577,6 @@ hipError_t launch_conv(const HiftConv& p_in, hipStream_t stream) {
            (!p.n_snakes || (aligned16(p.snakes[0].out) && aligned16(p.snakes[0].alpha) &&
                             aligned16(p.snakes[0].inv_alpha)));
   if (p.n_snakes > 1 || !p.docs) return hipErrorInvalidValue;
-  if (!p.n_snakes) p.snakes[0].amax = nullptr;
   // 64x64 tiles, or 32x32 where 64x64 tiles would not give every CU one (the grid covers the
   // capacity, so a captured call and its replays use the same size; results do not depend on it).
   // FCV_HIFT_TILE=32 or 64 forces one size: a test hook, since both must give the same bits.
@@ -683,21 +606,21 @@ hipError_t hift_conv_f32(const HiftConv& p, hipStream_t stream) {
 }
 
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
-                      const float* alpha, const float* inv_alpha, uint32_t* amax,
-                      const HiftDocs* docs, hipStream_t stream) {
+                      const float* alpha, const float* inv_alpha, const HiftDocs* docs,
+                      hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   const long n = (long)rows * (C / 4);
   hipLaunchKernelGGL(snake_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, x, ldx, out,
-                     ldo, C, alpha, inv_alpha, amax, docs);
+                     ldo, C, alpha, inv_alpha, docs);
   return hipGetLastError();
 }
 
-hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* amax,
-                     const HiftDocs* docs, hipStream_t stream) {
+hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, const HiftDocs* docs,
+                     hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   if (in.n < 1 || in.n > 4 || C % 4 != 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(mean_kernel, dim3(blocks_for((long)rows * (C / 4), 256)), dim3(256), 0, stream,
-                     in, out, C, amax, docs);
+                     in, out, C, docs);
   return hipGetLastError();
 }
 

@@ -26,9 +26,6 @@ struct HiftDocs {
 enum { HIFT_PRO_NONE = 0, HIFT_PRO_LEAKY = 1 };
 enum { HIFT_ACC_WRITE = 0, HIFT_ACC_ADD = 1, HIFT_ACC_ADD_DIV = 2 };
 
-// Largest magnitude of a tensor per document: kAmaxWords words per document (see hift_device.hpp).
-constexpr int kAmaxSub = 16, kAmaxStride = 16, kAmaxWords = kAmaxSub * kAmaxStride;
-
 // One 1-D convolution as an implicit GEMM: out[r][co] over output rows r of every document.
 // Input position of tap j for output position p of a document:
 //   u = p * stride + j * dil - pad;  q = up > 1 ? (u >= 0 ? u / up : -1) : u
@@ -46,19 +43,15 @@ struct HiftConv {
   const float* alpha; const float* inv_alpha;    // snake_out: out = snake(y)
   int snake_out;
   void* out; int ldo;
-  // further outputs snake_i(y), for the convolutions that read them (n_snakes <= kHiftSnakes; more
-  // than one in the split form only); amax: see amax_out
+  // further outputs snake_i(y), for the convolutions that read them (n_snakes <= 4; more than one in
+  // the split form only)
   int n_snakes;
-  struct Snake { float* out; const float* alpha; const float* inv_alpha; uint32_t* amax; };
+  struct Snake { float* out; const float* alpha; const float* inv_alpha; };
   Snake snakes[4];
   int vec4;                                // set by the launch: 16-byte epilogue accesses
   // split f16 form (hift_conv_split): packed weights of co_pad channels, their inverse scales and
-  // biases ([co_pad] each, one after the other);
-  // the largest finite |input| per document (fp32 bits)
+  // biases ([co_pad] each, one after the other)
   const void* wsplit; const float* winv; int co_pad;
-  const uint32_t* amax_in;
-  // per document, raised to the largest finite magnitude written to out (optional)
-  uint32_t* amax_out;
   const HiftDocs* docs;                    // the layout
 };
 
@@ -83,19 +76,18 @@ hipError_t hift_conv_split(const HiftConv* convs, int n, hipStream_t stream);
 size_t hift_split_bytes(int co_pad, int k, int cin);
 hipError_t hift_pack_split(const float* w, const float* bias, int cout, int co_pad, int k, int cin,
                            void* dst, float* inv, hipStream_t stream);
-hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream);
 
 // out[r][c] = snake(x[r][c]) for the live rows docs->b[docs->n] (grid: `rows`) x C channels
-// (C % 4 == 0), row strides ldx / ldo; amax (optional): see HiftConv::amax_out
+// (C % 4 == 0), row strides ldx / ldo
 hipError_t hift_snake(const float* x, int ldx, float* out, int ldo, int rows, int C,
-                      const float* alpha, const float* inv_alpha, uint32_t* amax,
-                      const HiftDocs* docs, hipStream_t stream);
+                      const float* alpha, const float* inv_alpha, const HiftDocs* docs,
+                      hipStream_t stream);
 
 // out[i] = (((x_0[i] + x_1[i]) + ...) / n over the live rows docs->b[docs->n] (grid: `rows`) x C
-// values (C % 4 == 0), n <= 4; amax: see HiftConv::amax_out
+// values (C % 4 == 0), n <= 4
 struct HiftMean { const float* x[4]; int n; };
-hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, uint32_t* amax,
-                     const HiftDocs* docs, hipStream_t stream);
+hipError_t hift_mean(const HiftMean& in, float* out, int rows, int C, const HiftDocs* docs,
+                     hipStream_t stream);
 
 // f0[r] = (float)|cls_w . h[r] + cls_b| (fp64 dot over C channels), one wave per live row
 // docs->b[docs->n] (grid: `rows`)

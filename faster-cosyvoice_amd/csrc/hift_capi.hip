@@ -149,11 +149,10 @@ struct Capacity {
   int frames, docs;
   int spec, samples, src;              // STFT frames, output samples, source samples
   std::vector<int> stage, stage_w;     // upsampling-conv rows and written rows per stage
-  size_t h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, y, fr, amax, tables, total;
+  size_t h64a, h64b, f0buf, sines, srcbuf, specbuf, xa, xn, xs, y, fr, tables, total;
   size_t si[2];                        // source branches of this stage and the next
   bool together;                       // a stage's resblocks run together (see run)
   size_t r[fcv::kHiftJobs], t1[fcv::kHiftJobs], s1[fcv::kHiftJobs];  // one set per resblock in flight
-  int amax_slots;                      // per document: one per tensor a split convolution reads
 };
 
 // Tables of one call, in launch order (see run): their count for n_stages stages.
@@ -196,8 +195,6 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
   }
   C.y = take(sizeof(float) * C.spec * kSpecLd);
   C.fr = take(sizeof(float) * C.spec * kFrameLd);
-  C.amax_slots = 1 + d.n_stages * (1 + 2 * d.n_dilations * (1 + d.n_kernels));
-  C.amax = take(sizeof(uint32_t) * fcv::kAmaxWords * C.amax_slots * docs);
   C.tables = take(sizeof(HiftDocs) * table_count(d));
   C.total = off;
   return C;
@@ -301,33 +298,23 @@ HiftConv conv_base(const void* x, int ldx, int cout, int cin_pad, int k, void* o
   return p;
 }
 
-// The convolutions of one call.  Where the handle has split weights for a convolution it runs on
-// the f16 matrix cores, scaled by the largest input its producer recorded in a slot of the
-// workspace (one per tensor, `docs` values each, zeroed at the start of the call).
+// The convolutions of one call: on the f16 matrix cores where the handle has split weights for one.
 struct Convs {
   const FcvHift* h;
-  uint32_t* amax;
-  int docs_cap, slots, used = 0;
   hipStream_t st;
 
-  // a slot for a tensor that a split convolution will read (null: the handle has no split weights)
-  uint32_t* slot() {
-    if (!h->packed_base || used >= slots) return nullptr;
-    return amax + (size_t)docs_cap * fcv::kAmaxWords * used++;
-  }
-  // n independent convolutions: p[i] with weight index wi[i] (bias wi[i] + 1) and its input's slot
-  // in[i]; one launch where all of them have split weights
-  int run(HiftConv* p, const int* wi, const uint32_t* const* in, int n) const {
+  // n independent convolutions: p[i] with weight index wi[i] (bias wi[i] + 1); one launch where all of
+  // them have split weights
+  int run(HiftConv* p, const int* wi, int n) const {
     bool all = true;
     for (int i = 0; i < n; ++i) {
       p[i].w = h->w[wi[i]];
       p[i].bias = h->w[wi[i] + 1];
       const FcvHift::Packed& k = h->packed[wi[i]];
-      if (h->packed_base && k.w >= 0 && in[i]) {
+      if (h->packed_base && k.w >= 0) {
         p[i].wsplit = h->packed_base + k.w;
         p[i].winv = reinterpret_cast<const float*>(h->packed_base + k.inv);
         p[i].co_pad = k.co_pad;
-        p[i].amax_in = in[i];
       } else {
         all = false;
       }
@@ -340,16 +327,15 @@ struct Convs {
       FCV_HIP(p[i].wsplit ? fcv::hift_conv_split(p + i, 1, st) : fcv::hift_conv_f32(p[i], st));
     return FCV_OK;
   }
-  int run(HiftConv p, int wi, const uint32_t* in) const { return run(&p, &wi, &in, 1); }
+  int run(HiftConv p, int wi) const { return run(&p, &wi, 1); }
   const float* f32(int i) const { return static_cast<const float*>(h->w[i]); }
 };
 
 // One ResBlock (generator.py:110-116) on x (rows by `docs`, C channels): for each dilation j:
 // r = r + conv2(snake2(conv1(snake1(r)))); the last conv2 writes its result per `mode` (write /
-// accin + y / (accin + y) / div) into `out`, its magnitude into `amax_out` (optional).  `wi` is the
-// index of the block's 8 * D weights.  x is read as the first residual; r holds the running value.
-// s1 holds snake1(x) already, of magnitude a_s1, where `ready`.  `rows` is the capacity the grids
-// cover.
+// accin + y / (accin + y) / div) into `out`.  `wi` is the index of the block's 8 * D weights.  x is
+// read as the first residual; r holds the running value.  s1 holds snake1(x) already where `ready`.
+// `rows` is the capacity the grids cover.
 struct ResBlock {
   int wi, k;
   const int* dils;
@@ -357,49 +343,42 @@ struct ResBlock {
   const HiftDocs* docs;
   const float* x;
   float *r, *t1, *s1, *out;
-  uint32_t* a_s1;
   bool ready;
   int mode;
   const float* accin;
   float div;
-  uint32_t* amax_out;
 };
 
 // n resblocks that do not depend on each other, one convolution of each at a time
-int run_resblocks(Convs& cv, ResBlock* blocks, int n) {
+int run_resblocks(const Convs& cv, ResBlock* blocks, int n) {
   const int D = cv.h->d.n_dilations;
   // the longest first: its workgroups start first
   std::stable_sort(blocks, blocks + n, [](const ResBlock& a, const ResBlock& b) {
     return (long)a.k * a.rows * a.C * a.C > (long)b.k * b.rows * b.C * b.C;
   });
   for (int i = 0; i < n; ++i) {
-    ResBlock& b = blocks[i];
+    const ResBlock& b = blocks[i];
     if (b.ready) continue;
-    b.a_s1 = cv.slot();
     FCV_HIP(fcv::hift_snake(b.x, b.C, b.s1, b.C, b.rows, b.C, cv.f32(b.wi + 4), cv.f32(b.wi + 5),
-                            b.a_s1, b.docs, cv.st));
+                            b.docs, cv.st));
   }
   HiftConv c[fcv::kHiftJobs];
   int wi[fcv::kHiftJobs];
-  const uint32_t* in[fcv::kHiftJobs];
   for (int j = 0; j < D; ++j) {
     const bool last = j == D - 1;
     for (int i = 0; i < n; ++i) {
       const ResBlock& b = blocks[i];
       wi[i] = b.wi + 8 * j;
-      in[i] = b.a_s1;
       c[i] = conv_base(b.s1, b.C, b.C, b.C, b.k, b.t1, b.C, b.rows, b.docs);
       c[i].dil = b.dils[j];
       c[i].pad = causal_padding(b.k, b.dils[j]);
       c[i].snake_out = 1;
       c[i].alpha = cv.f32(wi[i] + 6);
       c[i].inv_alpha = cv.f32(wi[i] + 7);
-      c[i].amax_out = cv.slot();
     }
-    if (int rc = cv.run(c, wi, in, n)) return rc;
+    if (int rc = cv.run(c, wi, n)) return rc;
     for (int i = 0; i < n; ++i) {
-      ResBlock& b = blocks[i];
-      in[i] = c[i].amax_out;
+      const ResBlock& b = blocks[i];
       wi[i] += 2;
       c[i] = conv_base(b.t1, b.C, b.C, b.C, b.k, last ? b.out : b.r, b.C, b.rows, b.docs);
       c[i].pad = causal_padding(b.k, 1);
@@ -409,15 +388,12 @@ int run_resblocks(Convs& cv, ResBlock* blocks, int n) {
         c[i].mode = b.mode;
         c[i].accin = b.accin;
         c[i].div = b.div;
-        c[i].amax_out = b.amax_out;
       } else {
-        b.a_s1 = cv.slot();
         c[i].n_snakes = 1;
-        c[i].snakes[0] = {b.s1, cv.f32(b.wi + 8 * (j + 1) + 4), cv.f32(b.wi + 8 * (j + 1) + 5),
-                          b.a_s1};
+        c[i].snakes[0] = {b.s1, cv.f32(b.wi + 8 * (j + 1) + 4), cv.f32(b.wi + 8 * (j + 1) + 5)};
       }
     }
-    if (int rc = cv.run(c, wi, in, n)) return rc;
+    if (int rc = cv.run(c, wi, n)) return rc;
   }
   return FCV_OK;
 }
@@ -482,14 +458,11 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- conv_pre (lookahead on the right) -------------------------------------------------
   float* xp = F32(C.xa);
   float* xn = F32(C.xn);
-  Convs cv{h, reinterpret_cast<uint32_t*>(ws + C.amax), C.docs, C.amax_slots, 0, st};
-  if (h->packed_base) FCV_HIP(fcv::hift_zero_u32(cv.amax, C.amax_slots * C.docs * fcv::kAmaxWords, st));
-  uint32_t* a_xp = cv.slot();  // magnitude of xp
+  const Convs cv{h, st};
   {
     HiftConv c = conv_base(mel, d.in_channels, d.base_channels, d.in_channels,
                            d.conv_pre_look_right + 1, xp, d.base_channels, C.frames, T + 4);
-    c.amax_out = a_xp;
-    if (int rc = cv.run(c, h->i_pre, nullptr)) return rc;
+    if (int rc = cv.run(c, h->i_pre)) return rc;
   }
 
   // ---- upsampling stages -----------------------------------------------------------------
@@ -504,14 +477,14 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
     float* si = F32(C.si[s & 1]);
     *b = ResBlock{h->i_srb + rb_size * s, d.source_kernels[s], d.source_dilations[s], Cs,
                   C.stage_w[s], T + 6 + 3 * s, si, F32(C.r[set]), F32(C.t1[set]), F32(C.s1[set]),
-                  si, cv.slot(), true, fcv::HIFT_ACC_WRITE, nullptr, 1.0f, nullptr};
+                  si, true, fcv::HIFT_ACC_WRITE, nullptr, 1.0f};
     HiftConv c = conv_base(F32(C.specbuf), kSpecLd, Cs, kSpecLd, kd.first, si, Cs, C.stage_w[s],
                            T + 5 + 3 * s);
     c.stride = kd.second;
     c.pad = kd.second - 1;
     c.n_snakes = 1;
-    c.snakes[0] = {b->s1, cv.f32(b->wi + 4), cv.f32(b->wi + 5), b->a_s1};
-    return cv.run(c, h->i_down + 2 * s, nullptr);
+    c.snakes[0] = {b->s1, cv.f32(b->wi + 4), cv.f32(b->wi + 5)};
+    return cv.run(c, h->i_down + 2 * s);
   };
   for (int s = 0; s < S; ++s) {
     const int Cs = stage_channels(d, s);
@@ -525,8 +498,7 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
     for (int j = 0; j < K; ++j)
       b[j] = ResBlock{h->i_rb + rb_size * (s * K + j), d.resblock_kernels[j],
                       d.resblock_dilations[j], Cs, nrows, t_w, xn, F32(C.r[j]), F32(C.t1[j]),
-                      F32(C.s1[j]), F32(C.r[j]), nullptr, false, fcv::HIFT_ACC_WRITE, nullptr, 1.0f,
-                      nullptr};
+                      F32(C.s1[j]), F32(C.r[j]), false, fcv::HIFT_ACC_WRITE, nullptr, 1.0f};
     // upsampling conv on LeakyReLU(x), plus the source branch (and, for resblocks that run
     // together, their first Snakes)
     {
@@ -543,15 +515,13 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
       if (C.together && h->packed_base && h->packed[wi].w >= 0) {
         c.n_snakes = K;
         for (int j = 0; j < K; ++j) {
-          b[j].a_s1 = cv.slot();
           b[j].ready = true;
-          c.snakes[j] = {b[j].s1, cv.f32(b[j].wi + 4), cv.f32(b[j].wi + 5), b[j].a_s1};
+          c.snakes[j] = {b[j].s1, cv.f32(b[j].wi + 4), cv.f32(b[j].wi + 5)};
         }
       }
-      if (int rc = cv.run(c, wi, a_xp)) return rc;
+      if (int rc = cv.run(c, wi)) return rc;
     }
     // mean of the resblocks
-    a_xp = cv.slot();
     if (C.together) {
       fcv::HiftMean mean{};
       mean.n = K;
@@ -562,7 +532,7 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
         ++n;
       }
       if (int rc = run_resblocks(cv, b, n)) return rc;
-      FCV_HIP(fcv::hift_mean(mean, xn, nrows, Cs, a_xp, t_w, st));
+      FCV_HIP(fcv::hift_mean(mean, xn, nrows, Cs, t_w, st));
     } else {
       for (int j = 0; j < K; ++j) {
         ResBlock& q = b[j];
@@ -575,7 +545,6 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
           if (K > 1) q.mode = fcv::HIFT_ACC_ADD_DIV;
           q.div = (float)K;
           q.out = xn;
-          q.amax_out = a_xp;
         }
         if (int rc = run_resblocks(cv, &q, 1)) return rc;
       }
@@ -591,7 +560,7 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
     c.pad = causal_padding(7, 1);
     c.pro = fcv::HIFT_PRO_LEAKY;
     c.slope = 0.01f;
-    if (int rc = cv.run(c, h->i_post, a_xp)) return rc;
+    if (int rc = cv.run(c, h->i_post)) return rc;
   }
   FCV_HIP(fcv::hift_istft(F32(C.y), kSpecLd, window, F32(C.fr), speech, d.audio_limit, C.spec,
                           C.samples, T + 6 + 3 * S, st));
@@ -675,14 +644,12 @@ void plan_packed(FcvHift* h) {
   const FcvHiftDims& d = h->d;
   h->packed.assign(h->w.size(), FcvHift::Packed{});
   size_t off = 0;
-  auto add = [&](int wi, int cout, int cin, int k, int dil, int up, float slope) {
+  auto add = [&](int wi, int cout, int cin, int k, int dil, int up) {
     HiftConv p = conv_base(nullptr, 0, cout, cin, k, nullptr, 0, 0, nullptr);
     p.dil = dil;
     p.up = up;
     p.pad = causal_padding(k, dil);
     if (up > 1) p.pad = k - 1;
-    p.pro = fcv::HIFT_PRO_LEAKY;
-    p.slope = slope;
     if (!fcv::hift_split_eligible(p)) return;
     FcvHift::Packed& e = h->packed[wi];
     e.co_pad = (cout + 63) / 64 * 64;
@@ -693,22 +660,22 @@ void plan_packed(FcvHift* h) {
   };
   auto resblock = [&](int wi, int C, int k, const int* dils) {
     for (int j = 0; j < d.n_dilations; ++j) {
-      add(wi + 8 * j, C, C, k, dils[j], 1, 0.0f);
-      add(wi + 8 * j + 2, C, C, k, 1, 1, 0.0f);
+      add(wi + 8 * j, C, C, k, dils[j], 1);
+      add(wi + 8 * j + 2, C, C, k, 1, 1);
     }
   };
   const int rb = 8 * d.n_dilations;
   int cprev = d.base_channels;
   for (int s = 0; s < d.n_stages; ++s) {
     const int C = stage_channels(d, s);
-    add(h->i_ups + 2 * s, C, cprev, d.upsample_kernels[s], 1, d.upsample_rates[s], d.lrelu_slope);
+    add(h->i_ups + 2 * s, C, cprev, d.upsample_kernels[s], 1, d.upsample_rates[s]);
     resblock(h->i_srb + rb * s, C, d.source_kernels[s], d.source_dilations[s]);
     for (int j = 0; j < d.n_kernels; ++j)
       resblock(h->i_rb + rb * (s * d.n_kernels + j), C, d.resblock_kernels[j],
                d.resblock_dilations[j]);
     cprev = C;
   }
-  add(h->i_post, d.n_fft + 2, cprev, 7, 1, 1, 0.01f);
+  add(h->i_post, d.n_fft + 2, cprev, 7, 1, 1);
   h->packed_bytes = off;
 }
 

@@ -24,35 +24,5 @@ __device__ __forceinline__ float snake(float x, float a, float inv) {
   return fmaf(inv, s * s, x);
 }
 
-// |v|, or 0 where v is infinite or NaN: a tensor's scale is that of its finite values
-__device__ __forceinline__ float finite_abs(float v) {
-  const float a = fabsf(v);
-  return a <= 3.402823466e38f ? a : 0.0f;
-}
-
-// A tensor's largest finite magnitude per document is kept as the maximum of kAmaxSub values (fp32
-// bits, which order like integers), kAmaxStride words apart: the workgroups of a launch raise
-// different ones, since atomics on one address run one after the other (some 25 ns each: a
-// Snake pass over 8 k rows took 53 us against 5 with one value).
-__device__ __forceinline__ uint32_t* amax_word(uint32_t* amax, int doc, int sub) {
-  return amax + ((long)doc * kAmaxSub + (sub & (kAmaxSub - 1))) * kAmaxStride;
-}
-__device__ __forceinline__ void raise_amax(uint32_t* amax, int doc, int sub, float v) {
-  if (v > 0.0f) atomicMax(amax_word(amax, doc, sub), __float_as_uint(v));
-}
-// the maximum over the wave, valid in every lane
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp_f<0xB1>(v));
-  v = fmaxf(v, dpp_f<0x4E>(v));
-  v = fmaxf(v, dpp_f<0x141>(v));
-  v = fmaxf(v, dpp_f<0x140>(v));
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
-}
-
 }  // namespace
 }  // namespace fcv

@@ -1,26 +1,27 @@
 // The HiFT vocoder's causal fp32 convolutions on the f16 matrix cores, at fp32 accuracy.
 //
-// Every operand is held as a sum of two f16 values, x = hi + lo (22 significant bits), scaled by a
-// power of two so that the largest magnitude lies in [2^14, 2^15): a weight row by its own
-// largest weight (once, when the weights are packed), an input row by the largest finite input of
-// its document (recorded by the kernel that wrote it).  Values down to 2^-28 of the largest then
-// keep all 22 bits and smaller ones an absolute error of 2^-39 of it.  A product is
-// lo hi + hi lo + hi hi on v_mfma_f32_32x32x16_f16 with fp32 accumulators; the scales are powers
-// of two, taken out exactly in the epilogue.  Against 64-bit results the operands' rounding adds
-// 1.7e-6 to the waveform's relative error, under a tenth of what fp32 accumulation over K =
-// 192..8192 terms leaves (2.0e-5 with v_mfma_f32_16x16x4_f32), and the 16-deep f16 form rounds
-// the accumulator less often.
+// Every operand is held as a sum of two f16 values, x = hi + lo, scaled by a power of two so that the
+// largest finite magnitude lies in [2^14, 2^15): a weight row by its own largest weight (once, when
+// the weights are packed), the inputs by the largest of the 32 channels of one row that a chunk
+// takes.  Values down to 2^-17 of the largest keep 22 significant bits, smaller ones an absolute error
+// of 2^-39 of it.  A product is lo hi + hi lo + hi hi on v_mfma_f32_32x32x16_f16; a step's sum (32
+// channels of one tap) starts from zero, and is taken back to the row's scale as it is added to the
+// fp32 running sum.  So an output depends on the inputs it reads and on nothing else, as on the fp32
+// kernels: not on what else is in its document, later or louder, or on the tile.
+// Against 64-bit results the waveform's relative error is 9.4e-6 (8 requests) where
+// v_mfma_f32_16x16x4_f32 left 2.6e-5: the operands' rounding adds 1.7e-6, and sums of 16 products at a
+// time round less often than sums of 4.
 //
 // Bound: three f16 MFMAs do a product's work at 16 times the fp32 form's rate each, so the ceiling
 // is a third of the f16 peak against the fp32 peak of 157 TFLOP/s.  Measured on one MI355X against
-// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.5 ms (91 -> 197 TFLOP/s
-// of fp32 work over the whole call), one 68-frame chunk 2.30 -> 0.94 ms (with the small form below
-// and launches shared by independent convolutions), the error against 64 bits 2.4e-5 -> 1.0e-5.
+// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.7 ms (91 -> 193 TFLOP/s of
+// fp32 work over the whole call), one 68-frame chunk 2.31 -> 0.79 ms (with the small form below and
+// launches shared by independent convolutions).  One scale per document in place of one per row and
+// chunk was 10.2 and 0.79 ms, but took precision from every row quieter than the loudest.
 // What is left of a large launch is latency: the document table, window and residual reads around
 // 14 to 88 steps of MFMAs, and LDS reads (1.3 KB per MFMA in the 64x64 tile).  128x128 and 64x256
-// tiles (half the weight copies, twice the registers) were no faster: 10.7 and 10.8 against 10.4
-// ms; nor were weights loaded straight into registers, which needs no barrier between steps: 10.8
-// ms with 64x128 tiles.
+// tiles (half the weight copies, twice the registers) were no faster, nor were weights loaded straight
+// into registers, which needs no barrier between steps.
 //
 // A workgroup owns TR output rows x TC output channels.  For each 32 input channels it splits a
 // window of input rows (the tile's rows and the left context) into LDS once, then walks the taps
@@ -42,8 +43,8 @@ namespace {
 constexpr int kRowBytes = 128;  // one row of 32 channels: 4 chunks of hi, 4 of lo, 16 bytes each
 constexpr int kMaxHalo = 62;    // largest left context of a tile, in rows
 // 64x64 tiles in a launch (all its convolutions) under which the small form runs.  One call, all
-// small against all 64x64: 24 frames 0.81 and 1.52 ms, 68 0.99 and 1.49, 100 1.19 and 1.53, 200
-// 1.80 and 1.77, 286 2.35 and 1.98; by this rule 1.08, 0.95, 1.11, 1.41 and 1.74.
+// small against all 64x64: 24 frames 0.68 and 1.19 ms, 68 0.88 and 1.21, 100 1.06 and 1.23, 200
+// 1.69 and 1.52, 286 2.30 and 1.71; by this rule 0.75, 0.80, 0.96, 1.33 and 1.59.
 constexpr long kSmallBelow = 256;
 
 // position of 16-byte chunk `chunk` in LDS row `row`: 16 consecutive rows read at one chunk index
@@ -61,40 +62,51 @@ __device__ __forceinline__ void wait_lgkm0() {
   __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x3 << 14));
 }
 
-// 2^e as a float exponent field: the scale that brings `amax` into [2^14, 2^15) (1 for an
-// all-zero tensor; tiny tensors are raised by at most 2^100), and its inverse
-__device__ __forceinline__ int scale_field(uint32_t amax_bits) {
-  const int e = (int)(amax_bits >> 23) & 255;
-  return amax_bits == 0 ? 127 : min(max(268 - e, 14), 227);
+// |v| as its bits, which order like the values; 0 where v is infinite or NaN
+__device__ __forceinline__ uint32_t finite_bits(float v) {
+  const uint32_t a = __float_as_uint(v) & 0x7FFFFFFFu;
+  return a < 0x7F800000u ? a : 0u;
+}
+// The scale that brings the magnitude of bits `m` into [2^14, 2^15), as a float's exponent field (that
+// of 1 for zero; magnitudes below 2^-86 are raised by 2^100 only)
+__device__ __forceinline__ int scale_field(uint32_t m) {
+  return m == 0 ? 127 : min(max(268 - (int)(m >> 23), 14), 227);
 }
 __device__ __forceinline__ float field_to_float(int f) { return __uint_as_float((uint32_t)f << 23); }
 
-// a document's largest magnitude (fp32 bits) over its kAmaxSub words: by the whole wave, by a lane
-__device__ __forceinline__ uint32_t doc_amax(const uint32_t* amax, int d, int lane) {
-  const uint32_t v = amax[((long)d * kAmaxSub + (lane & (kAmaxSub - 1))) * kAmaxStride];
-  return __float_as_uint(wave_max(__uint_as_float(v)));
+// scale of four values and those of the other seven lanes of an aligned group of eight
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, true));
 }
-__device__ __forceinline__ uint32_t amax_serial(const uint32_t* amax, int d) {
-  uint32_t m = 0;
-  for (int i = 0; i < kAmaxSub; ++i) m = max(m, amax[((long)d * kAmaxSub + i) * kAmaxStride]);
-  return m;
+__device__ __forceinline__ int scale_field8(const f32x4& v) {
+  uint32_t m = max(max(finite_bits(v[0]), finite_bits(v[1])),
+                   max(finite_bits(v[2]), finite_bits(v[3])));
+  m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
+  m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
+  m = dpp_max<0x141>(m);  // row_half_mirror
+  return scale_field(m);
 }
+// A step's sum times this is in units of the weights' scale over 2^15 (kUnscale), in which the weights
+// are below 1: the running sum overflows no earlier than the inputs times their number
+constexpr float kUnscale = 32768.0f;
+__device__ __forceinline__ float step_scale(int field) { return field_to_float(254 - 15 - field); }
 
 // An output's sum is taken over groups of consecutive chunks, each from zero, the groups added in
 // order: at most kGroups of group_chunks(chunks).  A small launch gives each group a wave.
 constexpr int kGroups = 4;
 __device__ __forceinline__ int group_chunks(int chunks) { return (chunks + kGroups - 1) / kGroups; }
 
-// four values, scaled, as their f16 halves
+// Four values, scaled, as their f16 halves.  A value that is not finite goes into lo alone: beside an
+// infinite hi, the other operand's lo, zero or of the other sign, would make NaN of its products.
 __device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4& lo) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float x = v[e] * s;
     const f16 h = (f16)x;
-    const float r = x - (float)h;
-    hi[e] = h;
-    // an infinite value has no remainder (inf - inf); NaN stays in hi
-    lo[e] = (f16)(fabsf(x) <= 3.402823466e38f ? r : 0.0f);
+    const bool finite = fabsf(x) <= 3.402823466e38f;
+    hi[e] = finite ? h : (f16)0.0f;
+    lo[e] = (f16)(finite ? x - (float)h : x);
   }
 }
 
@@ -128,14 +140,12 @@ struct SplitAdds {
   }
 };
 
-// the epilogue of channels c .. c + 3 of one row: unscale, bias, residual, resblock sum, Snakes; m1, m2:
-// raised to the largest finite magnitudes written to out and to each Snake output
+// the epilogue of channels c .. c + 3 of one row: unscale, bias, residual, resblock sum, Snakes
 __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& cols,
-                                            const SplitAdds& in, long row, int c, const f32x4& acc,
-                                            float inv, float& m1, float (&m2)[4]) {
+                                            const SplitAdds& in, long row, int c, const f32x4& acc) {
   f32x4 v;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = fmaf(acc[e] * inv, cols.winv[e], cols.bias[e]);
+  for (int e = 0; e < 4; ++e) v[e] = fmaf(acc[e] * cols.winv[e], kUnscale, cols.bias[e]);
   const long i = row * p.ldo + c;
   if (p.add) {
 #pragma unroll
@@ -153,17 +163,11 @@ __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& 
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = snake(v[e], cols.alpha[e], cols.inv_alpha[e]);
   }
-  if (p.amax_out) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) m1 = fmaxf(m1, finite_abs(v[e]));
-  }
   *reinterpret_cast<f32x4*>(static_cast<float*>(p.out) + i) = v;
   if (p.n_snakes) {
     f32x4 w;
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = snake(v[e], cols.alpha2[e], cols.inv_alpha2[e]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) m2[0] = fmaxf(m2[0], finite_abs(w[e]));
     *reinterpret_cast<f32x4*>(p.snakes[0].out + i) = w;
 #pragma unroll
     for (int n = 1; n < 4; ++n) {
@@ -171,8 +175,6 @@ __device__ __forceinline__ void split_store(const HiftConv& p, const SplitCols& 
       const f32x4 a = load4(p.snakes[n].alpha, c), ia = load4(p.snakes[n].inv_alpha, c);
 #pragma unroll
       for (int e = 0; e < 4; ++e) w[e] = snake(v[e], a[e], ia[e]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) m2[n] = fmaxf(m2[n], finite_abs(w[e]));
       *reinterpret_cast<f32x4*>(p.snakes[n].out + i) = w;
     }
   }
@@ -221,7 +223,8 @@ struct Cfg {
   static constexpr int kInfoOff = kXOff + (kWin + 1) * kRowBytes;  // + the zero row
   static constexpr int kPitch = 32 * MC + 4;                 // staged epilogue row, in floats
   static constexpr int kStage = 32 * kPitch * 4;             // per wave
-  static constexpr int kLds = kInfoOff + TR * 20;
+  static constexpr int kScaleOff = kInfoOff + TR * 16;
+  static constexpr int kLds = kScaleOff + (kWin + 1) * 4;
   static constexpr int kMinWaves = kThreads < 256 ? 1 : NI <= 3 ? 4 : 3;  // per SIMD
   static_assert(kWBytes % (1024 * kWaves) == 0, "weight copies");
   static_assert(kStage * kWaves <= kInfoOff, "the epilogue stages in the operand space");
@@ -235,9 +238,9 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   __shared__ __attribute__((aligned(1024))) char smem[C::kLds];
   char* sX = smem + C::kXOff;
   // per tile row: window row of the first tap (of input position 0 for up > 1), position and
-  // document; then the inverse input scale
+  // document; then each window row's step_scale
   int4* sInfo = reinterpret_cast<int4*>(smem + C::kInfoOff);
-  float* sInv = reinterpret_cast<float*>(smem + C::kInfoOff + C::TR * 16);
+  float* sScale = reinterpret_cast<float*>(smem + C::kScaleOff);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -274,38 +277,28 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   // the window starts at the first input row any tap of the tile's first row reads
   const int u0 = r0 - out0 - p.pad;
   const int win0 = in0 + (u0 > 0 ? u0 / p.up : 0);
-  // scale of the first document, which is that of every row of most tiles
-  const int f0 = scale_field(doc_amax(p.amax_in, d0, lane));
-  auto row_field = [&](int d) {
-    return d == d0 ? f0 : scale_field(amax_serial(p.amax_in, d));
-  };
   for (int t = tid; t < C::TR; t += C::kThreads) {
     const int r = r0 + t;
     int4 v{0, -(1 << 29), d0, 0};  // rows past the end read the zero row at every tap
-    float inv = 1.0f;
     if (r < rows_out) {
       const int d = one_doc ? d0 : doc_of(docs->b, n_docs, r);
       v.x = (one_doc ? in0 : docs->a[d]) - win0;
       v.y = r - (one_doc ? out0 : docs->b[d]);
       v.z = d;
-      inv = field_to_float(254 - row_field(d));
     }
     sInfo[t] = v;
-    sInv[t] = inv;
   }
+  if (tid == 0) sScale[C::kWin] = 1.0f;
   if (tid < 8) *reinterpret_cast<f32x4*>(sX + C::kWin * kRowBytes + tid * 16) = f32x4{0, 0, 0, 0};
 
   // window loads: pass i, thread tid -> window row i * kThreads / 8 + tid / 8, channels 4 (tid % 8)
-  const float* X = static_cast<const float*>(p.x) + (tid & 7) * 4;
-  long xoff[C::NI];
-  float xs[C::NI];
+  const float* X = static_cast<const float*>(p.x) + (long)win0 * p.ldx + (tid & 7) * 4;
+  // (rows of a window past the tile's own may belong to another document: nothing reads them)
+  const float slope = p.pro == HIFT_PRO_LEAKY ? p.slope : 1.0f;  // (x 1 is x)
+  int xoff[C::NI];
 #pragma unroll
-  for (int i = 0; i < C::NI; ++i) {
-    const int row = min(win0 + i * (C::kThreads / 8) + (tid >> 3), in_total - 1);
-    xoff[i] = (long)row * p.ldx;
-    // (rows of a window past the tile's own may belong to another document: nothing reads them)
-    xs[i] = field_to_float(one_doc ? f0 : row_field(doc_of(docs->a, n_docs, row)));
-  }
+  for (int i = 0; i < C::NI; ++i)
+    xoff[i] = min(i * (C::kThreads / 8) + (tid >> 3), in_total - 1 - win0) * p.ldx;
   f32x4 xr[C::NI];
   auto fetch_x = [&](int c) {
 #pragma unroll
@@ -315,27 +308,27 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 #pragma unroll
     for (int i = 0; i < C::NI; ++i) {
       f32x4 v = xr[i];
-      if (p.pro == HIFT_PRO_LEAKY) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * p.slope;
-      }
+      for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * slope;
       f16x4 hi, lo;
-      split4(v, xs[i], hi, lo);
+      const int field = scale_field8(v);
+      split4(v, field_to_float(field), hi, lo);
       const int row = i * (C::kThreads / 8) + (tid >> 3);
+      if ((tid & 7) == 0) sScale[row] = step_scale(field);
       char* dst = sX + row * kRowBytes + (tid & 1) * 8;
       *reinterpret_cast<f16x4*>(dst + 16 * swz(row, (tid & 7) >> 1)) = hi;
       *reinterpret_cast<f16x4*>(dst + 16 * swz(row, 4 + ((tid & 7) >> 1))) = lo;
     }
   };
 
-  // the sum of the chunk group at hand, and of the groups before it
-  f32x16 acc[C::MC][C::MR], total[C::MC][C::MR];
+  // the step at hand, the sum of the chunk group at hand, and of the groups before it
+  f32x16 acc[C::MC][C::MR], group[C::MC][C::MR], total[C::MC][C::MR];
 #pragma unroll
   for (int a = 0; a < C::MC; ++a)
 #pragma unroll
     for (int b = 0; b < C::MR; ++b)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[a][b][e] = total[a][b][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) group[a][b][e] = total[a][b][e] = 0.0f;
   const int per_group = group_chunks(chunks);
   auto end_group = [&]() {
 #pragma unroll
@@ -344,8 +337,8 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       for (int b = 0; b < C::MR; ++b)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          total[a][b][e] = total[a][b][e] + acc[a][b][e];
-          acc[a][b][e] = 0.0f;
+          total[a][b][e] = total[a][b][e] + group[a][b][e];
+          group[a][b][e] = 0.0f;
         }
   };
 
@@ -391,12 +384,13 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       xl[buf][b] = *reinterpret_cast<const f16x8*>(sX + (xoff_l[b] ^ (32 * ks + 64)));
     }
   };
-  auto mma = [&](int buf) {
+  // a k-step's products, on the sums `from`
+  auto mma = [&](int buf, const f32x16 (&from)[C::MC][C::MR]) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int a = 0; a < C::MC; ++a)
 #pragma unroll
-      for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wl[buf][a], xh[buf][b], acc[a][b]);
+      for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wl[buf][a], xh[buf][b], from[a][b]);
 #pragma unroll
     for (int a = 0; a < C::MC; ++a)
 #pragma unroll
@@ -406,6 +400,24 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 #pragma unroll
       for (int b = 0; b < C::MR; ++b) acc[a][b] = mfma32(wh[buf][a], xh[buf][b], acc[a][b]);
     __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x16 zero[C::MC][C::MR];
+#pragma unroll
+  for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+    for (int b = 0; b < C::MR; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) zero[a][b][e] = 0.0f;
+  float scale[C::MR];  // of the step at hand
+  // a finished step joins its group
+  auto fold = [&]() {
+#pragma unroll
+    for (int a = 0; a < C::MC; ++a)
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          group[a][b][e] = fmaf(acc[a][b][e], scale[b], group[a][b][e]);
   };
 
   int s = 0, stage_s = 0, in_group = 0;
@@ -418,7 +430,8 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       // in flight, and the window is written right after it.
       wait_lgkm0();
       __syncthreads();
-      mma(1);
+      mma(1, acc);
+      fold();
       if (++in_group == per_group) {
         end_group();
         in_group = 0;
@@ -438,10 +451,12 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 
       const char* sW = smem + stage_s * C::kWBytes;
       stage_s = stage_s == C::NS - 1 ? 0 : stage_s + 1;
+      float next[C::MR];
 #pragma unroll
       for (int b = 0; b < C::MR; ++b) {
         const bool ok = q[b] >= 0 && (unsigned)wrow[b] < (unsigned)C::kWin;
         const int row = ok ? wrow[b] : C::kWin;
+        next[b] = sScale[row];
         xoff_l[b] = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
         // next tap's input row
         if (p.up > 1) {
@@ -456,12 +471,16 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
         }
       }
       load(0, 0, sW);
-      if (j > 0) mma(1);
+      if (j > 0) mma(1, acc);
       load(1, 1, sW);
-      mma(0);
+      if (j > 0) fold();
+      mma(0, zero);
+#pragma unroll
+      for (int b = 0; b < C::MR; ++b) scale[b] = next[b];
     }
   }
-  mma(1);
+  mma(1, acc);
+  fold();
   end_group();
   SplitCols cols;
   cols.load(p, live_c ? c4 : 0);
@@ -474,8 +493,6 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   // whole 128-byte (256-byte) runs of a row.
   float* stage = reinterpret_cast<float*>(smem + wave * C::kStage);
   constexpr int RPI = 64 / LPR, NP = 32 / RPI;  // rows a pass, passes
-  float m1 = 0.0f, m2[4] = {};                  // largest finite magnitudes written
-  const int sub = blockIdx.x + blockIdx.y;
 #pragma unroll
   for (int b = 0; b < C::MR; ++b) {
     const int t0 = (wr * C::MR + b) * 32 + lane / LPR;
@@ -504,47 +521,14 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       if (r >= rows_out || !live_c) continue;
       const f32x4 v = *reinterpret_cast<const f32x4*>(stage + (i * RPI + lane / LPR) * C::kPitch + cl);
       const int4 info = sInfo[t];
-      const float inv = sInv[t];
       const long row = p.reflect ? (long)r + info.z + 1 : r;
-      float a1 = 0.0f, a2[4] = {};
-      split_store(p, cols, in[i], row, c4, v, inv, a1, a2);
+      split_store(p, cols, in[i], row, c4, v);
       // reflection padding (1, 0): row 0 of the document repeats the result's row 1
       if (p.reflect && info.y == 1) {
         SplitAdds first;
         first.load(p, (long)r - 1 + info.z, c4);
-        split_store(p, cols, first, (long)r - 1 + info.z, c4, v, inv, a1, a2);
+        split_store(p, cols, first, (long)r - 1 + info.z, c4, v);
       }
-      if (one_doc) {
-        m1 = fmaxf(m1, a1);
-#pragma unroll
-        for (int n = 0; n < 4; ++n) m2[n] = fmaxf(m2[n], a2[n]);
-      } else {
-        if (p.amax_out) raise_amax(p.amax_out, info.z, sub, a1);
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-          if (n < p.n_snakes) raise_amax(p.snakes[n].amax, info.z, sub, a2[n]);
-      }
-    }
-  }
-  if (one_doc && (p.amax_out || p.n_snakes)) {
-    float* wmax = sInv;  // the row scales are read
-    m1 = wave_max(m1);
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      if (n < p.n_snakes) m2[n] = wave_max(m2[n]);
-    __syncthreads();
-    if (lane == 0) {
-      wmax[wave] = m1;
-#pragma unroll
-      for (int n = 0; n < 4; ++n) wmax[4 + 4 * n + wave] = m2[n];
-    }
-    __syncthreads();
-    if (tid <= p.n_snakes) {
-      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[tid - 1].amax;
-      float m = 0.0f;
-#pragma unroll
-      for (int w = 0; w < C::kWaves; ++w) m = fmaxf(m, wmax[tid * 4 + w]);
-      if (slot) raise_amax(slot, d0, sub, m);
     }
   }
 }
@@ -558,11 +542,12 @@ template <int NI, int PD>
 __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const HiftJobs jobs) {
   constexpr int kWin = NI * 8, kWinBytes = kWin * kRowBytes, kPitch = 36;
   constexpr int kStage = 32 * kPitch * 4;  // a group's 32x32 sums
-  constexpr int kPart = kWinBytes + kRowBytes > kStage ? kWinBytes + kRowBytes : kStage;
+  constexpr int kScaleOff = kWinBytes + kRowBytes;  // each window row's step_scale, the zero row's too
+  constexpr int kOperands = kScaleOff + (kWin + 4) * 4;
+  constexpr int kPart = kOperands > kStage ? kOperands : kStage;
   const HiftConv& p = jobs.c[blockIdx.z];
   const HiftDocs* __restrict__ docs = p.docs;
   __shared__ __attribute__((aligned(1024))) char smem[kGroups * kPart];
-  __shared__ float wmax[kGroups][5];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -576,13 +561,10 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
   const int per_group = group_chunks(chunks);
   const int c_begin = wave * per_group, c_end = min(c_begin + per_group, chunks);
   char* win = smem + wave * kPart;
+  float* scales = reinterpret_cast<float*>(win + kScaleOff);
 
   const int u0 = r0 - td.out0 - p.pad;
   const int win0 = td.in0 + (u0 > 0 ? u0 / p.up : 0);
-  const int f0 = scale_field(doc_amax(p.amax_in, td.d0, lane));
-  auto row_field = [&](int d) {
-    return d == td.d0 ? f0 : scale_field(amax_serial(p.amax_in, d));
-  };
 
   if (c_begin < c_end) {
     const char* wbase = static_cast<const char*>(p.wsplit) + (long)(co0 / 32) * 4096;
@@ -599,15 +581,11 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
     for (int i = 0; i < PD - 1; ++i) fetch_w(w[i], c_begin * k + i);
 
     // window pass i, lane l: row 8 i + l / 8, channels 4 (l % 8)
-    const float* X = static_cast<const float*>(p.x) + (lane & 7) * 4;
-    long xoff[NI];
-    float xs[NI];
+    const float* X = static_cast<const float*>(p.x) + (long)win0 * p.ldx + (lane & 7) * 4;
+    const float slope = p.pro == HIFT_PRO_LEAKY ? p.slope : 1.0f;  // (x 1 is x)
+    int xoff[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int row = min(win0 + i * 8 + (lane >> 3), td.in_total - 1);
-      xoff[i] = (long)row * p.ldx;
-      xs[i] = field_to_float(one_doc ? f0 : row_field(doc_of(docs->a, td.n_docs, row)));
-    }
+    for (int i = 0; i < NI; ++i) xoff[i] = min(i * 8 + (lane >> 3), td.in_total - 1 - win0) * p.ldx;
     f32x4 xr[NI];
     auto fetch_x = [&](int c) {
 #pragma unroll
@@ -617,13 +595,13 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         f32x4 v = xr[i];
-        if (p.pro == HIFT_PRO_LEAKY) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * p.slope;
-        }
+        for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * slope;
         f16x4 hi, lo;
-        split4(v, xs[i], hi, lo);
+        const int field = scale_field8(v);
+        split4(v, field_to_float(field), hi, lo);
         const int row = i * 8 + (lane >> 3);
+        if ((lane & 7) == 0) scales[row] = step_scale(field);
         char* dst = win + row * kRowBytes + (lane & 1) * 8;
         *reinterpret_cast<f16x4*>(dst + 16 * swz(row, (lane & 7) >> 1)) = hi;
         *reinterpret_cast<f16x4*>(dst + 16 * swz(row, 4 + ((lane & 7) >> 1))) = lo;
@@ -631,6 +609,7 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
     };
     fetch_x(c_begin);
     // the wave's zero row, and this lane's row: window row and input position of tap 0
+    if (lane == 0) scales[kWin] = 1.0f;
     if (lane < 8) *reinterpret_cast<f32x4*>(win + kWinBytes + lane * 16) = f32x4{0, 0, 0, 0};
     int q0 = -(1 << 29), rem0 = 0, wrow0 = 0;
     if (r0 + li < td.rows_out) {
@@ -646,9 +625,15 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
     stash_x();
     if (c_begin + 1 < c_end) fetch_x(c_begin + 1);
 
-    f32x16 acc;
+    // the group's sum; the last step's, which is folded behind the next one's MFMAs, and its scale
+    f32x16 group, done;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    for (int e = 0; e < 16; ++e) group[e] = done[e] = 0.0f;
+    float scale = 0.0f;
+    auto fold = [&]() {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) group[e] = fmaf(done[e], scale, group[e]);
+    };
     int q = q0, rem = rem0, wrow = wrow0, c = c_begin, j = 0;
     for (int s0 = c_begin * k; s0 < s_end; s0 += PD) {
 #pragma unroll
@@ -665,6 +650,7 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
         const bool ok = q >= 0 && (unsigned)wrow < (unsigned)kWin;
         const int row = ok ? wrow : kWin;
         const uint32_t off = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
+        const float next = scales[row];
         if (p.up > 1) {
           rem += 1;
           const int step = rem == p.up ? 1 : 0;
@@ -676,6 +662,9 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
           wrow += p.dil;
         }
         ++j;
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
           const f16x8 xh = *reinterpret_cast<const f16x8*>(win + (off ^ (32 * ks)));
@@ -684,13 +673,17 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
           acc = mfma32(w[u][2 * ks], xl, acc);
           acc = mfma32(w[u][2 * ks], xh, acc);
         }
+        fold();
+        done = acc;
+        scale = next;
       }
     }
+    fold();
     // the sums go where the window was: this wave has read it
     float* stage = reinterpret_cast<float*>(win);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const f32x4 v{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+      const f32x4 v{group[4 * g], group[4 * g + 1], group[4 * g + 2], group[4 * g + 3]};
       *reinterpret_cast<f32x4*>(stage + li * kPitch + g * 8 + hl * 4) = v;
     }
   }
@@ -712,50 +705,22 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
   }
   wait_lgkm0();
   __syncthreads();
-  float m1 = 0.0f, m2[4] = {};
-  const int sub = blockIdx.x + blockIdx.y;
-  if (live) {
-    f32x4 v{0, 0, 0, 0};
-    for (int g = 0; g * per_group < chunks; ++g)
-      v += *reinterpret_cast<const f32x4*>(smem + g * kPart + (t * kPitch + cl) * 4);
-    const float inv = field_to_float(254 - row_field(d));
-    split_store(p, cols, in, row, c4, v, inv, m1, m2);
-    // reflection padding (1, 0): row 0 of the document repeats the result's row 1
-    if (p.reflect && pos == 1) {
-      SplitAdds first;
-      first.load(p, (long)r - 1 + d, c4);
-      split_store(p, cols, first, (long)r - 1 + d, c4, v, inv, m1, m2);
-    }
-    if (!one_doc) {
-      if (p.amax_out) raise_amax(p.amax_out, d, sub, m1);
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-        if (n < p.n_snakes) raise_amax(p.snakes[n].amax, d, sub, m2[n]);
-    }
-  }
-  if (one_doc && (p.amax_out || p.n_snakes)) {
-    m1 = wave_max(m1);
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      if (n < p.n_snakes) m2[n] = wave_max(m2[n]);
-    if (lane == 0) {
-      wmax[wave][0] = m1;
-#pragma unroll
-      for (int n = 0; n < 4; ++n) wmax[wave][1 + n] = m2[n];
-    }
-    __syncthreads();
-    if (tid <= p.n_snakes) {
-      uint32_t* slot = tid == 0 ? p.amax_out : p.snakes[tid - 1].amax;
-      float m = 0.0f;
-#pragma unroll
-      for (int g = 0; g < kGroups; ++g) m = fmaxf(m, wmax[g][tid]);
-      if (slot) raise_amax(slot, td.d0, sub, m);
-    }
+  if (!live) return;
+  f32x4 v{0, 0, 0, 0};
+  for (int g = 0; g * per_group < chunks; ++g)
+    v += *reinterpret_cast<const f32x4*>(smem + g * kPart + (t * kPitch + cl) * 4);
+  split_store(p, cols, in, row, c4, v);
+  // reflection padding (1, 0): row 0 of the document repeats the result's row 1
+  if (p.reflect && pos == 1) {
+    SplitAdds first;
+    first.load(p, (long)r - 1 + d, c4);
+    split_store(p, cols, first, (long)r - 1 + d, c4, v);
   }
 }
 
 // One wave per output channel of [co_pad][k][cin] weights: the row's scale from its largest finite
-// weight, then both halves in the order the kernels' fragments take them; inv[co] = the inverse scale, inv[co_pad + co] = the bias (zero past cout).
+// weight, then both halves in the order the kernels' fragments take them; inv[co] = the inverse scale,
+// inv[co_pad + co] = the bias (zero past cout).
 __global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict__ w,
                                                         const float* __restrict__ bias, int cout,
                                                         int co_pad, int k, int cin,
@@ -764,11 +729,11 @@ __global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict_
   const int co = blockIdx.x, lane = threadIdx.x;
   const float* row = w + (long)co * k * cin;
   const int n = k * cin;
-  float m = 0.0f;
-  for (int i = lane; i < n; i += 64) m = fmaxf(m, finite_abs(row[i]));
+  uint32_t m = 0;
+  for (int i = lane; i < n; i += 64) m = max(m, finite_bits(row[i]));
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  const int f = scale_field(__float_as_uint(m));
+  for (int off = 32; off >= 1; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+  const int f = scale_field(m);
   const float s = field_to_float(f);
   if (lane == 0) {
     inv[co] = field_to_float(254 - f);
@@ -786,17 +751,11 @@ __global__ __launch_bounds__(64) void pack_split_kernel(const float* __restrict_
   }
 }
 
-__global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ x, int n) {
-  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i < n) *reinterpret_cast<uint4*>(x + i) = uint4{0, 0, 0, 0};
-}
-
 bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; }
 
 template <class C>
 hipError_t launch(const HiftJobs& jobs, int n, int rows, int cout, hipStream_t stream) {
   static_assert(C::kLds <= 160 * 1024, "LDS");
-  static_assert(C::TR >= 20, "the epilogue's maxima fit the row scales' place");
   const dim3 grid((rows + C::TR - 1) / C::TR, (cout + C::TC - 1) / C::TC, n);
   hipLaunchKernelGGL(split_conv_kernel<C>, grid, dim3(C::kThreads), 0, stream, jobs);
   return hipGetLastError();
@@ -836,14 +795,14 @@ hipError_t launch_small(const HiftJobs& jobs, int n, int rows, int cout, hipStre
 }
 
 bool launchable(const HiftConv& p) {
-  if (!hift_split_eligible(p) || !p.docs || !p.wsplit || !p.winv || !p.amax_in ||
+  if (!hift_split_eligible(p) || !p.docs || !p.wsplit || !p.winv ||
       p.co_pad % 64 != 0 || p.ldx % 4 != 0 || p.ldo % 4 != 0 || (p.add && p.ld_add % 4 != 0) ||
       !aligned16(p.x) || !aligned16(p.out) || !aligned16(p.add) || !aligned16(p.accin) ||
       !aligned16(p.wsplit) || !aligned16(p.winv) || (long)p.co_pad * kRowBytes >= (1L << 31) ||
       p.n_snakes < 0 || p.n_snakes > 4)
     return false;
   for (int i = 0; i < p.n_snakes; ++i)
-    if (!aligned16(p.snakes[i].out) || !p.snakes[i].amax) return false;
+    if (!aligned16(p.snakes[i].out)) return false;
   // channels go four at a time: a partial last group writes zeros into the row's padding and has
   // no other row or parameter to read
   return p.cout % 4 == 0 || ((p.cout + 3) / 4 * 4 <= p.ldo && !p.add && !p.snake_out &&
@@ -854,8 +813,7 @@ bool launchable(const HiftConv& p) {
 
 bool hift_split_eligible(const HiftConv& p) {
   return p.stride == 1 && p.cin_pad % 32 == 0 && p.up >= 1 && p.dil >= 1 &&
-         (p.up == 1 || p.dil == 1) && p.pad == (p.k - 1) * p.dil && p.pad <= kMaxHalo &&
-         (p.pro == HIFT_PRO_NONE || (p.slope >= -1.0f && p.slope <= 1.0f));
+         (p.up == 1 || p.dil == 1) && p.pad == (p.k - 1) * p.dil && p.pad <= kMaxHalo;
 }
 
 size_t hift_split_bytes(int co_pad, int k, int cin) {
@@ -866,13 +824,6 @@ hipError_t hift_pack_split(const float* w, const float* bias, int cout, int co_p
                            void* dst, float* inv, hipStream_t stream) {
   hipLaunchKernelGGL(pack_split_kernel, dim3(co_pad), dim3(64), 0, stream, w, bias, cout, co_pad, k,
                      cin, static_cast<f16*>(dst), inv);
-  return hipGetLastError();
-}
-
-hipError_t hift_zero_u32(uint32_t* x, int n, hipStream_t stream) {
-  if (n <= 0) return hipSuccess;
-  if (n % 4 != 0 || !aligned16(x)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3((n / 4 + 255) / 256), dim3(256), 0, stream, x, n);
   return hipGetLastError();
 }
 

@@ -79,7 +79,10 @@ int fcv_hift_destroy(FcvHift* hift);
 
 /* Split weights (optional): the causal unit-stride convolutions with input channels a multiple of
  * 32 then run on the f16 matrix cores at fp32 accuracy, both operands held as two f16 halves
- * (without them, and for the other convolutions, on the fp32 matrix cores).  fcv_hift_pack_weights
+ * (without them, and for the other convolutions, on the fp32 matrix cores).  The halves hold 22
+ * significant bits of values down to 2^-17 of the largest beside them, which are the 32 channels of a
+ * time step that a chunk takes, or an output channel's weights; an output depends on the inputs that
+ * its taps read and on no others, as on the fp32 matrix cores.  fcv_hift_pack_weights
  * computes them on `stream` into caller-owned memory of fcv_hift_packed_bytes (0: no such
  * convolution in this shape), 256-byte aligned, which must outlive the handle; it is called before
  * the handle's first inference.  fcv_hift_use_packed gives another handle over the same weights

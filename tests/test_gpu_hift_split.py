@@ -73,7 +73,7 @@ def test_split_matches_fp32(fcv, monkeypatch, frames, tile):
 
 @pytest.mark.parametrize("gain", [2.0 ** 24, 2.0 ** -40], ids=["large", "small"])
 def test_split_holds_the_fp32_range(fcv, monkeypatch, gain):
-    """Activations of 10^7 and 10^-12, past what f16 holds: the per-document scale keeps them."""
+    """Activations of 10^7 and 10^-12, past what f16 holds: the operands' scales keep them."""
     split, fp32 = _pair(fcv, monkeypatch, gain)
     g = torch.Generator().manual_seed(94)
     mels = [torch.randn(80, n, generator=g).cuda() for n in (20, 7)]
@@ -111,3 +111,43 @@ def test_concurrent_groups_repeat_bit_for_bit(fcv, monkeypatch):
     for _ in range(40):
         got = split.inference_batched(mels)
         assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+@pytest.mark.parametrize("channels", [slice(0, 80), slice(7, 8)], ids=["frame", "channel"])
+@pytest.mark.parametrize("loud", [1e6, 1e10, 1e20])
+def test_loud_frame_costs_the_others_no_precision(fcv, monkeypatch, loud, channels):
+    """One frame of large finite values: the audio before its right context reaches it (4 frames) is
+    bit for bit what it is without that frame, and the audio past the convolutions' reach (some 20
+    frames) matches the fp32 kernels as ever."""
+    split, fp32 = _pair(fcv, monkeypatch)
+    g = torch.Generator().manual_seed(97)
+    mel = torch.randn(80, 90, generator=g).cuda()
+    bad = mel.clone()
+    bad[channels, 20] *= loud
+    say(f"[split] one frame times {loud:.0e}")
+    quiet, = split.inference_batched([mel])
+    got, = split.inference_batched([bad])
+    ref, = fp32.inference_batched([bad])
+    before, after = (20 - 4 - 1) * 480, (20 + 35) * 480
+    assert torch.equal(got[:, :before], quiet[:, :before])
+    assert torch.isfinite(ref).all() and float(ref[:, after:].std()) > 1e-4
+    for part in (slice(0, before), slice(after, None)):
+        err = rel_l2(got[:, part], ref[:, part])
+        say(f"[split] rel_l2 {err:.2e}")
+        assert err <= 1e-4
+
+
+def test_output_before_a_change_stays_bit_for_bit(fcv, monkeypatch):
+    """A frame's audio depends on the frames its convolutions read, on none after them: what follows,
+    and how long the request is, leaves it bit for bit (a session re-vocodes its prefix)."""
+    split, _ = _pair(fcv, monkeypatch)
+    g = torch.Generator().manual_seed(98)
+    mel = torch.randn(80, 60, generator=g).cuda()
+    other = mel.clone()
+    other[:, 41:] *= 3.0
+    say("[split] prefix")
+    a, = split.inference_batched([mel])
+    b, = split.inference_batched([other])
+    c, = split.inference_batched([mel[:, :50]], [False])
+    keep = (41 - 4 - 1) * 480
+    assert torch.equal(a[:, :keep], b[:, :keep]) and torch.equal(a[:, :keep], c[:, :keep])
