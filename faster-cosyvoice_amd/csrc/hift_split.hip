@@ -14,10 +14,12 @@
 //
 // Bound: three f16 MFMAs do a product's work at 16 times the fp32 form's rate each, so the ceiling
 // is a third of the f16 peak against the fp32 peak of 157 TFLOP/s.  Measured on one MI355X against
-// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.7 ms (91 -> 193 TFLOP/s of
-// fp32 work over the whole call), one 68-frame chunk 2.31 -> 0.79 ms (with the small form below and
+// v_mfma_f32_16x16x4_f32 (hift.hip): 8 requests of 3065 frames 22.6 -> 10.2 ms (91 -> 202 TFLOP/s of
+// fp32 work over the whole call), one 68-frame chunk 2.31 -> 0.77 ms (with the small form below and
 // launches shared by independent convolutions).  One scale per document in place of one per row and
-// chunk was 10.2 and 0.79 ms, but took precision from every row quieter than the loudest.
+// chunk was 10.1 and 0.79 ms, but took precision from every row quieter than the loudest.  The large
+// form fits its 128 registers only just: seven spilled ones put a wait for every copy into its loop
+// (11.0 ms), so the tile's row table stays in LDS.
 // What is left of a large launch is latency: the document table, window and residual reads around
 // 14 to 88 steps of MFMAs, and LDS reads (1.3 KB per MFMA in the 64x64 tile).  128x128 and 64x256
 // tiles (half the weight copies, twice the registers) were no faster, nor were weights loaded straight
@@ -74,18 +76,16 @@ __device__ __forceinline__ int scale_field(uint32_t m) {
 }
 __device__ __forceinline__ float field_to_float(int f) { return __uint_as_float((uint32_t)f << 23); }
 
-// scale of four values and those of the other seven lanes of an aligned group of eight
+// the largest of four bit patterns and those of the other seven lanes of an aligned group of eight
 template <int kCtrl>
 __device__ __forceinline__ uint32_t dpp_max(uint32_t v) {
   return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, true));
 }
-__device__ __forceinline__ int scale_field8(const f32x4& v) {
-  uint32_t m = max(max(finite_bits(v[0]), finite_bits(v[1])),
-                   max(finite_bits(v[2]), finite_bits(v[3])));
-  m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
-  m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
-  m = dpp_max<0x141>(m);  // row_half_mirror
-  return scale_field(m);
+__device__ __forceinline__ uint32_t max_of8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  uint32_t m = max(max(a, b), max(c, d));
+  m = dpp_max<0xB1>(m);      // quad_perm [1, 0, 3, 2]
+  m = dpp_max<0x4E>(m);      // quad_perm [2, 3, 0, 1]
+  return dpp_max<0x141>(m);  // row_half_mirror
 }
 // A step's sum times this is in units of the weights' scale over 2^15 (kUnscale), in which the weights
 // are below 1: the running sum overflows no earlier than the inputs times their number
@@ -108,6 +108,29 @@ __device__ __forceinline__ void split4(const f32x4& v, float s, f16x4& hi, f16x4
     hi[e] = finite ? h : (f16)0.0f;
     lo[e] = (f16)(finite ? x - (float)h : x);
   }
+}
+
+// Splits four values of a window row, whose 32 channels eight lanes hold, and returns the row's scale
+// field.  Values that are not finite take the longer way, a wave at a time.
+__device__ __forceinline__ int split_row(const f32x4& v, f16x4& hi, f16x4& lo) {
+  constexpr uint32_t kAbs = 0x7FFFFFFFu;
+  const uint32_t m = max_of8(__float_as_uint(v[0]) & kAbs, __float_as_uint(v[1]) & kAbs,
+                             __float_as_uint(v[2]) & kAbs, __float_as_uint(v[3]) & kAbs);
+  if (__ballot(m >= 0x7F800000u) != 0) {
+    const int field = scale_field(max_of8(finite_bits(v[0]), finite_bits(v[1]), finite_bits(v[2]),
+                                          finite_bits(v[3])));
+    split4(v, field_to_float(field), hi, lo);
+    return field;
+  }
+  const int field = scale_field(m);
+  const float s = field_to_float(field);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x = v[e] * s;
+    hi[e] = (f16)x;
+    lo[e] = (f16)(x - (float)hi[e]);
+  }
+  return field;
 }
 
 __device__ __forceinline__ f32x4 load4(const void* q, long i) {
@@ -223,7 +246,8 @@ struct Cfg {
   static constexpr int kInfoOff = kXOff + (kWin + 1) * kRowBytes;  // + the zero row
   static constexpr int kPitch = 32 * MC + 4;                 // staged epilogue row, in floats
   static constexpr int kStage = 32 * kPitch * 4;             // per wave
-  static constexpr int kScaleOff = kInfoOff + TR * 16;
+  static constexpr int kRemOff = kInfoOff + TR * 16;
+  static constexpr int kScaleOff = kRemOff + TR * 4;
   static constexpr int kLds = kScaleOff + (kWin + 1) * 4;
   static constexpr int kMinWaves = kThreads < 256 ? 1 : NI <= 3 ? 4 : 3;  // per SIMD
   static_assert(kWBytes % (1024 * kWaves) == 0, "weight copies");
@@ -237,9 +261,11 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   const HiftDocs* __restrict__ docs = p.docs;
   __shared__ __attribute__((aligned(1024))) char smem[C::kLds];
   char* sX = smem + C::kXOff;
-  // per tile row: window row of the first tap (of input position 0 for up > 1), position and
-  // document; then each window row's step_scale
+  // per tile row: window row of tap 0, position, document and the window row of the document's first
+  // input row, before which a tap reads zeros; then tap 0's remainder (up > 1); then each window
+  // row's step_scale
   int4* sInfo = reinterpret_cast<int4*>(smem + C::kInfoOff);
+  int* sRem = reinterpret_cast<int*>(smem + C::kRemOff);
   float* sScale = reinterpret_cast<float*>(smem + C::kScaleOff);
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -255,16 +281,17 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   const int co0 = blockIdx.y * C::TC;
   if (co0 >= p.cout) return;
   const int chunks = p.cin_pad / 32;
-  const int k = p.k;
+  const int k = p.k, up = p.up, dil = p.dil;  // (read once: the copies below may write memory)
 
   // weight copies: step (chunk, tap) is a contiguous block of co_pad rows
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
-  const char* wbase = static_cast<const char*>(p.wsplit) + (long)co0 * kRowBytes;
+  const char* wnext = static_cast<const char*>(p.wsplit) + (long)co0 * kRowBytes;
   const long wstep = (long)p.co_pad * kRowBytes;
   const uint32_t wlane = (uint32_t)(wave * C::kCopies * 1024 + lane * 16);
   const int steps = chunks * k;
-  auto issue_w = [&](int s, int stage) {
-    const char* src = wbase + (long)s * wstep;
+  auto issue_w = [&](int stage) {
+    const char* src = wnext;
+    wnext += wstep;
     const uint32_t dst = lds0 + (uint32_t)stage * C::kWBytes + wave * C::kCopies * 1024;
 #pragma unroll
     for (int i = 0; i < C::kCopies; ++i) lds_dma16(src, wlane + i * 1024, dst + i * 1024);
@@ -272,37 +299,48 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 
 #pragma unroll
   for (int s = 0; s < C::NS - 1; ++s)
-    if (s < steps) issue_w(s, s);
+    if (s < steps) issue_w(s);
 
   // the window starts at the first input row any tap of the tile's first row reads
   const int u0 = r0 - out0 - p.pad;
-  const int win0 = in0 + (u0 > 0 ? u0 / p.up : 0);
+  const int win0 = in0 + (u0 > 0 ? u0 / up : 0);
   for (int t = tid; t < C::TR; t += C::kThreads) {
     const int r = r0 + t;
-    int4 v{0, -(1 << 29), d0, 0};  // rows past the end read the zero row at every tap
+    int4 v{-(1 << 29), -1, d0, 0};  // rows past the end read the zero row at every tap
+    int rem = 0;
     if (r < rows_out) {
       const int d = one_doc ? d0 : doc_of(docs->b, n_docs, r);
-      v.x = (one_doc ? in0 : docs->a[d]) - win0;
+      const int base = (one_doc ? in0 : docs->a[d]) - win0;
       v.y = r - (one_doc ? out0 : docs->b[d]);
       v.z = d;
+      v.w = max(base, 0);
+      int q = v.y - p.pad;
+      if (up > 1) {
+        const int u = q;
+        q = u >= 0 ? u / up : -((-u + up - 1) / up);
+        rem = u - q * up;
+      }
+      v.x = base + q;
     }
     sInfo[t] = v;
+    sRem[t] = rem;
   }
   if (tid == 0) sScale[C::kWin] = 1.0f;
   if (tid < 8) *reinterpret_cast<f32x4*>(sX + C::kWin * kRowBytes + tid * 16) = f32x4{0, 0, 0, 0};
 
   // window loads: pass i, thread tid -> window row i * kThreads / 8 + tid / 8, channels 4 (tid % 8)
-  const float* X = static_cast<const float*>(p.x) + (long)win0 * p.ldx + (tid & 7) * 4;
+  const char* X = reinterpret_cast<const char*>(static_cast<const float*>(p.x) + (long)win0 * p.ldx);
   // (rows of a window past the tile's own may belong to another document: nothing reads them)
   const float slope = p.pro == HIFT_PRO_LEAKY ? p.slope : 1.0f;  // (x 1 is x)
-  int xoff[C::NI];
+  uint32_t xoff[C::NI];  // bytes from the window's first row
 #pragma unroll
   for (int i = 0; i < C::NI; ++i)
-    xoff[i] = min(i * (C::kThreads / 8) + (tid >> 3), in_total - 1 - win0) * p.ldx;
+    xoff[i] = min(i * (C::kThreads / 8) + (tid >> 3), in_total - 1 - win0) * p.ldx * 4 +
+              (tid & 7) * 16;
   f32x4 xr[C::NI];
   auto fetch_x = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < C::NI; ++i) xr[i] = *reinterpret_cast<const f32x4*>(X + xoff[i] + c * 32);
+    for (int i = 0; i < C::NI; ++i) xr[i] = *reinterpret_cast<const f32x4*>(X + c * 128 + xoff[i]);
   };
   auto stash_x = [&]() {
 #pragma unroll
@@ -311,8 +349,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * slope;
       f16x4 hi, lo;
-      const int field = scale_field8(v);
-      split4(v, field_to_float(field), hi, lo);
+      const int field = split_row(v, hi, lo);
       const int row = i * (C::kThreads / 8) + (tid >> 3);
       if ((tid & 7) == 0) sScale[row] = step_scale(field);
       char* dst = sX + row * kRowBytes + (tid & 1) * 8;
@@ -343,27 +380,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   };
 
   fetch_x(0);
-  constexpr int LPR = 8 * C::MC;              // lanes per staged output row
-  const int cl = (lane % LPR) * 4;            // channel within the wave's columns
-  const int c4 = co0 + wc * C::MC * 32 + cl;
-  const bool live_c = c4 < p.cout;
   __syncthreads();  // the row table
-  // this lane's rows: window row and input position of tap 0; up > 1 walks (position, remainder)
-  int wrow0[C::MR], q0[C::MR], rem0[C::MR];
-#pragma unroll
-  for (int b = 0; b < C::MR; ++b) {
-    const int4 v = sInfo[(wr * C::MR + b) * 32 + li];
-    const int u = v.y - p.pad;
-    int q = u, rem = 0;
-    if (p.up > 1) {
-      q = u >= 0 ? u / p.up : -((-u + p.up - 1) / p.up);
-      rem = u - q * p.up;
-    }
-    q0[b] = q;
-    rem0[b] = rem;
-    wrow0[b] = v.x + q;
-  }
-
   // Two fragment buffers: the reads of k-step ks + 1 are in flight while the MFMAs of ks run.  A
   // step's second k-step runs after the barrier that publishes the next step, over that step's
   // first reads.  A weight block of 32 channels is 4 KB: k-steps 0 and 1, hi then lo, lane l's 16
@@ -422,9 +439,14 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
 
   int s = 0, stage_s = 0, in_group = 0;
   for (int c = 0; c < chunks; ++c) {
-    int q[C::MR], rem[C::MR], wrow[C::MR];
+    int wrow[C::MR], first[C::MR], rem[C::MR];  // this lane's rows
 #pragma unroll
-    for (int b = 0; b < C::MR; ++b) { q[b] = q0[b]; rem[b] = rem0[b]; wrow[b] = wrow0[b]; }
+    for (int b = 0; b < C::MR; ++b) {
+      const int t = (wr * C::MR + b) * 32 + li;
+      wrow[b] = sInfo[t].x;
+      first[b] = sInfo[t].w;
+      rem[b] = sRem[t];
+    }
     if (c > 0) {
       // Every wave has read the previous window: a barrier alone does not wait for a wave's reads
       // in flight, and the window is written right after it.
@@ -446,7 +468,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
         wait_vm<0>();
       wait_lgkm0();  // and this wave's reads of the stage the next copies overwrite
       __syncthreads();
-      if (s + C::NS - 1 < steps) issue_w(s + C::NS - 1, stage_s == 0 ? C::NS - 1 : stage_s - 1);
+      if (s + C::NS - 1 < steps) issue_w(stage_s == 0 ? C::NS - 1 : stage_s - 1);
       if (j == 0 && c + 1 < chunks) fetch_x(c + 1);
 
       const char* sW = smem + stage_s * C::kWBytes;
@@ -454,20 +476,17 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
       float next[C::MR];
 #pragma unroll
       for (int b = 0; b < C::MR; ++b) {
-        const bool ok = q[b] >= 0 && (unsigned)wrow[b] < (unsigned)C::kWin;
-        const int row = ok ? wrow[b] : C::kWin;
+        const int row = wrow[b] >= first[b] && wrow[b] < C::kWin ? wrow[b] : C::kWin;
         next[b] = sScale[row];
         xoff_l[b] = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
         // next tap's input row
-        if (p.up > 1) {
+        if (up > 1) {
           rem[b] += 1;
-          const int step = rem[b] == p.up ? 1 : 0;
+          const int step = rem[b] == up ? 1 : 0;
           rem[b] = step ? 0 : rem[b];
-          q[b] += step;
           wrow[b] += step;
         } else {
-          q[b] += p.dil;
-          wrow[b] += p.dil;
+          wrow[b] += dil;
         }
       }
       load(0, 0, sW);
@@ -482,6 +501,10 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWaves) void split_conv_kernel(
   mma(1, acc);
   fold();
   end_group();
+  constexpr int LPR = 8 * C::MC;              // lanes per staged output row
+  const int cl = (lane % LPR) * 4;            // channel within the wave's columns
+  const int c4 = co0 + wc * C::MC * 32 + cl;
+  const bool live_c = c4 < p.cout;
   SplitCols cols;
   cols.load(p, live_c ? c4 : 0);
   wait_vm<0>();
@@ -557,14 +580,14 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
   if (!td.load(docs, r0, lane)) return;
   if (co0 >= p.cout) return;
   const bool one_doc = min(r0 + 32, td.rows_out) <= td.out1;
-  const int chunks = p.cin_pad / 32, k = p.k;
+  const int chunks = p.cin_pad / 32, k = p.k, up = p.up, dil = p.dil;
   const int per_group = group_chunks(chunks);
   const int c_begin = wave * per_group, c_end = min(c_begin + per_group, chunks);
   char* win = smem + wave * kPart;
   float* scales = reinterpret_cast<float*>(win + kScaleOff);
 
   const int u0 = r0 - td.out0 - p.pad;
-  const int win0 = td.in0 + (u0 > 0 ? u0 / p.up : 0);
+  const int win0 = td.in0 + (u0 > 0 ? u0 / up : 0);
 
   if (c_begin < c_end) {
     const char* wbase = static_cast<const char*>(p.wsplit) + (long)(co0 / 32) * 4096;
@@ -598,8 +621,7 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.0f ? v[e] : v[e] * slope;
         f16x4 hi, lo;
-        const int field = scale_field8(v);
-        split4(v, field_to_float(field), hi, lo);
+        const int field = split_row(v, hi, lo);
         const int row = i * 8 + (lane >> 3);
         if ((lane & 7) == 0) scales[row] = step_scale(field);
         char* dst = win + row * kRowBytes + (lane & 1) * 8;
@@ -616,9 +638,9 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
       const int d = one_doc ? td.d0 : doc_of(docs->b, td.n_docs, r0 + li);
       const int u = r0 + li - (one_doc ? td.out0 : docs->b[d]) - p.pad;
       q0 = u;
-      if (p.up > 1) {
-        q0 = u >= 0 ? u / p.up : -((-u + p.up - 1) / p.up);
-        rem0 = u - q0 * p.up;
+      if (up > 1) {
+        q0 = u >= 0 ? u / up : -((-u + up - 1) / up);
+        rem0 = u - q0 * up;
       }
       wrow0 = (one_doc ? td.in0 : docs->a[d]) - win0 + q0;
     }
@@ -651,15 +673,15 @@ __global__ __launch_bounds__(64 * kGroups, 1) void split_conv_small_kernel(const
         const int row = ok ? wrow : kWin;
         const uint32_t off = row * kRowBytes + 16 * (hl ^ ((row >> 1) & 7));
         const float next = scales[row];
-        if (p.up > 1) {
+        if (up > 1) {
           rem += 1;
-          const int step = rem == p.up ? 1 : 0;
+          const int step = rem == up ? 1 : 0;
           rem = step ? 0 : rem;
           q += step;
           wrow += step;
         } else {
-          q += p.dil;
-          wrow += p.dil;
+          q += dil;
+          wrow += dil;
         }
         ++j;
         f32x16 acc;
