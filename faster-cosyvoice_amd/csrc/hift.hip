@@ -577,10 +577,11 @@ hipError_t launch_conv(const HiftConv& p_in, hipStream_t stream) {
            (!p.n_snakes || (aligned16(p.snakes[0].out) && aligned16(p.snakes[0].alpha) &&
                             aligned16(p.snakes[0].inv_alpha)));
   if (p.n_snakes > 1 || !p.docs) return hipErrorInvalidValue;
-  // 64x64 tiles, or 32x32 where 64x64 tiles would not give every CU one (the grid covers the
-  // capacity, so a captured call and its replays use the same size; results do not depend on it).
+  // 64x64 tiles, or 32x32 where 64x64 tiles would not give every CU one (results do not depend on
+  // it).
   // FCV_HIFT_TILE=32 or 64 forces one size: a test hook, since both must give the same bits.
-  const long tiles64 = (long)((p.rows_out + kTileR - 1) / kTileR) * ((p.cout + kTileC - 1) / kTileC);
+  const long tiles64 =
+      (long)((p.rows_live + kTileR - 1) / kTileR) * ((p.cout + kTileC - 1) / kTileC);
   const char* forced = std::getenv("FCV_HIFT_TILE");
   const int force = forced ? std::atoi(forced) : 0;
   if (force == 32 || (force != 64 && tiles64 < kSmallTileBelow)) {

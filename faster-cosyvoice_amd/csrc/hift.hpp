@@ -36,6 +36,7 @@ struct HiftConv {
   const void* w; const void* bias;
   int cout, cin_pad, k, stride, dil, pad, up;
   int rows_out;                            // capacity the grid covers (live: docs->b[docs->n])
+  int rows_live;                           // rows the launch's form is chosen by (no result is)
   int reflect;                             // write row p + 1 (row 0 = row 2 of the result)
   int pro; float slope;                    // prologue on the inputs (fp32 only)
   const void* add; int ld_add;             // y += add[row] (layout of out)

@@ -293,7 +293,7 @@ HiftConv conv_base(const void* x, int ldx, int cout, int cin_pad, int k, void* o
   HiftConv p{};
   p.docs = docs;
   p.x = x; p.ldx = ldx; p.cout = cout; p.cin_pad = cin_pad; p.k = k;
-  p.stride = 1; p.dil = 1; p.pad = 0; p.up = 1; p.rows_out = rows_out;
+  p.stride = 1; p.dil = 1; p.pad = 0; p.up = 1; p.rows_out = p.rows_live = rows_out;
   p.out = out; p.ldo = ldo; p.div = 1.0f;
   return p;
 }
@@ -302,6 +302,7 @@ HiftConv conv_base(const void* x, int ldx, int cout, int cin_pad, int k, void* o
 struct Convs {
   const FcvHift* h;
   hipStream_t st;
+  int frames, cap;  // Mel frames to expect, of the capacity's
 
   // n independent convolutions: p[i] with weight index wi[i] (bias wi[i] + 1); one launch where all of
   // them have split weights
@@ -310,6 +311,7 @@ struct Convs {
     for (int i = 0; i < n; ++i) {
       p[i].w = h->w[wi[i]];
       p[i].bias = h->w[wi[i] + 1];
+      p[i].rows_live = (int)(((long)p[i].rows_out * frames + cap - 1) / cap);
       const FcvHift::Packed& k = h->packed[wi[i]];
       if (h->packed_base && k.w >= 0) {
         p[i].wsplit = h->packed_base + k.w;
@@ -398,8 +400,9 @@ int run_resblocks(const Convs& cv, ResBlock* blocks, int n) {
   return FCV_OK;
 }
 
-// The launch sequence of one call over capacity C; the layout is in the table block.
-int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* source_out,
+// The launch sequence of one call over capacity C; the layout is in the table block.  `frames`: the
+// Mel frames its launches are shaped for (this call's, or the capacity where it is captured).
+int run(FcvHift* h, const float* mel, const Capacity& C, int frames, float* speech, float* source_out,
         char* ws, hipStream_t st) {
   const FcvHiftDims& d = h->d;
   const void* const* w = h->w.data();
@@ -458,7 +461,7 @@ int run(FcvHift* h, const float* mel, const Capacity& C, float* speech, float* s
   // ---- conv_pre (lookahead on the right) -------------------------------------------------
   float* xp = F32(C.xa);
   float* xn = F32(C.xn);
-  const Convs cv{h, st};
+  const Convs cv{h, st, frames, C.frames};
   {
     HiftConv c = conv_base(mel, d.in_channels, d.base_channels, d.in_channels,
                            d.conv_pre_look_right + 1, xp, d.base_channels, C.frames, T + 4);
@@ -595,7 +598,8 @@ int infer(FcvHift* h, const float* mel, const int32_t* frames, const int32_t* fi
   FCV_HIP(hipMemcpyAsync(ws + C.tables, tables.data(), tables.size() * sizeof(HiftDocs),
                          hipMemcpyHostToDevice, st));
   // the table copy reads pageable host memory: it is done once this call returns
-  if (!use_graph) return run(h, mel, C, speech, source_out, ws, st);
+  const int live = P.mel[n_docs];
+  if (!use_graph) return run(h, mel, C, live, speech, source_out, ws, st);
 
   const std::vector<uintptr_t> key = {(uintptr_t)frames_cap, (uintptr_t)docs_cap,
                                       (uintptr_t)ws, (uintptr_t)mel, (uintptr_t)speech,
@@ -608,11 +612,11 @@ int infer(FcvHift* h, const float* mel, const int32_t* frames, const int32_t* fi
     if (seen == h->seen.end()) {
       h->seen.insert(h->seen.begin(), key);
       if (h->seen.size() > kSeenKeys) h->seen.pop_back();
-      return run(h, mel, C, speech, source_out, ws, st);
+      return run(h, mel, C, live, speech, source_out, ws, st);
     }
     h->seen.erase(seen);
     FCV_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int r = run(h, mel, C, speech, source_out, ws, st);
+    int r = run(h, mel, C, frames_cap, speech, source_out, ws, st);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(st, &graph);
     if (r != FCV_OK) {

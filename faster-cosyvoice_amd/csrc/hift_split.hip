@@ -44,9 +44,10 @@ namespace {
 
 constexpr int kRowBytes = 128;  // one row of 32 channels: 4 chunks of hi, 4 of lo, 16 bytes each
 constexpr int kMaxHalo = 62;    // largest left context of a tile, in rows
-// 64x64 tiles in a launch (all its convolutions) under which the small form runs.  One call, all
-// small against all 64x64: 24 frames 0.68 and 1.19 ms, 68 0.88 and 1.21, 100 1.06 and 1.23, 200
-// 1.69 and 1.52, 286 2.30 and 1.71; by this rule 0.75, 0.80, 0.96, 1.33 and 1.59.
+// 64x64 tiles in a launch (all its convolutions, at the call's own rows) under which the small form
+// runs.  One call, all small, all 64x64, and by this rule, ms: 24 frames 0.67, 1.11, 0.67; 40 0.73,
+// 1.11, 0.73; 68 0.87, 1.12, 0.77; 100 1.03, 1.15, 0.91; 200 1.64, 1.44, 1.25; 286 2.23, 1.66, 1.56;
+// 600 4.27, 2.54, 2.53.  (By the capacity's rows, 64 frames at least, 24 frames took 0.74.)
 constexpr long kSmallBelow = 256;
 
 // position of 16-byte chunk `chunk` in LDS row `row`: 16 consecutive rows read at one chunk index
@@ -859,7 +860,7 @@ hipError_t hift_conv_split(const HiftConv* convs, int n, hipStream_t stream) {
     jobs.c[i] = convs[i];
     rows = std::max(rows, convs[i].rows_out);
     cout = std::max(cout, convs[i].cout);
-    tiles64 += (long)((convs[i].rows_out + 63) / 64) * ((convs[i].cout + 63) / 64);
+    tiles64 += (long)((convs[i].rows_live + 63) / 64) * ((convs[i].cout + 63) / 64);
   }
   if (rows <= 0) return hipSuccess;
   // FCV_HIFT_TILE = 32 or 64 forces a tile: a test hook, both must give the same bits
