@@ -135,10 +135,11 @@ constexpr size_t kGraphPool = 4;  // captured calls kept per handle (least recen
 // Mel frames of a capacity up to which a stage's resblocks run together.  A resblock is a chain of
 // six convolutions that depend on each other; the three of a stage and the next stage's source
 // branch do not, so one launch takes one convolution of each: 79 convolution launches a call
-// become 33, each with three to four times the workgroups.  One call, apart against together: 24
-// frames 2.00 -> 1.20 ms, 68 2.05 -> 1.26, 286 2.53 -> 1.91, 900 4.68 -> 4.08, 8 requests of 3065
-// frames 10.6 either way.  It takes 16 stage buffers instead of 7 (0.5 MB a frame), hence the limit.
-constexpr int kTogetherFrames = 1 << 16;
+// become 33, each with three to four times the workgroups.  One call, apart against together: 286
+// frames 2.14 -> 1.65 ms, 900 4.27 -> 3.69, 1500 5.70 -> 5.47, 2000 7.33 -> 7.24, 3065 10.87 -> 10.76,
+// 4000 14.1 -> 14.0, 6000 and 12000 the same.  It takes 16 stage buffers in place of 7 (0.49 MB a frame
+// against 0.21), hence the limit, about where the gain ends.
+constexpr int kTogetherFrames = 3072;
 constexpr size_t kSeenKeys = 8;   // keys remembered for the capture-on-second-call rule
 
 // The workspace carve-up and the grids of a capacity: at most `frames` Mel frames in at most
@@ -158,7 +159,7 @@ struct Capacity {
 // Tables of one call, in launch order (see run): their count for n_stages stages.
 int table_count(const FcvHiftDims& d) { return 7 + 3 * d.n_stages; }
 
-Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
+Capacity make_capacity(const FcvHiftDims& d, int frames, int docs, bool together) {
   Capacity C;
   C.frames = frames;
   C.docs = docs;
@@ -184,9 +185,11 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
   C.sines = take(sizeof(float) * frames * H);
   C.srcbuf = take(sizeof(float) * C.src);
   C.specbuf = take(sizeof(float) * C.spec * kSpecLd);
-  for (size_t* b : {&C.xa, &C.xn, &C.xs, &C.si[0]}) *b = take(sizeof(float) * smax);
-  C.together = frames <= kTogetherFrames;
-  C.si[1] = C.together ? take(sizeof(float) * smax) : C.si[0];
+  for (size_t* b : {&C.xa, &C.xn, &C.si[0]}) *b = take(sizeof(float) * smax);
+  C.together = together;
+  // the resblocks' running sum where they run apart, the next stage's source branch elsewhere
+  C.xs = C.si[1] = take(sizeof(float) * smax);
+  if (!C.together) C.si[1] = C.si[0];
   for (int i = 0; i <= d.n_kernels; ++i) {
     const bool own = i == 0 || C.together;
     C.r[i] = own ? take(sizeof(float) * smax) : C.r[0];
@@ -198,6 +201,11 @@ Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
   C.tables = take(sizeof(HiftDocs) * table_count(d));
   C.total = off;
   return C;
+}
+
+// The workspace to ask for at a capacity.
+Capacity make_capacity(const FcvHiftDims& d, int frames, int docs) {
+  return make_capacity(d, frames, docs, frames <= kTogetherFrames);
 }
 
 // The layout of one call: per-document lengths and their prefix sums.
@@ -588,7 +596,9 @@ int infer(FcvHift* h, const float* mel, const int32_t* frames, const int32_t* fi
                 " documents)");
   FCV_CHECK((long)frames_cap * upsample_scale(h->d) < (1L << 30), FCV_ERR_INVALID,
             "capacity too large");
-  const Capacity C = make_capacity(h->d, frames_cap, docs_cap);
+  Capacity C = make_capacity(h->d, frames_cap, docs_cap);
+  // a smaller workspace, one for a larger capacity among them, takes the resblocks one by one
+  if (workspace_bytes < C.total && C.together) C = make_capacity(h->d, frames_cap, docs_cap, false);
   FCV_CHECK(workspace_bytes >= C.total, FCV_ERR_INVALID,
             "workspace too small: need " + std::to_string(C.total) + " bytes");
   FCV_CHECK(reinterpret_cast<uintptr_t>(workspace) % kAlign == 0, FCV_ERR_INVALID,
@@ -603,7 +613,7 @@ int infer(FcvHift* h, const float* mel, const int32_t* frames, const int32_t* fi
 
   const std::vector<uintptr_t> key = {(uintptr_t)frames_cap, (uintptr_t)docs_cap,
                                       (uintptr_t)ws, (uintptr_t)mel, (uintptr_t)speech,
-                                      (uintptr_t)source_out};
+                                      (uintptr_t)source_out, (uintptr_t)C.together};
   auto hit = std::find_if(h->graphs.begin(), h->graphs.end(),
                           [&](const FcvHift::Graph& g) { return g.key == key; });
   if (hit == h->graphs.end()) {

@@ -97,7 +97,9 @@ int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes);
  * (generator.py:700-731).  -1 if the document is too short. */
 int64_t fcv_hift_output_samples(const FcvHift* hift, int32_t frames, int32_t finalize);
 
-/* Device workspace for one fcv_hift_inference call over these documents. */
+/* Device workspace for one fcv_hift_inference call over these documents.  Up to 3072 frames it lets a
+ * stage's resblocks run together (0.54 MB a frame at the CosyVoice3 shape); a call whose workspace is
+ * smaller, down to 0.27 MB a frame, takes them one after another, with the same results. */
 size_t fcv_hift_workspace_bytes(const FcvHift* hift, const int32_t* frames_host,
                                 const int32_t* finalize_host, int32_t n_docs);
 
@@ -112,7 +114,8 @@ int fcv_hift_inference(FcvHift* hift, const float* mel, const int32_t* frames_ho
                        float* source_out, void* workspace, size_t workspace_bytes,
                        hipStream_t stream);
 
-/* Device workspace of a call capacity: at most frames_cap Mel frames in docs_cap documents. */
+/* Device workspace of a call capacity: at most frames_cap Mel frames in docs_cap documents (see
+ * fcv_hift_workspace_bytes). */
 size_t fcv_hift_workspace_bytes_capacity(const FcvHift* hift, int32_t frames_cap,
                                          int32_t docs_cap);
 

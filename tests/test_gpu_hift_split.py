@@ -151,3 +151,25 @@ def test_output_before_a_change_stays_bit_for_bit(fcv, monkeypatch):
     c, = split.inference_batched([mel[:, :50]], [False])
     keep = (41 - 4 - 1) * 480
     assert torch.equal(a[:, :keep], b[:, :keep]) and torch.equal(a[:, :keep], c[:, :keep])
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("packed", [True, False], ids=["split", "fp32"])
+def test_resblocks_one_by_one_give_the_same_bits(fcv, monkeypatch, packed, graph):
+    """A workspace too small for a stage's resblocks to run together takes them one after another
+    (running sum, then the mean in the last one's epilogue), as every capacity past the limit does:
+    final and non-final documents, one of them of a single row, and replays of a captured call."""
+    voc = _pair(fcv, monkeypatch)[0 if packed else 1]
+    g = torch.Generator().manual_seed(99)
+    mels = [torch.randn(80, n, generator=g).cuda() for n in (33, 1, 24, 70)]
+    fin = [True, True, False, False]
+    say(f"[split] resblocks one by one, packed {packed}, graph {graph}")
+    run = lambda: voc.inference_batched(mels, fin, concurrency=1, graph=graph)
+    ref = [run() for _ in range(3)][-1]
+    need = voc._lib.fcv_hift_workspace_bytes_capacity
+    monkeypatch.setattr(voc._lib, "fcv_hift_workspace_bytes_capacity",
+                        lambda h, f, d: need(h, f, d) // 2)
+    voc._lanes[0][1] = None
+    for _ in range(3):
+        got = run()
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))

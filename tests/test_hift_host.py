@@ -62,6 +62,24 @@ def test_output_lengths_and_short_chunks(fcv):
         v._lib.fcv_hift_destroy(h)
 
 
+def test_workspace_of_large_calls(fcv):
+    """Past 3072 frames the resblocks of a stage run one after another, in under half the memory a
+    frame: a call as large as the card is asked for no more than it needs."""
+    from faster_cosyvoice_amd import _lib
+    v = _vocoder(fcv)
+    v._cdims.noise_samples = 1000
+    h = ctypes.c_void_p()
+    arr = (ctypes.c_void_p * 321)(*([4096] * 321))
+    _lib.check(v._lib.fcv_hift_create(v._cdims, arr, 321, h))
+    try:
+        size = lambda f: v._lib.fcv_hift_workspace_bytes_capacity(h, f, 8) / f
+        assert 0.50e6 < size(3072) < 0.55e6
+        for frames in (3073, 12000, 65536):
+            assert 0.25e6 < size(frames) < 0.27e6, frames
+    finally:
+        v._lib.fcv_hift_destroy(h)
+
+
 def test_strict_state_dict_load(fcv):
     syn = fcv.synthetic
     dims = syn.HiFTDims()
