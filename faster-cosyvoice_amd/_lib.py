@@ -117,6 +117,7 @@ SIGNATURES = {
     "fcv_hift_packed_bytes": (c_size_t, [c_void_p]),
     "fcv_hift_pack_weights": (c_int32, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "fcv_hift_use_packed": (c_int32, [c_void_p, c_void_p, c_size_t]),
+    "fcv_hift_weight_packed": (c_int32, [c_void_p, c_int32]),
     "fcv_hift_output_samples": (ctypes.c_int64, [c_void_p, c_int32, c_int32]),
     "fcv_hift_workspace_bytes": (c_size_t, [c_void_p, POINTER(c_int32), POINTER(c_int32),
                                             c_int32]),

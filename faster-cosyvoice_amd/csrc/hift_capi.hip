@@ -693,13 +693,7 @@ void plan_packed(FcvHift* h) {
   h->packed_bytes = off;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t fcv_hift_packed_bytes(const FcvHift* hift) { return hift ? hift->packed_bytes : 0; }
-
-int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes) {
+int check_packed(const FcvHift* hift, const void* packed, size_t bytes) {
   FCV_CHECK(hift, FCV_ERR_INVALID, "null handle");
   FCV_CHECK(hift->packed_bytes > 0, FCV_ERR_INVALID, "no convolution of this shape has split weights");
   FCV_CHECK(packed, FCV_ERR_INVALID, "null argument");
@@ -709,12 +703,30 @@ int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes) {
             "packed weights must be 256-byte aligned");
   FCV_CHECK(hift->graphs.empty() && hift->seen.empty(), FCV_ERR_STATE,
             "set the packed weights before the first inference");
+  return FCV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t fcv_hift_packed_bytes(const FcvHift* hift) { return hift ? hift->packed_bytes : 0; }
+
+int32_t fcv_hift_weight_packed(const FcvHift* hift, int32_t index) {
+  return hift && index >= 0 && index < (int32_t)hift->packed.size() && hift->packed_base &&
+                 hift->packed[index].w >= 0
+             ? 1
+             : 0;
+}
+
+int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes) {
+  if (int rc = check_packed(hift, packed, bytes)) return rc;
   hift->packed_base = static_cast<const char*>(packed);
   return FCV_OK;
 }
 
 int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t stream) {
-  if (int rc = fcv_hift_use_packed(hift, packed, bytes)) return rc;
+  if (int rc = check_packed(hift, packed, bytes)) return rc;
   const FcvHiftDims& d = hift->d;
   char* base = static_cast<char*>(packed);
   auto pack = [&](int wi, int cout, int cin, int k) -> int {
@@ -743,7 +755,10 @@ int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t
         return rc;
     cprev = C;
   }
-  return pack(hift->i_post, d.n_fft + 2, cprev, 7);
+  if (int rc = pack(hift->i_post, d.n_fft + 2, cprev, 7)) return rc;
+  // only a table that every launch fills is used
+  hift->packed_base = base;
+  return FCV_OK;
 }
 
 int32_t fcv_hift_weight_count(const FcvHiftDims* dims) {

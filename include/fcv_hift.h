@@ -85,11 +85,15 @@ int fcv_hift_destroy(FcvHift* hift);
  * its taps read and on no others, as on the fp32 matrix cores.  fcv_hift_pack_weights
  * computes them on `stream` into caller-owned memory of fcv_hift_packed_bytes (0: no such
  * convolution in this shape), 256-byte aligned, which must outlive the handle; it is called before
- * the handle's first inference.  fcv_hift_use_packed gives another handle over the same weights
- * the memory that was filled. */
+ * the handle's first inference, and where it fails the handle keeps what it ran on.
+ * fcv_hift_use_packed gives another handle over the same weights the memory that was filled.
+ * Inference on any other stream, through either handle, must be ordered after `stream`'s packing.
+ * fcv_hift_weight_packed: 1 where the handle runs on the split form of the weight at `index` of the
+ * table (its fp32 values are not read again), else 0. */
 size_t fcv_hift_packed_bytes(const FcvHift* hift);
 int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t stream);
 int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes);
+int32_t fcv_hift_weight_packed(const FcvHift* hift, int32_t index);
 
 /* Waveform samples produced for a document of `frames` Mel frames:
  * finalize != 0: frames * upsample_scale (480 for CosyVoice3); otherwise the last

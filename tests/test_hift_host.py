@@ -62,6 +62,30 @@ def test_output_lengths_and_short_chunks(fcv):
         v._lib.fcv_hift_destroy(h)
 
 
+def test_failed_packing_leaves_the_handle_as_it_was(fcv):
+    """Where a packing launch fails (here: no GPU at all) the handle does not run on the memory that
+    was to be filled."""
+    from faster_cosyvoice_amd import _lib
+    if torch.cuda.is_available():
+        pytest.skip("the launches would run")
+    v = _vocoder(fcv)
+    v._cdims.noise_samples = 1000
+    h = ctypes.c_void_p()
+    arr = (ctypes.c_void_p * 321)(*([4096] * 321))
+    _lib.check(v._lib.fcv_hift_create(v._cdims, arr, 321, h))
+    try:
+        need = v._lib.fcv_hift_packed_bytes(h)
+        used = lambda: sum(v._lib.fcv_hift_weight_packed(h, i) for i in range(-1, 322))
+        with pytest.raises(RuntimeError):
+            _lib.check(v._lib.fcv_hift_pack_weights(h, 4096, need, None))
+        assert used() == 0
+        _lib.check(v._lib.fcv_hift_use_packed(h, 4096, need))
+        # ups, both convolutions of 12 resblocks at 3 dilations, conv_post
+        assert used() == 3 + 2 * 12 * 3 + 1
+    finally:
+        v._lib.fcv_hift_destroy(h)
+
+
 def test_workspace_of_large_calls(fcv):
     """Past 3072 frames the resblocks of a stage run one after another, in under half the memory a
     frame: a call as large as the card is asked for no more than it needs."""
