@@ -208,6 +208,9 @@ class HiFTVocoder:
             _lib.check(self._lib.fcv_hift_pack_weights(handle, self._packed.data_ptr(), need,
                                                        stream.cuda_stream))
             stream.synchronize()  # other streams' calls read them
+            # no handle reads the fp32 values of a packed weight again
+            self._keep = [t for i, t in enumerate(keep)
+                          if not self._lib.fcv_hift_weight_packed(handle, i)]
 
     def __del__(self):
         try:

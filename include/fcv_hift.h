@@ -89,7 +89,8 @@ int fcv_hift_destroy(FcvHift* hift);
  * fcv_hift_use_packed gives another handle over the same weights the memory that was filled.
  * Inference on any other stream, through either handle, must be ordered after `stream`'s packing.
  * fcv_hift_weight_packed: 1 where the handle runs on the split form of the weight at `index` of the
- * table (its fp32 values are not read again), else 0. */
+ * table, else 0; its fp32 values are then not read again and may be freed once the packing is done,
+ * as long as every handle made over the table is given the packed memory before its first use. */
 size_t fcv_hift_packed_bytes(const FcvHift* hift);
 int fcv_hift_pack_weights(FcvHift* hift, void* packed, size_t bytes, hipStream_t stream);
 int fcv_hift_use_packed(FcvHift* hift, const void* packed, size_t bytes);

@@ -173,3 +173,18 @@ def test_resblocks_one_by_one_give_the_same_bits(fcv, monkeypatch, packed, graph
     for _ in range(3):
         got = run()
         assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_packed_weights_take_the_place_of_the_fp32_ones(fcv):
+    """After the packing only the weights that some kernel reads in fp32 stay on the card."""
+    dims = fcv.synthetic.HiFTDims()
+    v = fcv.HiFTVocoder(dims, device="cuda:0",
+                        buffers=fcv.synthetic.random_hift_buffers(dims, max_samples=4800, seed=92))
+    v.load_reference_state_dict(fcv.synthetic.random_hift_state_dict(dims, seed=91))
+    before = torch.cuda.memory_allocated()
+    v.finalize_weights()
+    held = torch.cuda.memory_allocated() - before
+    packed = v._packed.numel()
+    say(f"[split] {packed >> 20} MB packed, {held >> 20} MB held")
+    assert len(v._keep) == 321 - 76
+    assert held < 1.5 * packed
