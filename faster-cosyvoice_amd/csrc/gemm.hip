@@ -735,13 +735,16 @@ hipError_t launch_tile(const f16* A, int lda, const f16* W, int ldw, int M, int 
 // capacities one request plans into (340-3090 rows) with every shape and ring depth forced;
 // its pick is within 3 % of the fastest at every measured size, and the four GEMMs of a block
 // take 12-20 % less time at 340-1170 rows than the estimate's pick.  32x64 tiles of two waves (six
-// stages while two per CU hold every tile, four and three per CU above; eight were no better) give the 1024-column GEMMs
-// twice the workgroups where 64x64 tiles leave CUs idle, and QKV an even share where 64x64 tiles put
-// two on some CUs: whole solves of one request -5 % at 270-400 rows, -3 % at 460-530, -1 to -3 % at
-// 590-780 for the former (even at 910), -4 to -5 % at 366-398 rows for the latter (+1 to +7 % outside).  The choice only changes
-// which rows and columns share a workgroup: every output element still accumulates its K
-// slices in the same order, so results are bitwise identical for every tile shape (batch
-// invariance holds).
+// stages while two per CU hold every tile, four and three per CU above; eight were no better) give
+// the 1024-column GEMMs twice the workgroups where 64x64 tiles leave CUs idle: whole solves of one
+// request -5 % at 270-400 rows, -3 % at 460-530, -1 to -3 % at 590-780 (even at 910).  For QKV they fill
+// the gap between 64x64 tiles one a CU (240 up to 320 rows; 288 above, two on some CUs) and 128x64
+// tiles (192 from 385 rows on), here at the rows with the padding of one request's two documents.
+// 22-block forwards, us, 64x64 against 32x64: 310 rows 1137 and 1166, 325 1234 and 1182, 352 1247 and
+// 1201, 370 1258 and 1209, 384 1258 and 1209; 386 rows 1235 with 32x64 and 1231 with 128x64; solves of
+// 336 to 384 rows -4 to -5 %.  The choice only changes which rows and columns share a workgroup:
+// every output element still accumulates its K slices in the same order, so results are bitwise
+// identical for every tile shape (batch invariance holds).
 constexpr int kCus = 256;
 constexpr int kTileShapes = 12;
 constexpr int kTileShape[kTileShapes][2] = {{256, 256}, {192, 256}, {128, 256}, {256, 128},
@@ -765,8 +768,8 @@ constexpr SmallStep kSmall2048[] = {  // FF1
     {600, kTile64x64}, {1000, kTile128x64}, {1536, kTile96x128}, {2048, kTile128x128},
     {2200, kTile128x64}};
 constexpr SmallStep kSmall3072[] = {  // QKV
-    {350, kTile64x64}, {400, kTile32x64}, {850, kTile128x64}, {1000, kTile64x128}, {1200, kTile128x64},
-    {1440, kTile64x128}, {2100, kTile96x128}};
+    {334, kTile64x64},   {398, kTile32x64},  {850, kTile128x64}, {1000, kTile64x128},
+    {1200, kTile128x64}, {1440, kTile64x128}, {2100, kTile96x128}};
 
 template <int L>
 inline int small_step(const SmallStep (&steps)[L], int M) {
