@@ -51,9 +51,9 @@ __device__ __forceinline__ void conv_finish(const f32x4& v, const float4& b, con
 // from 1100 rows up: two workgroups of 128 rows on a CU hide each other's taps, one of 256 has
 // nothing beside it.)  MFMA 32x32x16 with the weights as the A operand, so lane l accumulates output
 // row l % 32 and, in register group g of channel tile t, channels 32 t + 8 g + 4 (l / 32) + 0..3.
-// The epilogue stages each wave's 32 x 64 block through LDS and reads it back row-major (16 lanes per row), so stores are contiguous runs of
-// 128 B (f16 out) or 256 B (fp32 residual); the residual form issues all its h loads before
-// its first store.
+// The epilogue stages each wave's 32 x 64 block through LDS and reads it back row-major (16 lanes per
+// row), so stores are contiguous runs of 128 B (f16 out) or 256 B (fp32 residual); the residual form
+// issues all its h loads before its first store.
 __global__ __launch_bounds__(256, 2) void conv_kernel(const f16* __restrict__ x, int C,
                                                       const f16* __restrict__ w,
                                                       const float* __restrict__ bias, int taps,

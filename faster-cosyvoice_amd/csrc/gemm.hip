@@ -737,8 +737,8 @@ hipError_t launch_tile(const f16* A, int lda, const f16* W, int ldw, int M, int 
 // take 12-20 % less time at 340-1170 rows than the estimate's pick.  32x64 tiles of two waves (six
 // stages while two per CU hold every tile, four and three per CU above; eight were no better) give
 // the 1024-column GEMMs twice the workgroups where 64x64 tiles leave CUs idle: whole solves of one
-// request -5 % at 270-400 rows, -3 % at 460-530, -1 to -3 % at 590-780 (even at 910).  For QKV they fill
-// the gap between 64x64 tiles one a CU (240 up to 320 rows; 288 above, two on some CUs) and 128x64
+// request -5 % at 270-400 rows, -3 % at 460-530, -1 to -3 % at 590-780 (even at 910).  For QKV they
+// fill the gap between 64x64 tiles one a CU (240 up to 320 rows; 288 above, two on some CUs) and 128x64
 // tiles (192 from 385 rows on), here at the rows with the padding of one request's two documents.
 // 22-block forwards, us, 64x64 against 32x64: 310 rows 1137 and 1166, 325 1234 and 1182, 352 1247 and
 // 1201, 370 1258 and 1209, 384 1258 and 1209; 386 rows 1235 with 32x64 and 1231 with 128x64; solves of

@@ -3,9 +3,9 @@
 // Every convolution of the vocoder is one implicit GEMM on the matrix cores.  The causal
 // unit-stride ones (upsampling, resblocks, conv_post) run in hift_split.hip where the handle has
 // split weights; the rest -- conv_pre, the strided source convs, and the fp64 F0 predictor with a
-// kernel of its own -- run here on v_mfma_{f32,f64}_16x16x4: weights are the A operand (rows = output channels),
-// the gathered input rows the B operand, so a lane's four accumulators are four channels of one
-// time step (consecutive in fp32; four apart in fp64, whose 16x16 result is laid out by rows
+// kernel of its own -- run here on v_mfma_{f32,f64}_16x16x4: weights are the A operand (rows = output
+// channels), the gathered input rows the B operand, so a lane's four accumulators are four channels
+// of one time step (consecutive in fp32; four apart in fp64, whose 16x16 result is laid out by rows
 // 4 e + lane / 16).  Operands of the fp32 convolutions go through LDS K-contiguous, 32 (or 16)
 // input channels of one tap per chunk, with a register-prefetched double buffer.  A workgroup owns
 // 64 time rows x 64 output channels (32 x 32 in launches too small to give every CU a 64 x 64
@@ -279,8 +279,8 @@ __global__ __launch_bounds__(256) void mean_kernel(const HiftMean in, float* __r
 // quarter of K each (added in order in LDS), straight from global memory: these products have 72 to
 // a few thousand rows, so what counts is the chain of MFMAs a wave runs (64 cycles each), and a
 // quarter of K on four times the waves cuts it to a quarter.  One layer at 72 rows 44 -> 15 us
-// against 32x32 tiles with K in one chain through LDS (1664 rows: the same); T = 2 halves the operand reads where 16x16
-// tiles would be many (the sums are the same).
+// against 32x32 tiles with K in one chain through LDS (1664 rows: the same); T = 2 halves the operand
+// reads where 16x16 tiles would be many (the sums are the same).
 template <typename X, int T>
 __global__ __launch_bounds__(256) void f0_conv_kernel(const HiftConv p) {
   constexpr int TS = 16 * T;

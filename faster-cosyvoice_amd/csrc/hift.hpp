@@ -108,7 +108,7 @@ struct HiftSource {
   float* sines;             // [frames][H] work: sin(phase) * sine_amp per frame
   float* s;                 // [samples] source, rows by docs.b
 };
-// per-frame phases (sequential sum per document and harmonic) then per-sample merge
+// per-frame phases (running sum per document and harmonic, a scan) then per-sample merge
 hipError_t hift_source(const HiftSource& p, const HiftDocs* docs, hipStream_t stream);
 
 // dst[i] = src[i] for the live rows docs->b[docs->n] (grid: `rows`)

@@ -53,7 +53,7 @@ def test_vocoder_matches_oracle(hift, finalize):
 def test_long_requests_packed_match_oracle(fcv):
     """Three requests of 600-700 frames (12-14 s of audio each) in one packed call against the
     oracle run on each alone: the harmonic source phase reaches ~1e6 rad over such a request and
-    is accumulated sequentially in the reference's fp32 order, so the source stays within 1e-5
+    is the running sum that the reference takes over fp32 increments, so the source stays within 1e-5
     absolute and the waveform within rel-L2 1e-4 over the whole length."""
     dims = fcv.synthetic.HiFTDims()
     sd = fcv.synthetic.random_hift_state_dict(dims, seed=75)
