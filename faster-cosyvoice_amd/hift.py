@@ -32,8 +32,8 @@ def _ceil(v: int, m: int) -> int:
 # Smallest capacity (Mel frames of one packed call) whose call replays its captured graph when
 # the caller leaves ``graph`` to the vocoder.  The eager call is one C-ABI call that enqueues the
 # launch sequence faster than the GPU drains it, so a replay saves host time but no device time:
-# on one MI355X a 68-frame streaming chunk took 0.788 ms replayed and 0.784 eagerly, and config 3's
-# packed groups 8.71 and 8.69 ms.  Small calls (streaming chunks) therefore launch eagerly.
+# on one MI355X a 68-frame streaming chunk took 0.768 ms replayed and 0.762 eagerly, and config 3's
+# packed groups 8.72 and 8.64 ms.  Small calls (streaming chunks) therefore launch eagerly.
 HIFT_GRAPH_MIN_FRAMES = 1024
 
 
