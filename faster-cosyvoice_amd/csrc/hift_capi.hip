@@ -658,12 +658,14 @@ void plan_packed(FcvHift* h) {
   const FcvHiftDims& d = h->d;
   h->packed.assign(h->w.size(), FcvHift::Packed{});
   size_t off = 0;
-  auto add = [&](int wi, int cout, int cin, int k, int dil, int up) {
+  auto add = [&](int wi, int cout, int cin, int k, int dil, int up, float slope) {
     HiftConv p = conv_base(nullptr, 0, cout, cin, k, nullptr, 0, 0, nullptr);
     p.dil = dil;
     p.up = up;
     p.pad = causal_padding(k, dil);
     if (up > 1) p.pad = k - 1;
+    p.pro = fcv::HIFT_PRO_LEAKY;
+    p.slope = slope;
     if (!fcv::hift_split_eligible(p)) return;
     FcvHift::Packed& e = h->packed[wi];
     e.co_pad = (cout + 63) / 64 * 64;
@@ -674,22 +676,22 @@ void plan_packed(FcvHift* h) {
   };
   auto resblock = [&](int wi, int C, int k, const int* dils) {
     for (int j = 0; j < d.n_dilations; ++j) {
-      add(wi + 8 * j, C, C, k, dils[j], 1);
-      add(wi + 8 * j + 2, C, C, k, 1, 1);
+      add(wi + 8 * j, C, C, k, dils[j], 1, 0.0f);
+      add(wi + 8 * j + 2, C, C, k, 1, 1, 0.0f);
     }
   };
   const int rb = 8 * d.n_dilations;
   int cprev = d.base_channels;
   for (int s = 0; s < d.n_stages; ++s) {
     const int C = stage_channels(d, s);
-    add(h->i_ups + 2 * s, C, cprev, d.upsample_kernels[s], 1, d.upsample_rates[s]);
+    add(h->i_ups + 2 * s, C, cprev, d.upsample_kernels[s], 1, d.upsample_rates[s], d.lrelu_slope);
     resblock(h->i_srb + rb * s, C, d.source_kernels[s], d.source_dilations[s]);
     for (int j = 0; j < d.n_kernels; ++j)
       resblock(h->i_rb + rb * (s * d.n_kernels + j), C, d.resblock_kernels[j],
                d.resblock_dilations[j]);
     cprev = C;
   }
-  add(h->i_post, d.n_fft + 2, cprev, 7, 1, 1);
+  add(h->i_post, d.n_fft + 2, cprev, 7, 1, 1, 0.01f);
   h->packed_bytes = off;
 }
 

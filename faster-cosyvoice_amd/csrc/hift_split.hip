@@ -10,7 +10,8 @@
 // kernels: not on what else is in its document, later or louder, or on the tile.
 // Against 64-bit results the waveform's relative error is 9.4e-6 (8 requests) where
 // v_mfma_f32_16x16x4_f32 left 2.6e-5: the operands' rounding adds 1.7e-6, and sums of 16 products at a
-// time round less often than sums of 4.
+// time round less often than sums of 4.  Where one conv's input channels lie up to 2^16 apart, its
+// weights the other way, it stays at 9.6e-6; 2^24 apart it is 7.5e-5 (the fp32 form 2.7e-5).
 //
 // Bound: three f16 MFMAs do a product's work at 16 times the fp32 form's rate each, so the ceiling
 // is a third of the f16 peak against the fp32 peak of 157 TFLOP/s.  Measured on one MI355X against
@@ -836,7 +837,8 @@ bool launchable(const HiftConv& p) {
 
 bool hift_split_eligible(const HiftConv& p) {
   return p.stride == 1 && p.cin_pad % 32 == 0 && p.up >= 1 && p.dil >= 1 &&
-         (p.up == 1 || p.dil == 1) && p.pad == (p.k - 1) * p.dil && p.pad <= kMaxHalo;
+         (p.up == 1 || p.dil == 1) && p.pad == (p.k - 1) * p.dil && p.pad <= kMaxHalo &&
+         (p.pro == HIFT_PRO_NONE || (p.slope >= -1.0f && p.slope <= 1.0f));
 }
 
 size_t hift_split_bytes(int co_pad, int k, int cin) {
